@@ -5,6 +5,8 @@
 //   daxpy / waxpby / fill / copy : grid-stride elementwise kernels
 //   fill_uniform : counter-based SplitMix64 inputs (bitwise equal to the host)
 
+#include <algorithm>
+
 #include "common.hpp"
 #include "rng.hpp"
 
@@ -95,15 +97,36 @@ __global__ __launch_bounds__(kBlock) void dot_final_kernel(const double* __restr
 // ---------------------------------------------------------------------------
 // dgemv: y = A x, column-major A.
 //
-// A block of 4 waves owns a 128-row panel; lane l of every wave handles rows
-// 2l, 2l+1 of the panel with one 16-byte load per column, so each wave reads
-// 1 KiB contiguous per column.  The block's column slab is split into four
-// contiguous quarters, one per wave; x[j] is wave-uniform and comes through
-// the scalar cache.  The four wave sums are combined in LDS in wave order and
-// written as one partial per (slab, row); a second kernel adds the slabs in
-// slab order.  The slab count depends only on (m, n): about 256 workgroups
-// (one per CU) with at least 256 columns per wave measured fastest from
-// N = 4096 (cache-resident) to N = 131072 (HBM).
+// A workgroup of NW waves owns a panel of 2 RL rows and one slab of columns.
+// RL lanes of a wave hold two rows each (one 16-byte load per column), its
+// 64 / RL lane groups take column pairs side by side, and the waves take
+// contiguous shares of the slab.  Lane groups are added by xor-shuffles, waves
+// in wave order through LDS, and a second kernel adds the slabs in slab order;
+// every split depends only on (m, n).
+//
+// Column strides are whatever lda is: a 16-byte load needs 4-byte alignment
+// only, so matrices of odd lda (or a base that is 8-byte aligned) take the
+// same loads as even ones.  Two 8-byte loads per lane and column, as such
+// matrices had before, ran a 30001 x 20003 product at 2.9 TB/s; 16-byte loads
+// run it at 6.4 TB/s (1663 -> 751 us).
+//
+// Two geometries:
+// * streamed (RL = 64, 4 waves): each load instruction reads 1 KiB of one
+//   column; bound by HBM or the Infinity Cache.  A product keeps the memory
+//   system busy from about 152 workgroups, and above 256 (one per CU) a last
+//   round that is nearly empty costs up to a third (n = 16385: 465 us at 258
+//   workgroups, 363 us at 2064), so the slab count is the smallest with 152
+//   to 256 workgroups, or else with at least 90 % of the last round filled.
+// * panels of 16 rows (RL = 8, 16 waves): a matrix of up to 40 MB has too few
+//   128-row panels to fill the chip and is bound by latency; 16-row panels
+//   put 16 waves on each of m / 16 CUs with every load of a wave in flight
+//   at once and mostly need no second kernel (1000 x 1000: 4.9 us against
+//   9.9 us streamed, 1500 x 1500: 7.0 us against 7.4 us; 2500 x 2500: 14.1 us
+//   against 11.7 us, so the line lies between the last two).  Fewer than 256
+//   columns leave its 128 column slots idle (30000 x 64: 12.4 us against
+//   4.3 us streamed).  Matrices of up to 64 rows take it at any size: most
+//   lanes of a 128-row panel would hold no row (64 x 30000: 7.5 us in 32
+//   slabs).
 //
 // A matrix larger than the 256 MiB Infinity Cache is read with nontemporal
 // loads (STREAM): every element is used once, and the hint keeps the stream
@@ -113,142 +136,198 @@ __global__ __launch_bounds__(kBlock) void dot_final_kernel(const double* __restr
 // 32 us).
 // ---------------------------------------------------------------------------
 
-constexpr int kGvRows = 128;
-constexpr int kGvTargetBlocks = 256;  // ~one 4-wave workgroup per CU (swept on MI355X)
-constexpr int64_t kGvStreamBytes = int64_t(256) << 20;  // Infinity Cache capacity
+constexpr int kGvUnroll = 8;                                // columns of a lane in flight
+constexpr int kGvStreamLanes = 64, kGvStreamWaves = 4;      // 128-row panels
+constexpr int kGvPanelLanes = 8, kGvPanelWaves = 16;        // 16-row panels
+constexpr double kGvPanelBytes = 40e6;                      // largest matrix of the 16-row panels
+constexpr int64_t kGvPanelRows = 64;                        // or most rows at any size
+constexpr int64_t kGvPanelCols = 256;                       // fewest columns
+constexpr int64_t kGvCus = 256;
+constexpr int64_t kGvBusy = 152;                            // workgroups that saturate the memory system
+constexpr int64_t kGvStreamBytes = int64_t(256) << 20;      // Infinity Cache capacity
 
-typedef double gv_f64x2 __attribute__((ext_vector_type(2)));
+typedef double gv_f64x2 __attribute__((ext_vector_type(2), aligned(8)));
 
 template <bool STREAM>
-__device__ inline gv_f64x2 gv_load2(const double* p) {
+__device__ __forceinline__ gv_f64x2 gv_load2(const double* p) {
   const gv_f64x2* q = reinterpret_cast<const gv_f64x2*>(p);
   if constexpr (STREAM) return __builtin_nontemporal_load(q);
   else return *q;
 }
 
-template <bool STREAM>
-__device__ inline double gv_load1(const double* p) {
-  if constexpr (STREAM) return __builtin_nontemporal_load(p);
-  else return *p;
-}
-
 struct GemvPlan {
-  int64_t row_tiles;
-  int64_t slabs;
-  int64_t slab_cols;
+  bool panels;  // 16-row panels
+  int64_t row_tiles, slabs, slab_cols;
 };
 
 inline GemvPlan gemv_plan(int64_t m, int64_t n) {
   GemvPlan p;
-  p.row_tiles = (m + kGvRows - 1) / kGvRows;
-  int64_t ks = (kGvTargetBlocks + p.row_tiles - 1) / p.row_tiles;
-  int64_t max_ks = n / 1024;  // keep at least 256 columns per wave
-  if (max_ks < 1) max_ks = 1;
-  if (ks > max_ks) ks = max_ks;
+  p.panels = n >= kGvPanelCols && (m <= kGvPanelRows || (double)m * (double)n * sizeof(double) <= kGvPanelBytes);
+  const int64_t rows = 2 * (p.panels ? kGvPanelLanes : kGvStreamLanes);
+  p.row_tiles = (m + rows - 1) / rows;
+  int64_t ks = 1;
+  if (p.panels) {
+    // a lane walks n / 128 columns: wide matrices of few rows are split further
+    if (n >= 4096) ks = std::min((kGvCus + p.row_tiles - 1) / p.row_tiles, n / 1024);
+  } else {
+    const int64_t most = std::min<int64_t>(std::max<int64_t>(n / (8 * kGvUnroll), 1), 4096);
+    double best = 0.0;
+    for (int64_t k = 1; k <= most; ++k) {
+      const int64_t w = p.row_tiles * k;
+      const double full = (double)w / (double)(kGvCus * ((w + kGvCus - 1) / kGvCus));
+      if (full > best) best = full, ks = k;
+      if ((w >= kGvBusy && w <= kGvCus) || (w > kGvCus && full >= 0.9)) {
+        ks = k;
+        break;
+      }
+    }
+  }
   if (ks < 1) ks = 1;
-  if (ks > 65535) ks = 65535;
   p.slab_cols = (n + ks - 1) / ks;
   p.slabs = (n + p.slab_cols - 1) / p.slab_cols;
   return p;
 }
 
-template <bool VEC2, bool STREAM>
-__global__ __launch_bounds__(kBlock) void dgemv_partial_kernel(
-    int64_t m, int64_t n, const double* __restrict__ A, int64_t lda,
-    const double* __restrict__ x, int64_t slab_cols, double* __restrict__ out,
-    const int32_t* __restrict__ skip) {
+// ROWS = 2: the lane holds rows b and b + 1; the last lane of an odd m holds
+// m - 2 and m - 1, so no load leaves the matrix.  ROWS = 1 (m == 1): one row.
+template <int RL, int NW, int ROWS, bool STREAM>
+__global__ __launch_bounds__(NW* kWave) void dgemv_partial_kernel(int64_t m, int64_t n, const double* __restrict__ A,
+                                                                  int64_t lda, const double* __restrict__ x,
+                                                                  int64_t slab_cols, double* __restrict__ out,
+                                                                  const int32_t* __restrict__ skip) {
   if (skip != nullptr && *skip != 0) return;
-  __shared__ double red[kBlock / kWave][kGvRows];
+  constexpr int CG = kWave / RL;  // lane groups: column pairs side by side
+  constexpr int U = kGvUnroll;
+  constexpr int R = 2 * RL;
+  __shared__ double red[NW][R];
   const int lane = threadIdx.x & (kWave - 1);
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const int64_t panel = (int64_t)blockIdx.x * kGvRows;
-  const int64_t row = panel + 2 * lane;
+  const int rl = lane % RL;
+  const int g = CG == 1 ? 0 : lane / RL;
+  const int64_t panel = (int64_t)blockIdx.x * R;
+  const int64_t row = panel + 2 * rl;
+  const int64_t b = ROWS == 2 ? (row < m - 2 ? row : m - 2) : 0;
   const int64_t c0 = (int64_t)blockIdx.y * slab_cols;
-  const int64_t c1 = (c0 + slab_cols < n) ? c0 + slab_cols : n;
-  const int64_t qlen = (slab_cols + 3) / 4;
-  const int64_t j0 = (c0 + w * qlen < c1) ? c0 + w * qlen : c1;
-  const int64_t j1 = (j0 + qlen < c1) ? j0 + qlen : c1;
+  const int64_t c1 = c0 + slab_cols < n ? c0 + slab_cols : n;
+  // the wave's columns: a whole number of pairs per lane group
+  const int64_t share = ((slab_cols + NW - 1) / NW + 2 * CG - 1) / (2 * CG) * (2 * CG);
+  const int64_t j0 = c0 + w * share < c1 ? c0 + w * share : c1;
+  const int64_t j1 = j0 + share < c1 ? j0 + share : c1;
+  auto load = [](const double* p) {
+    if constexpr (ROWS == 2) {
+      return gv_load2<STREAM>(p);
+    } else {
+      const gv_f64x2 v = {*p, 0.0};
+      return v;
+    }
+  };
+  // column offset of the lane's u-th load of a round
+  auto col = [](int u) { return (u / 2) * 2 * CG + (u & 1); };
 
   double acc0 = 0.0, acc1 = 0.0;
-  if (row + 1 < m) {
-    const double* a = A + row + j0 * lda;
-    int64_t j = j0;
-    if (VEC2) {
-      for (; j + 8 <= j1; j += 8) {
-        gv_f64x2 v[8];
+  int64_t j = j0 + 2 * g;
+  const double* a = A + b + j * lda;
+  for (int64_t jw = j0; jw + U * CG <= j1; jw += U * CG) {
+    gv_f64x2 v[U];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = gv_load2<STREAM>(a + u * lda);
+    for (int u = 0; u < U; ++u) v[u] = load(a + col(u) * lda);
+    double xv[U];
+    if constexpr (CG == 1) {
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          const double xj = x[j + u];
-          acc0 = fma(v[u].x, xj, acc0);
-          acc1 = fma(v[u].y, xj, acc1);
-        }
-        a += 8 * lda;
-      }
-      for (; j < j1; ++j) {
-        const gv_f64x2 v = gv_load2<STREAM>(a);
-        const double xj = x[j];
-        acc0 = fma(v.x, xj, acc0);
-        acc1 = fma(v.y, xj, acc1);
-        a += lda;
-      }
+      for (int u = 0; u < U; ++u) xv[u] = x[jw + u];  // wave-uniform: scalar loads
     } else {
-      for (; j + 4 <= j1; j += 4) {
-        double v0[4], v1[4];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          v0[u] = gv_load1<STREAM>(a + u * lda);
-          v1[u] = gv_load1<STREAM>(a + u * lda + 1);
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const double xj = x[j + u];
-          acc0 = fma(v0[u], xj, acc0);
-          acc1 = fma(v1[u], xj, acc1);
-        }
-        a += 4 * lda;
-      }
-      for (; j < j1; ++j) {
-        const double xj = x[j];
-        acc0 = fma(gv_load1<STREAM>(a), xj, acc0);
-        acc1 = fma(gv_load1<STREAM>(a + 1), xj, acc1);
-        a += lda;
+      for (int u = 0; u < U; u += 2) {
+        const gv_f64x2 q = *reinterpret_cast<const gv_f64x2*>(x + j + col(u));
+        xv[u] = q.x;
+        xv[u + 1] = q.y;
       }
     }
-  } else if (row < m) {
-    const double* a = A + row + j0 * lda;
-    for (int64_t j = j0; j < j1; ++j) {
-      acc0 = fma(gv_load1<STREAM>(a), x[j], acc0);
-      a += lda;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      acc0 = fma(v[u].x, xv[u], acc0);
+      acc1 = fma(v[u].y, xv[u], acc1);
+    }
+    j += U * CG;
+    a += (int64_t)(U * CG) * lda;
+  }
+  {
+    // the last columns of the share, fewer than U CG: an absent column is
+    // neither loaded nor multiplied
+    gv_f64x2 v[U];
+    double xv[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const gv_f64x2 zero = {0.0, 0.0};
+      v[u] = zero;
+      xv[u] = 0.0;
+      if (j + col(u) < j1) {
+        v[u] = load(a + col(u) * lda);
+        xv[u] = x[j + col(u)];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (j + col(u) < j1) {
+        acc0 = fma(v[u].x, xv[u], acc0);
+        acc1 = fma(v[u].y, xv[u], acc1);
+      }
     }
   }
-  red[w][2 * lane] = acc0;
-  red[w][2 * lane + 1] = acc1;
+#pragma unroll
+  for (int s = RL; s < kWave; s <<= 1) {
+    acc0 += __shfl_xor(acc0, s, kWave);
+    acc1 += __shfl_xor(acc1, s, kWave);
+  }
+  if (g == 0 && row < m) {
+    // the last lane of an odd m repeats its neighbour's second row (the same
+    // value) and may begin one row before the panel
+    const int64_t k = b - panel;
+    if (k >= 0) red[w][k] = acc0;
+    if (ROWS == 2) red[w][k + 1] = acc1;
+  }
   __syncthreads();
-  if (threadIdx.x < kGvRows) {
+  if (threadIdx.x < R) {
     const int r = threadIdx.x;
     const int64_t gr = panel + r;
     if (gr < m) {
       double s = red[0][r];
 #pragma unroll
-      for (int q = 1; q < kBlock / kWave; ++q) s += red[q][r];
+      for (int q = 1; q < NW; ++q) s += red[q][r];
       out[(int64_t)blockIdx.y * m + gr] = s;
     }
   }
 }
 
+// y[i] = sum of the slab partials in slab order, eight loads in flight.
 __global__ __launch_bounds__(kBlock) void slab_sum_kernel(int64_t m, int64_t slabs,
                                                           const double* __restrict__ part,
                                                           double* __restrict__ y,
                                                           const int32_t* __restrict__ skip) {
   if (skip != nullptr && *skip != 0) return;
+  constexpr int kBatch = 8;
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < m; i += stride) {
     double s = part[i];
-    for (int64_t k = 1; k < slabs; ++k) s += part[k * m + i];
+    for (int64_t k = 1; k < slabs; k += kBatch) {
+      double v[kBatch];
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) v[u] = k + u < slabs ? part[(k + u) * m + i] : 0.0;
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u)
+        if (k + u < slabs) s += v[u];
+    }
     y[i] = s;
   }
+}
+
+template <int RL, int NW>
+void launch_gemv(const GemvPlan& p, bool stream, int64_t m, int64_t n, const double* A, int64_t lda, const double* x,
+                 double* out, const int32_t* skip, hipStream_t s) {
+  const dim3 grid((unsigned)p.row_tiles, (unsigned)p.slabs);
+  auto kern = m == 1 ? dgemv_partial_kernel<RL, NW, 1, false>
+                     : (stream ? dgemv_partial_kernel<RL, NW, 2, true> : dgemv_partial_kernel<RL, NW, 2, false>);
+  hipLaunchKernelGGL(kern, grid, dim3(NW * kWave), 0, s, m, n, A, lda, x, p.slab_cols, out, skip);
 }
 
 }  // namespace
@@ -315,13 +394,11 @@ int mplak_dgemv_f64(int64_t m, int64_t n, const double* A, int64_t lda, const do
   const size_t need = mplak_dgemv_workspace_bytes(m, n);
   if (work_bytes < need || (need > 0 && work == nullptr)) return MPLAK_ERR_WORKSPACE;
   double* out = p.slabs > 1 ? static_cast<double*>(work) : y;
-  const bool vec2 = (lda % 2 == 0) && ((reinterpret_cast<uintptr_t>(A) & 15) == 0);
-  const dim3 grid((unsigned)p.row_tiles, (unsigned)p.slabs);
   const bool stream = (double)m * (double)n * sizeof(double) > (double)kGvStreamBytes;
-  auto kern = vec2 ? (stream ? dgemv_partial_kernel<true, true> : dgemv_partial_kernel<true, false>)
-                   : (stream ? dgemv_partial_kernel<false, true> : dgemv_partial_kernel<false, false>);
-  hipLaunchKernelGGL(kern, grid, dim3(kBlock), 0, as_stream(s), m, n, A, lda, x, p.slab_cols, out,
-                     skip_if);
+  if (p.panels)
+    launch_gemv<kGvPanelLanes, kGvPanelWaves>(p, stream, m, n, A, lda, x, out, skip_if, as_stream(s));
+  else
+    launch_gemv<kGvStreamLanes, kGvStreamWaves>(p, stream, m, n, A, lda, x, out, skip_if, as_stream(s));
   int st = launch_status();
   if (st != MPLAK_OK || p.slabs == 1) return st;
   hipLaunchKernelGGL(slab_sum_kernel, dim3(elementwise_grid(m)), dim3(kBlock), 0, as_stream(s), m,
