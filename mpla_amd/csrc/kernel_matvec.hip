@@ -646,7 +646,8 @@ template <int KIND, int DIM, typename P>
 __device__ __forceinline__ void sym_mfma_pair(const double* const* __restrict__ points, int64_t off, int64_t n,
                                               double scale, const double* __restrict__ x, P* __restrict__ rows_i,
                                               P* __restrict__ rows_j, int64_t p, int64_t I, int64_t J,
-                                              float4 centre, const uint32_t* __restrict__ tmask, float* mf) {
+                                              float4 centre, const uint32_t* __restrict__ tmask, uint32_t groups,
+                                              float* mf) {
   constexpr bool FACTOR = KIND == MPLAK_KERNEL_GAUSSIAN;
   const int tid = threadIdx.x, lane = tid & (kWave - 1);
   const int w = __builtin_amdgcn_readfirstlane(tid / kWave);
@@ -705,7 +706,8 @@ __device__ __forceinline__ void sym_mfma_pair(const double* const* __restrict__ 
   uint32_t gmask[kSymGroups];
   const uint32_t* tm = tmask + p * kTmaskWords + w * kSymGroups;
 #pragma unroll
-  for (int g = 0; g < kSymGroups; ++g) gmask[g] = (uint32_t)__builtin_amdgcn_readfirstlane((int)tm[g]);
+  for (int g = 0; g < kSymGroups; ++g)
+    gmask[g] = (groups >> g) & 1u ? (uint32_t)__builtin_amdgcn_readfirstlane((int)tm[g]) : 0u;
   __syncthreads();
 
   float A[8], accR[8][4];
@@ -858,6 +860,10 @@ __device__ __forceinline__ void sym_mfma_pair(const double* const* __restrict__ 
 // level 0's plan in its own slotted layout (below), which is all the finish
 // reads.  A single plan is the case nlev = 1.
 constexpr int kMaxLevels = 3;
+// `split` workgroups share a listed pair: workgroup b takes pair b / split
+// and, of its 8 source groups, those of part b % split.  Each writes a row
+// set of its own for both tiles (slot * split + part; zero columns outside
+// its groups), which the finish adds in part order.
 struct PlanLevels {
   const uint32_t* list[kMaxLevels];
   const int64_t* count[kMaxLevels];
@@ -870,6 +876,22 @@ struct PlanLevels {
   const double* sel;
   int64_t pcap;
   int nlev;
+  int split;  // 1, 2, 4 or 8
+};
+
+// A workgroup's pair in the plan's list, its part of the pair and the bits of
+// the source groups of that part.  SPLIT = false: whole pairs, all of it
+// constant (at n = 65536 the divisions alone cost a planned FP32 product 3 %).
+template <bool SPLIT>
+struct PairPart {
+  int64_t item;
+  int split, sub;
+  uint32_t groups;
+  __device__ __forceinline__ explicit PairPart(int s)
+      : item(SPLIT ? blockIdx.x / (unsigned)s : blockIdx.x),
+        split(SPLIT ? s : 1),
+        sub(SPLIT ? (int)(blockIdx.x % (unsigned)s) : 0),
+        groups(SPLIT ? ((1u << (kSymGroups / s)) - 1u) << (sub * (kSymGroups / s)) : 0xffu) {}
 };
 
 
@@ -889,13 +911,14 @@ __device__ __forceinline__ int plan_level(const PlanLevels& lv) {
   return l;
 }
 
-template <int KIND, int DIM>
+template <int KIND, int DIM, bool SPLIT>
 __global__ __launch_bounds__(kBlock) void kmv_sym_planned_kernel(
     const double* const* __restrict__ points, int64_t off, int64_t n, double scale, const double* __restrict__ x,
     float* __restrict__ part, const PlanLevels lv, const int32_t* __restrict__ skip) {
   if (skip != nullptr && *skip != 0) return;
   const int lev = plan_level(lv);
-  if ((int64_t)blockIdx.x >= *level_pick(lv.count, lev)) return;
+  const PairPart<SPLIT> part_of(lv.split);
+  if (part_of.item >= *level_pick(lv.count, lev)) return;
   const uint32_t* __restrict__ list = level_pick(lv.list, lev);
   const float4* __restrict__ tinfo = level_pick(lv.tinfo, lev);
   const uint32_t* __restrict__ bmask = level_pick(lv.bmask, lev);
@@ -904,17 +927,19 @@ __global__ __launch_bounds__(kBlock) void kmv_sym_planned_kernel(
   static_assert((kBlock / kWave) * kSymTile <= kMfFloats, "column sums reuse the staging buffer");
   static_assert(sizeof(SymSrc<float>) * kSymGroups <= sizeof(mf), "vector-unit staging fits");
   const int32_t* __restrict__ slots = level_pick(lv.slots, lev);
-  const int64_t p = (int64_t)list[blockIdx.x];
+  const int64_t p = (int64_t)list[part_of.item];
   int64_t I, J;
   decode_pair(p, I, J);
-  float* rows_i = slot_row(part, I, J, slots[2 * p], lv.pcap);
-  float* rows_j = I != J ? slot_row(part, J, I, slots[2 * p + 1], lv.pcap) : rows_i;
+  const int64_t pcap = lv.pcap * part_of.split;
+  float* rows_i = slot_row(part, I, J, slots[2 * p] * part_of.split + part_of.sub, pcap);
+  float* rows_j = I != J ? slot_row(part, J, I, slots[2 * p + 1] * part_of.split + part_of.sub, pcap) : rows_i;
   const float4 centre = tinfo[I];
   if (centre.w != 0.0f) {
-    sym_mfma_pair<KIND, DIM, float>(points, off, n, scale, x, rows_i, rows_j, p, I, J, centre, tmask, mf);
+    sym_mfma_pair<KIND, DIM, float>(points, off, n, scale, x, rows_i, rows_j, p, I, J, centre, tmask, part_of.groups, mf);
   } else {
     sym_valu_pair<float, KIND, DIM, false, true, true, float>(points, off, n, scale, 0.0, 0.0, 0.0, x, rows_i, rows_j, p,
-                                                       bmask[p], reinterpret_cast<SymSrc<float>*>(mf), nullptr,
+                                                       bmask[p] & (0x01010101u * part_of.groups),
+                                                       reinterpret_cast<SymSrc<float>*>(mf), nullptr,
                                                        nullptr, nullptr);
   }
 }
@@ -975,7 +1000,7 @@ __device__ __forceinline__ void sym_tile64_pair(const double* const* __restrict_
                                                 double scale, const double* __restrict__ x,
                                                 double* __restrict__ rows_i, double* __restrict__ rows_j, int64_t p,
                                                 int64_t I, int64_t J, const uint32_t* __restrict__ tmask,
-                                                double* lds) {
+                                                uint32_t groups, double* lds) {
   const int tid = threadIdx.x, lane = tid & (kWave - 1);
   const int w = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int c16 = lane & 15, r4 = lane >> 4;
@@ -1015,7 +1040,8 @@ __device__ __forceinline__ void sym_tile64_pair(const double* const* __restrict_
   uint32_t gmask[kSymGroups];
   const uint32_t* tm = tmask + p * kTmaskWords + w * kSymGroups;
 #pragma unroll
-  for (int g = 0; g < kSymGroups; ++g) gmask[g] = (uint32_t)__builtin_amdgcn_readfirstlane((int)tm[g]);
+  for (int g = 0; g < kSymGroups; ++g)
+    gmask[g] = (groups >> g) & 1u ? (uint32_t)__builtin_amdgcn_readfirstlane((int)tm[g]) : 0u;
   __syncthreads();
 
   // Two passes over the source groups, each for half of the wave's target
@@ -1147,7 +1173,7 @@ __device__ __forceinline__ void sym_mfma64_pair(const double* const* __restrict_
                                                 double scale, const double* __restrict__ x,
                                                 double* __restrict__ rows_i, double* __restrict__ rows_j, int64_t p,
                                                 int64_t I, int64_t J, float4 centre,
-                                                const uint32_t* __restrict__ tmask, double* lds) {
+                                                const uint32_t* __restrict__ tmask, uint32_t groups, double* lds) {
   const int tid = threadIdx.x, lane = tid & (kWave - 1);
   const int w = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int c16 = lane & 15, r4 = lane >> 4;
@@ -1200,7 +1226,8 @@ __device__ __forceinline__ void sym_mfma64_pair(const double* const* __restrict_
   uint32_t gmask[kSymGroups];
   const uint32_t* tm = tmask + p * kTmaskWords + w * kSymGroups;
 #pragma unroll
-  for (int g = 0; g < kSymGroups; ++g) gmask[g] = (uint32_t)__builtin_amdgcn_readfirstlane((int)tm[g]);
+  for (int g = 0; g < kSymGroups; ++g)
+    gmask[g] = (groups >> g) & 1u ? (uint32_t)__builtin_amdgcn_readfirstlane((int)tm[g]) : 0u;
   __syncthreads();
 
   double tg[kSymGroups];
@@ -1295,27 +1322,29 @@ __device__ __forceinline__ void sym_mfma64_pair(const double* const* __restrict_
 
 // Four waves per SIMD (128 registers): left to itself the compiler gives the
 // Gaussian kernel, which holds both tile forms, 146 and three waves.
-template <int KIND, int DIM>
+template <int KIND, int DIM, bool SPLIT>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 4))) void kmv_sym_planned64_kernel(
     const double* const* __restrict__ points, int64_t off, int64_t n, double scale, const double* __restrict__ x,
     double* __restrict__ part, const uint32_t* __restrict__ list, const int64_t* __restrict__ count,
     const uint32_t* __restrict__ tmask, const float4* __restrict__ tinfo, const int32_t* __restrict__ slots,
-    int64_t pcap, const int32_t* __restrict__ skip) {
+    int64_t pair_pcap, int split, const int32_t* __restrict__ skip) {
   if (skip != nullptr && *skip != 0) return;
-  if ((int64_t)blockIdx.x >= *count) return;
+  const PairPart<SPLIT> part_of(split);
+  if (part_of.item >= *count) return;
   constexpr int kBufDoubles = kM64Doubles > kT64Doubles ? kM64Doubles : kT64Doubles;
   __shared__ __attribute__((aligned(16))) double buf[kBufDoubles];
-  const int64_t p = (int64_t)list[blockIdx.x];
+  const int64_t p = (int64_t)list[part_of.item];
   int64_t I, J;
   decode_pair(p, I, J);
-  double* rows_i = slot_row(part, I, J, slots[2 * p], pcap);
-  double* rows_j = I != J ? slot_row(part, J, I, slots[2 * p + 1], pcap) : rows_i;
+  const int64_t pcap = pair_pcap * part_of.split;
+  double* rows_i = slot_row(part, I, J, slots[2 * p] * part_of.split + part_of.sub, pcap);
+  double* rows_j = I != J ? slot_row(part, J, I, slots[2 * p + 1] * part_of.split + part_of.sub, pcap) : rows_i;
   // FP64 plans mark compact tiles 2, the others 1 (both take the tile screen)
   const float4 centre = tinfo[I];
   if (KIND == MPLAK_KERNEL_GAUSSIAN && centre.w == 2.0f)
-    sym_mfma64_pair<DIM>(points, off, n, scale, x, rows_i, rows_j, p, I, J, centre, tmask, buf);
+    sym_mfma64_pair<DIM>(points, off, n, scale, x, rows_i, rows_j, p, I, J, centre, tmask, part_of.groups, buf);
   else
-    sym_tile64_pair<KIND, DIM>(points, off, n, scale, x, rows_i, rows_j, p, I, J, tmask, buf);
+    sym_tile64_pair<KIND, DIM>(points, off, n, scale, x, rows_i, rows_j, p, I, J, tmask, part_of.groups, buf);
 }
 
 // y_i = sum over partner tiles P of row i's tile X of that pair's partial,
@@ -1345,6 +1374,7 @@ __global__ __launch_bounds__(kBlock) void kmv_sym_finish_kernel(
     const int32_t* __restrict__ skip, double* __restrict__ dots) {
   if (skip != nullptr && *skip != 0) return;
   const int lev = LIST ? plan_level(lv) : 0;
+  pcap *= LIST ? lv.split : 1;
   const int32_t* __restrict__ pcount = level_pick(lv.pcount, lev);
   __shared__ double red[kFinishSlices][kFinishRows];
   const int r = threadIdx.x % kFinishRows, k = threadIdx.x / kFinishRows;
@@ -1368,7 +1398,7 @@ __global__ __launch_bounds__(kBlock) void kmv_sym_finish_kernel(
     const double xi = (k == 0 && i < n) ? x[i] : 0.0;
     double s = 0.0;
     if (LIST) {
-      const int cnt = __builtin_amdgcn_readfirstlane(craw);
+      const int cnt = __builtin_amdgcn_readfirstlane(craw) * lv.split;
 #pragma unroll
       for (int u = 0; u < kFinishBatch; ++u) s += u < cnt ? v0[u] : 0.0;
       for (int q = kFinishBatch; q < cnt; q += kFinishBatch) {
@@ -1443,18 +1473,21 @@ template <typename T, int KIND, int DIM, int MODE>
 void launch_sym_dim(hipStream_t st, bool coinc, const mplak_kernel_desc* d, const SymArgs& a) {
   const int64_t nt = sym_tiles(d->row_count);
   const dim3 grid((unsigned)(nt * (nt + 1) / 2));
+  const dim3 parts((unsigned)(nt * (nt + 1) / 2 * (a.lv != nullptr ? a.lv->split : 1)));
   if constexpr (MODE == kSymPlanned && sizeof(T) == 8) {
     if (a.lv != nullptr && !coinc) {
-      hipLaunchKernelGGL((kmv_sym_planned64_kernel<KIND, DIM>), grid, dim3(kBlock), 0, st, d->points, d->row_offset,
-                         d->row_count, a.scale, a.x, a.pi, a.lv->list[0], a.lv->count[0], a.lv->tmask[0],
-                         a.lv->tinfo[0], a.lv->slots[0], a.lv->pcap, a.skip);
+      auto kern = a.lv->split > 1 ? kmv_sym_planned64_kernel<KIND, DIM, true> : kmv_sym_planned64_kernel<KIND, DIM, false>;
+      hipLaunchKernelGGL(kern, parts, dim3(kBlock), 0, st, d->points, d->row_offset, d->row_count, a.scale, a.x, a.pi,
+                         a.lv->list[0], a.lv->count[0], a.lv->tmask[0], a.lv->tinfo[0], a.lv->slots[0], a.lv->pcap,
+                         a.lv->split, a.skip);
       return;
     }
   }
   if constexpr (MODE == kSymPlanned && sizeof(T) == 4) {
     if (a.lv != nullptr && !coinc) {
-      hipLaunchKernelGGL((kmv_sym_planned_kernel<KIND, DIM>), grid, dim3(kBlock), 0, st, d->points, d->row_offset,
-                         d->row_count, a.scale, a.x, reinterpret_cast<float*>(a.pi), *a.lv, a.skip);
+      auto kern = a.lv->split > 1 ? kmv_sym_planned_kernel<KIND, DIM, true> : kmv_sym_planned_kernel<KIND, DIM, false>;
+      hipLaunchKernelGGL(kern, parts, dim3(kBlock), 0, st, d->points, d->row_offset, d->row_count, a.scale, a.x,
+                         reinterpret_cast<float*>(a.pi), *a.lv, a.skip);
       return;
     }
   }
@@ -1498,6 +1531,23 @@ bool sym_eligible(const mplak_kernel_desc* d) {
          sym_tiles(d->row_count) < 65536;  // pair count fits a 1-D grid
 }
 
+// Workgroups per listed pair of a planned product: the largest power of two
+// up to 8 that keeps tile pairs times workgroups below 2400.  A workgroup
+// walks its pair's 16 x 16 tiles one after the other, so with few pairs the
+// launch takes as long as one whole pair (33 us at n = 4096, 36 pairs) on a
+// chip that is mostly idle.  Measured over whole mixed solves, per operator
+// application at 1 / 2 / 4 / 8 workgroups a pair: 2-D Matern n = 4096 42.9 /
+// 28.6 / 21.4 / 19.3 us, 3-D Gaussian n = 12000 42.9 / 30.7 / 27.5 / 29.8 us,
+// n = 24576 35.2 / 33.0 / 36.6 / 47.3 us; from 2400 pairs on (n > 35000) the
+// extra staging and row sets cost more than the balance gives (n = 49152 50.6
+// / 55.8 us).
+inline int sym_split(int64_t nt) {
+  const int64_t np = nt * (nt + 1) / 2;
+  int k = 1;
+  while (k < kSymGroups && np * (2 * k) < 2400) k *= 2;
+  return k;
+}
+
 size_t sym_workspace_bytes(int64_t n) {
   const int64_t nt = sym_tiles(n);
   return (size_t)2 * (size_t)(nt * (nt + 1) / 2) * kSymTile * sizeof(double);
@@ -1506,11 +1556,13 @@ size_t sym_workspace_bytes(int64_t n) {
 // Symmetric product: tile-pair kernel (exact, screened or planned) and the
 // finish.  `work` holds part_i then part_j ([pairs][512] doubles each).
 // Planned: `lv` holds the plan(s); more than one level only with FP32 tiles.
-int run_sym(const mplak_kernel_desc* d, int precision, int mode, double drop_s, const PlanLevels* lv, int64_t pcap,
+int run_sym(const mplak_kernel_desc* d, int precision, int mode, double drop_s, PlanLevels* lv, int64_t pcap,
             const double* x, double* y, void* work, const int32_t* skip_if, mplak_stream_t s,
             double* dots = nullptr) {
   SymArgs a;
   const bool coinc = d->coincident_shift != 0.0;
+  // the vector-unit kernel a coincidence shift takes works on whole pairs
+  if (lv != nullptr) lv->split = coinc ? 1 : sym_split(sym_tiles(d->row_count));
   // planned FP32 without coincidence shift: the planned kernel, FP32 partials
   const bool tiles = mode == kSymPlanned && precision == MPLAK_PREC_F32 && lv != nullptr && !coinc;
   // planned FP64 without coincidence shift: the FP64 tile form
@@ -1611,7 +1663,7 @@ PlanLayout plan_layout(int64_t n) {
   L.slots = L.pcount + align_up(sizeof(int32_t) * kFinishSlices * (size_t)nt, 256);
   L.part = L.slots + align_up(sizeof(int32_t) * 2 * np, 256);
   // partial rows: by pair (2 per pair) without a plan, slotted with one
-  const size_t rows = std::max((size_t)2 * np, (size_t)nt * kFinishSlices * (size_t)L.pcap);
+  const size_t rows = std::max((size_t)2 * np, (size_t)nt * kFinishSlices * (size_t)(L.pcap * sym_split(nt)));
   L.total = L.part + rows * kSymTile * sizeof(double);
   return L;
 }

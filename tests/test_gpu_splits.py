@@ -44,3 +44,45 @@ def test_dgemv_panels_slabs_and_strides(lib, m, n, lda, shift):
     # a sum of n products in any order: at most n roundings of a partial sum
     assert np.all(np.abs(got[:m] - Af @ xl) <= (n + 1) * EPS * (np.abs(Af) @ np.abs(xl)))
     assert got[m] == 7.0
+
+
+# Planned products share a tile pair between 8, 4, 2 and 1 workgroups, by the
+# number of 512-point tiles (16, 24, 48 and more); one tile, a ragged last
+# tile, unordered points (the vector-unit form) and ordered ones.
+@pytest.mark.parametrize("n", [1, 511, 513, 4097, 8192, 8193, 12288, 17000, 25088])
+@pytest.mark.parametrize("kind,dim,ordered", [(0, 3, True), (1, 2, True), (0, 2, False), (1, 3, False)])
+def test_planned_product_pair_splits(lib, n, kind, dim, ordered):
+    import ctypes as C
+
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(n + 10 * dim + kind)
+    P = torch.rand((dim, n), generator=g, dtype=torch.float64, device="cuda")
+    x = torch.rand(n, generator=g, dtype=torch.float64, device="cuda") - 0.5
+    table = torch.tensor([P[d].data_ptr() for d in range(dim)], dtype=torch.int64, device="cuda")
+    if ordered:
+        perm = torch.empty(n, dtype=torch.int64, device="cuda")
+        ob = lib.mplak_spatial_order_workspace_bytes(n, dim)
+        ow = workspace(ob)
+        ck(lib.mplak_spatial_order(table.data_ptr(), dim, 0, n, perm.data_ptr(), ow.data_ptr(), ob, stream()))
+        P = P[:, perm].contiguous()
+        table = torch.tensor([P[d].data_ptr() for d in range(dim)], dtype=torch.int64, device="cuda")
+    ell, nugget = (0.05, 0.1)[kind], 0.75
+    desc = _native.mplak_kernel_desc(table.data_ptr(), dim, kind, ell, nugget, 0.0, 0, n, 0, n)
+    ref, mag = torch.empty_like(x), torch.empty_like(x)
+    for i in range(0, n, 4096):
+        s = sum((P[d, i:i + 4096, None] - P[d][None, :]) ** 2 for d in range(dim))
+        r = (3.0 * s).sqrt() / ell
+        k = (-0.5 * s / ell ** 2).exp() if kind == 0 else (1.0 + r) * (-r).exp()
+        ref[i:i + 4096], mag[i:i + 4096] = k @ x, k @ x.abs()
+    ref += nugget * x
+    mag = host(mag + nugget * x.abs())
+    y = torch.empty_like(x)
+    pb = lib.mplak_screen_plan_bytes(C.byref(desc))
+    plan = workspace(pb)
+    # dropped entries are below 2^-60 (FP64) and 2^-30 (FP32) and number at most n per row; kept ones carry the
+    # entry error of their precision (FP32 2e-5 of the row's sum of magnitudes, FP64 1e-12: the oracle's bars)
+    for prec, drop, bar in ((_native.MPLAK_PREC_F64, 60.0, 1e-12), (_native.MPLAK_PREC_F32, 30.0, 2e-5)):
+        ck(lib.mplak_screen_plan_build(C.byref(desc), prec, drop, plan.data_ptr(), pb, stream()))
+        ck(lib.mplak_kernel_matvec_planned(C.byref(desc), prec, drop, plan.data_ptr(), pb, x.data_ptr(), y.data_ptr(),
+                                           None, stream()))
+        assert np.all(np.abs(host(y) - host(ref)) <= bar * mag + 0.5 * n * 2.0 ** -drop)
