@@ -1,9 +1,9 @@
 // Multi-right-hand-side kernel-matrix products Y = K V (V is N x R) on gfx950.
 //
 // No counterpart in the reference (its only product is single-vector,
-// src/kernel.cu:87-171).  Two kernels:
+// src/kernel.cu:87-171).  Three kernels:
 //
-// * VALU kernel (FP64, and FP32 for narrow V): one target per thread, a tile
+// * VALU kernel (FP64 and FP32 for narrow V): one target per thread, a tile
 //   of RT columns of V accumulated per thread, sources streamed through LDS.
 //   Each kernel entry is computed once per column tile.
 //
@@ -18,9 +18,12 @@
 //   three leading products (K_hi V_hi + K_hi V_lo + K_lo V_hi).  FP32 uses
 //   v_mfma_f32_32x32x2_f32 with eight K=2 products per step.
 //
-// Both kernels split the sources into slabs (FP32 accumulation within a slab,
-// FP64 partials per slab) and a finish kernel sums the slabs in order and adds
-// the nugget term: deterministic for a given shape.
+// * FP64 MFMA kernel (FP64, wide V): below.
+//
+// All split the sources into slabs (accumulation within a slab in FP64 for
+// FP64 entries, in FP32 on the matrix cores otherwise) and a finish kernel
+// adds the slabs' partials in FP64, in slab order, with the nugget term:
+// deterministic for a given shape.
 
 #include <math.h>
 
@@ -55,6 +58,31 @@ inline Slabs slab_plan(int64_t rows, int64_t cols, int tile_rows, int64_t col_ti
   const int64_t per = (chunks + ks - 1) / ks;
   p.slab_cols = per * kChunk;
   p.slabs = (cols + p.slab_cols - 1) / p.slab_cols;
+  return p;
+}
+
+// Split of the sources for a kernel that has `slots` workgroups resident at a
+// time: the slab count (of whole chunks) that minimises rounds of workgroups x
+// slab length, with 1 % of the product charged per slab for its partials
+// (written and read back once each).
+inline Slabs balanced_slabs(int64_t rows, int64_t cols, int tile_rows, int chunk, int64_t slots) {
+  Slabs p;
+  p.tiles = (rows + tile_rows - 1) / tile_rows;
+  const int64_t chunks = (cols + chunk - 1) / chunk;
+  const int64_t most = std::min<int64_t>(chunks, std::max<int64_t>(4 * slots / p.tiles, 1));
+  double best = 0.0;
+  for (int64_t ks = 1; ks <= most; ++ks) {
+    const int64_t per = (chunks + ks - 1) / ks;
+    const int64_t slabs = (chunks + per - 1) / per;
+    const int64_t rounds = (p.tiles * slabs + slots - 1) / slots;
+    const double ideal = (double)(p.tiles * chunks) / (double)slots;
+    const double cost = (double)(rounds * per) + 0.01 * (double)slabs * std::max(ideal, 1.0);
+    if (ks == 1 || cost < best) {
+      best = cost;
+      p.slabs = slabs;
+      p.slab_cols = per * chunk;
+    }
+  }
   return p;
 }
 
@@ -325,6 +353,127 @@ __global__ __launch_bounds__(kBlock) void mrhs_mfma_kernel(
     }
 }
 
+// ---------------------------------------------------------------------------
+// FP64 matrix-core kernel (MPLAK_PREC_F64, kMfma64MinR columns or more, dim <= 4).
+//
+// A wave owns 32 targets (two 16-row blocks) and all columns of a group of up
+// to 64.  For every step of 4 sources a lane evaluates one entry per row block
+// in FP64 (coordinate differences and the table exponential, as on the vector
+// unit), directly in the A layout of v_mfma_f64_16x16x4_f64, and the matrix
+// cores contract it with the step's V operands from LDS.  Each entry is
+// evaluated once whatever R (the vector-unit form evaluates it once per 16
+// columns and reads every V value of the tile from LDS per source).  The FP64
+// matrix rate equals the vector FMA rate on gfx950 and the two do not overlap
+// (per 16 columns 224 us at n = 20001, 3-D Gaussian, of which 163 us are the
+// products at 78.6 TFLOP/s, on top of 270 us for the entries), so the gain is
+// the entries and LDS reads saved.
+//
+// Row 4 v + r of A takes target 4 r + v of the block, so result v of lane
+// 16 r + c is target 4 r + v, column c, and a lane's four results are
+// consecutive rows of the partials.
+
+constexpr int kSrc64 = 64;                                 // sources per LDS chunk
+constexpr int kTile64 = 32 * (kBlock / kWave);             // 128 targets per workgroup
+constexpr int kSteps64 = kSrc64 / 4;
+// resident waves per SIMD (and workgroups per CU) by column blocks
+constexpr int waves64(int cblocks) { return cblocks <= 2 ? 4 : 3; }
+
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+typedef double f64x2u __attribute__((ext_vector_type(2), aligned(8)));
+
+template <int KIND, int DIM, int CB>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(waves64(CB), waves64(CB)))) void mrhs_mfma64_kernel(
+    const double* const* __restrict__ points, int64_t row_off, int64_t rows, int64_t col_off, int64_t cols,
+    int64_t slab_cols, double scale, int64_t R, const double* __restrict__ V, int64_t ldv, double* __restrict__ part,
+    const int32_t* __restrict__ skip) {
+  if (skip != nullptr && *skip != 0) return;
+  // V operands of a step: CB blocks of 64 lanes (source k = lane / 16, column
+  // lane % 16); two doubles of padding spread the staging writes over the banks
+  constexpr int kStep = CB * kWave + 2;
+  __shared__ double lv[kSteps64 * kStep];
+  __shared__ double lp[DIM][kSrc64];
+  __shared__ double tab[kExp2Table];
+  fill_exp2_table(tab);  // first read after the chunk barrier below
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), w = tid / kWave;
+  const int c16 = lane & 15, r4 = lane >> 4;
+  const int64_t base = (int64_t)blockIdx.x * kTile64 + w * 32;
+
+  double p[2][DIM];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    int64_t i = base + 16 * h + 4 * (c16 & 3) + (c16 >> 2);
+    if (i >= rows) i = rows - 1;
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) p[h][d] = points[d][row_off + i] * scale;
+  }
+  f64x4 acc[2][CB];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int c = 0; c < CB; ++c) acc[h][c] = f64x4{0.0, 0.0, 0.0, 0.0};
+
+  const int64_t c0 = (int64_t)blockIdx.y * slab_cols;
+  const int64_t c1 = c0 + slab_cols < cols ? c0 + slab_cols : cols;
+  for (int64_t cb = c0; cb < c1; cb += kSrc64) {
+    // lane = source, wave w takes columns w, w + 4, ...: all loads before the
+    // barrier, sources and columns past the end are zero
+    const int64_t j = cb + lane;
+    double v[CB * 4], q = 0.0;
+#pragma unroll
+    for (int u = 0; u < CB * 4; ++u) {
+      const int col = 4 * u + w;
+      v[u] = j < c1 && col < R ? V[col * ldv + j] : 0.0;
+    }
+    if (w < DIM && j < c1) q = points[w][col_off + j] * scale;
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < CB * 4; ++u) {
+      const int col = 4 * u + w;
+      lv[(lane / 4) * kStep + (col / 16) * kWave + (lane % 4) * 16 + col % 16] = v[u];
+    }
+    if (w < DIM) lp[w][lane] = q;
+    __syncthreads();
+#pragma unroll 2
+    for (int st = 0; st < kSteps64; ++st) {
+      double e[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        double s = 0.0;
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) {
+          const double df = p[h][d] - lp[d][4 * st + r4];
+          s = d == 0 ? df * df : fma(df, df, s);
+        }
+        e[h] = kernel_entry<double, KIND>(s, tab);
+      }
+#pragma unroll
+      for (int c = 0; c < CB; ++c) {
+        const double b = lv[st * kStep + c * kWave + lane];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) acc[h][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(e[h], b, acc[h][c], 0, 0, 0);
+      }
+    }
+  }
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int c = 0; c < CB; ++c) {
+      const int64_t r = 16 * c + c16;
+      if (r >= R) continue;
+      const int64_t i = base + 16 * h + 4 * r4;
+      double* out = part + ((int64_t)blockIdx.y * R + r) * rows + i;
+      const f64x2u lo = {acc[h][c][0], acc[h][c][1]}, hi = {acc[h][c][2], acc[h][c][3]};
+      if (i + 4 <= rows) {
+        *reinterpret_cast<f64x2u*>(out) = lo;
+        *reinterpret_cast<f64x2u*>(out + 2) = hi;
+      } else {
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+          if (i + v < rows) out[v] = acc[h][c][v];
+      }
+    }
+}
+
 // Y[i + r ldy] = sum over slabs (slab order) + nugget * V at the global diagonal.
 __global__ __launch_bounds__(kBlock) void mrhs_finish_kernel(int64_t rows, int64_t R, int64_t slabs,
                                                              const double* __restrict__ part, int64_t row_off,
@@ -348,9 +497,17 @@ __global__ __launch_bounds__(kBlock) void mrhs_finish_kernel(int64_t rows, int64
 // ---------------------------------------------------------------------------
 // host-side planning and dispatch
 
+// Fewest columns of the FP64 matrix-core kernel.  Its products are 16 columns
+// wide, so up to 8 columns the vector unit's narrower tiles do less work
+// (n = 20001, 3-D Gaussian, R = 8: 402 us against 488 us); from 9 the vector
+// unit works on 16 as well (R = 12: 611 us against 493 us, R = 64: 2443 us
+// against 1169 us; Matern R = 64: 3141 us against 1438 us).
+constexpr int64_t kMfma64MinR = 9;
+
 struct MrhsPlan {
   bool mfma;
   int mode;       // MfmaMode when mfma
+  bool mfma64;    // FP64 matrix-core kernel
   int rt;         // VALU column tile
   int64_t cblocks;
   Slabs s;
@@ -368,6 +525,13 @@ inline int valu_rt(int64_t R) {
 
 inline MrhsPlan make_plan(const mplak_kernel_desc* d, int precision, int64_t R) {
   MrhsPlan p{};
+  if (precision == MPLAK_PREC_F64 && R >= kMfma64MinR && d->dim <= 4) {
+    p.mfma64 = true;
+    p.cblocks = (R + 15) / 16;
+    p.s = balanced_slabs(d->row_count, d->col_count, kTile64, kSrc64, 256 * waves64((int)std::min<int64_t>(p.cblocks, 4)));
+    p.part_bytes = align_up((size_t)p.s.slabs * (size_t)R * (size_t)d->row_count * sizeof(double), 256);
+    return p;
+  }
   const bool wide = R >= 16;
   p.mfma = (precision == MPLAK_PREC_BF16 || precision == MPLAK_PREC_BF16X3 ||
             (precision == MPLAK_PREC_F32 && wide)) && d->dim <= 4;
@@ -388,6 +552,12 @@ inline MrhsPlan make_plan(const mplak_kernel_desc* d, int precision, int64_t R) 
   }
   p.part_bytes = align_up((size_t)p.s.slabs * (size_t)R * (size_t)d->row_count * sizeof(double), 256);
   return p;
+}
+
+// Columns per launch: the matrix-core kernels hold at most kMfmaGroup.
+inline int64_t column_group(const mplak_kernel_desc* d, int precision, int64_t nrhs) {
+  const MrhsPlan p = make_plan(d, precision, nrhs);
+  return p.mfma || p.mfma64 ? kMfmaGroup : nrhs;
 }
 
 template <typename T, int KIND, int DIM>
@@ -448,6 +618,31 @@ void launch_mfma_mode(const mplak_kernel_desc* d, const MrhsPlan& p, hipStream_t
 }
 
 template <int KIND>
+void launch_mfma64(const mplak_kernel_desc* d, const MrhsPlan& p, hipStream_t st, double scale, int64_t R,
+                   const double* V, int64_t ldv, double* part, const int32_t* skip) {
+  const dim3 grid((unsigned)p.s.tiles, (unsigned)p.s.slabs);
+  auto go = [&](auto cb_tag, auto dim_tag) {
+    constexpr int CBV = decltype(cb_tag)::value, DIMV = decltype(dim_tag)::value;
+    hipLaunchKernelGGL((mrhs_mfma64_kernel<KIND, DIMV, CBV>), grid, dim3(kBlock), 0, st, d->points, d->row_offset,
+                       d->row_count, d->col_offset, d->col_count, p.s.slab_cols, scale, R, V, ldv, part, skip);
+  };
+  auto with_dim = [&](auto cb_tag) {
+    switch (d->dim) {
+      case 1: go(cb_tag, std::integral_constant<int, 1>{}); break;
+      case 2: go(cb_tag, std::integral_constant<int, 2>{}); break;
+      case 3: go(cb_tag, std::integral_constant<int, 3>{}); break;
+      default: go(cb_tag, std::integral_constant<int, 4>{}); break;
+    }
+  };
+  switch (p.cblocks) {
+    case 1: with_dim(std::integral_constant<int, 1>{}); break;
+    case 2: with_dim(std::integral_constant<int, 2>{}); break;
+    case 3: with_dim(std::integral_constant<int, 3>{}); break;
+    default: with_dim(std::integral_constant<int, 4>{}); break;
+  }
+}
+
+template <int KIND>
 void launch_mfma(const mplak_kernel_desc* d, const MrhsPlan& p, hipStream_t st, double scale, int64_t R,
                  const void* vpk, double* part, const int32_t* skip) {
   if (p.mode == kModeBf16)
@@ -476,10 +671,16 @@ extern "C" {
 
 size_t mplak_kernel_mrhs_workspace_bytes(const mplak_kernel_desc* d, int precision, int64_t nrhs) {
   if (check_desc(d) != MPLAK_OK || nrhs <= 0 || d->row_count <= 0 || d->col_count <= 0) return 0;
-  // the MFMA path works on groups of at most kMfmaGroup columns
-  const MrhsPlan p = make_plan(d, precision, nrhs);
-  const MrhsPlan g = p.mfma ? make_plan(d, precision, std::min<int64_t>(nrhs, kMfmaGroup)) : p;
-  return g.vpk_bytes + g.part_bytes;
+  // the MFMA paths work on groups of at most kMfmaGroup columns; a narrow
+  // last group may take another kernel (and slab count) than the full ones
+  const int64_t group = column_group(d, precision, nrhs);
+  const MrhsPlan p = make_plan(d, precision, std::min(nrhs, group));
+  size_t bytes = p.vpk_bytes + p.part_bytes;
+  if (nrhs > group && nrhs % group != 0) {
+    const MrhsPlan q = make_plan(d, precision, nrhs % group);
+    bytes = std::max(bytes, q.vpk_bytes + q.part_bytes);
+  }
+  return bytes;
 }
 
 int mplak_kernel_mrhs(const mplak_kernel_desc* d, int precision, int64_t nrhs, const double* V, int64_t ldv,
@@ -502,8 +703,7 @@ int mplak_kernel_mrhs(const mplak_kernel_desc* d, int precision, int64_t nrhs, c
   if (work == nullptr || work_bytes < mplak_kernel_mrhs_workspace_bytes(d, precision, nrhs)) return MPLAK_ERR_WORKSPACE;
   hipStream_t hs = as_stream(s);
   const double scale = coord_scale(d->kind, d->length_scale);
-  const MrhsPlan whole = make_plan(d, precision, nrhs);
-  const int64_t group = whole.mfma ? kMfmaGroup : nrhs;
+  const int64_t group = column_group(d, precision, nrhs);
   for (int64_t r0 = 0; r0 < nrhs; r0 += group) {
     const int64_t R = std::min(group, nrhs - r0);
     const MrhsPlan p = make_plan(d, precision, R);
@@ -523,6 +723,11 @@ int mplak_kernel_mrhs(const mplak_kernel_desc* d, int precision, int64_t nrhs, c
         launch_mfma<MPLAK_KERNEL_GAUSSIAN>(d, p, hs, scale, R, w, part, skip_if);
       else
         launch_mfma<MPLAK_KERNEL_MATERN32>(d, p, hs, scale, R, w, part, skip_if);
+    } else if (p.mfma64) {
+      if (d->kind == MPLAK_KERNEL_GAUSSIAN)
+        launch_mfma64<MPLAK_KERNEL_GAUSSIAN>(d, p, hs, scale, R, Vg, ldv, part, skip_if);
+      else
+        launch_mfma64<MPLAK_KERNEL_MATERN32>(d, p, hs, scale, R, Vg, ldv, part, skip_if);
     } else {
       if (precision == MPLAK_PREC_F64) {
         if (d->kind == MPLAK_KERNEL_GAUSSIAN)

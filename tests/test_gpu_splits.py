@@ -86,3 +86,39 @@ def test_planned_product_pair_splits(lib, n, kind, dim, ordered):
         ck(lib.mplak_kernel_matvec_planned(C.byref(desc), prec, drop, plan.data_ptr(), pb, x.data_ptr(), y.data_ptr(),
                                            None, stream()))
         assert np.all(np.abs(host(y) - host(ref)) <= bar * mag + 0.5 * n * 2.0 ** -drop)
+
+
+# FP64 multi-right-hand-side products on the matrix cores (from 9 columns):
+# rows around the 16-row blocks and 128-row tiles, columns around the 16- and
+# 64-column blocks, sources around the 64-point chunks, blocks off the diagonal,
+# padded leading dimensions; 8 columns and 5 dimensions take the vector unit.
+@pytest.mark.parametrize("rows,cols,row_off,R,dim", [
+    (1, 1, 0, 9, 1), (15, 63, 3, 16, 2), (17, 65, 0, 17, 3), (127, 64, 0, 33, 4), (128, 130, 5, 48, 3),
+    (129, 129, 0, 64, 2), (1000, 517, 100, 65, 3), (700, 1500, 0, 73, 2), (300, 300, 0, 8, 3), (300, 300, 0, 20, 5)])
+@pytest.mark.parametrize("kind", [0, 1])
+def test_mrhs_f64_tiles(lib, rows, cols, row_off, R, dim, kind):
+    import ctypes as C
+
+    import torch
+    rng = np.random.default_rng(rows + cols + R)
+    n = max(cols, row_off + rows)
+    P = rng.random((dim, n))
+    ell, nugget = (0.3, 0.4)[kind], 0.7
+    ldv, ldy = cols + 3, rows + 5
+    V = rng.standard_normal((R, ldv))
+    s = sum((P[d, row_off:row_off + rows, None] - P[d, None, :cols]) ** 2 for d in range(dim))
+    r = np.sqrt(3.0 * s) / ell
+    K = np.exp(-0.5 * s / ell ** 2) if kind == 0 else (1.0 + r) * np.exp(-r)
+    K[np.arange(row_off, row_off + rows)[:, None] == np.arange(cols)[None, :]] += nugget
+    P_dev, V_dev = dev(P), dev(V)
+    Y = torch.full((R, ldy), 7.0, dtype=torch.float64, device="cuda")
+    table = torch.tensor([P_dev[d].data_ptr() for d in range(dim)], dtype=torch.int64, device="cuda")
+    desc = _native.mplak_kernel_desc(table.data_ptr(), dim, kind, ell, nugget, 0.0, row_off, rows, 0, cols)
+    wb = lib.mplak_kernel_mrhs_workspace_bytes(C.byref(desc), _native.MPLAK_PREC_F64, R)
+    w = workspace(wb)
+    ck(lib.mplak_kernel_mrhs(C.byref(desc), _native.MPLAK_PREC_F64, R, V_dev.data_ptr(), ldv, Y.data_ptr(), ldy,
+                             w.data_ptr(), wb, None, stream()))
+    got = host(Y)
+    # the oracle's FP64 bar: 1e-12 of the sum of magnitudes
+    assert np.all(np.abs(got[:, :rows] - V[:, :cols] @ K.T) <= 1e-12 * (np.abs(V[:, :cols]) @ K.T))
+    assert np.all(got[:, rows:] == 7.0)
