@@ -41,7 +41,10 @@ constexpr int kMaxDim = 16;
 constexpr int kTargetBlocks = 2048;
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 
 struct Slabs {
   int64_t tiles, slabs, slab_cols;
@@ -61,22 +64,27 @@ inline Slabs slab_plan(int64_t rows, int64_t cols, int tile_rows, int64_t col_ti
   return p;
 }
 
-// Split of the sources for a kernel that has `slots` workgroups resident at a
-// time: the slab count (of whole chunks) that minimises rounds of workgroups x
-// slab length, with 1 % of the product charged per slab for its partials
-// (written and read back once each).
-inline Slabs balanced_slabs(int64_t rows, int64_t cols, int tile_rows, int chunk, int64_t slots) {
+// Split of the sources for a matrix-core kernel with `occ` workgroups resident
+// per CU: the slab count (of whole chunks of 64 sources) that minimises, in
+// units of one workgroup's chunk on a full CU, the chunks of the busiest CU
+// plus the slabs' partials, written and read back once each.  A CU with fewer
+// than `occ` workgroups takes a chunk down to a quarter of that time.  Measured:
+// partials 4 TB/s, against 8 us for a 64-column BF16x3 chunk and 18 us for an
+// FP64 one (n = 20001, 64 columns in FP64: 1.44 ms in 8 slabs, five workgroups
+// on the busiest CU; 1.66 ms in 4, three).
+inline Slabs balanced_slabs(int64_t rows, int64_t cols, int tile_rows, int chunk, int occ, int64_t R) {
+  constexpr int64_t kCus = 256;
   Slabs p;
   p.tiles = (rows + tile_rows - 1) / tile_rows;
   const int64_t chunks = (cols + chunk - 1) / chunk;
-  const int64_t most = std::min<int64_t>(chunks, std::max<int64_t>(4 * slots / p.tiles, 1));
+  const int64_t most = std::min<int64_t>(chunks, std::max<int64_t>(4 * kCus * occ / p.tiles, 1));
+  const double slab_cost = 2.4e-7 * (double)rows * (double)R;
   double best = 0.0;
   for (int64_t ks = 1; ks <= most; ++ks) {
     const int64_t per = (chunks + ks - 1) / ks;
     const int64_t slabs = (chunks + per - 1) / per;
-    const int64_t rounds = (p.tiles * slabs + slots - 1) / slots;
-    const double ideal = (double)(p.tiles * chunks) / (double)slots;
-    const double cost = (double)(rounds * per) + 0.01 * (double)slabs * std::max(ideal, 1.0);
+    const double m = (double)((p.tiles * slabs + kCus - 1) / kCus) / occ;  // of the busiest CU, in full CUs
+    const double cost = (double)per * (m >= 1.0 ? m : 0.25 + 0.75 * m) + slab_cost * (double)slabs;
     if (ks == 1 || cost < best) {
       best = cost;
       p.slabs = slabs;
@@ -152,48 +160,80 @@ __global__ __launch_bounds__(kBlock) void mrhs_valu_kernel(
 // ---------------------------------------------------------------------------
 // MFMA kernel.
 //
-// Packed V (built by pack_v_kernel), per 16-source step s and 32-column block
-// cb, 64 lanes x one operand each:
-//   BF16 / BF16X3 : 8 bf16 per lane, lane l holds V[16 s + 8 (l/32) + t][32 cb + l%32]
-//   FP32          : 8 floats per lane, lane l holds V[16 s + 2 t + l/32][32 cb + l%32]
-// (t = 0..7).  BF16X3 stores the hi part and then, in a second array of the
-// same size, the lo part.
+// Sources are packed once per call (pack_kernel) into blocks of 64, each the
+// image of its LDS staging:
+//   64 float4            scaled coordinates (padding: far away)
+//   BF16 / BF16X3 : per 16-source step and 32-column block 64 lanes x 8 bf16,
+//                   lane l holds V[16 s + 8 (l/32) + t][32 cb + l%32]; BF16X3
+//                   stores the hi parts of the block, then its lo parts
+//   FP32          : the same with 8 floats, V[16 s + 2 t + l/32][32 cb + l%32]
+// (t = 0..7).  A workgroup copies two blocks at a time straight into LDS and
+// its four waves read their operands from there: read from global memory by
+// every wave, the operands (4 KiB per wave and step in BF16x3) took up to 45
+// bytes a clock and CU through a 64-byte L1.
 
 enum MfmaMode { kModeBf16 = 0, kModeBf16x3 = 1, kModeF32 = 2 };
 
 constexpr int kWaveTargets = 64;                    // two 32-row MFMA blocks
 constexpr int kMfmaTile = kWaveTargets * (kBlock / kWave);  // 256 targets per workgroup
+constexpr int kMfmaSlab = 64;                       // sources per packed block
+constexpr int kMfmaStage = 2;                       // blocks in LDS at a time
+constexpr int kBlockSteps = kMfmaSlab / 16;
+constexpr size_t kPackAlign = 16;                   // the copies into LDS move aligned 16-byte words
+// resident waves per SIMD (and workgroups per CU) by 32-column blocks
+constexpr int mfma_waves(int cblocks) { return cblocks == 1 ? 5 : 4; }
 constexpr int64_t kMfmaGroup = 64;  // columns per MFMA launch (two 32-column blocks)
 
-__global__ __launch_bounds__(kBlock) void pack_v_kernel(const double* __restrict__ V, int64_t ldv, int64_t R,
-                                                        int64_t cols, int64_t steps, int64_t cblocks, int mode,
-                                                        void* __restrict__ out) {
-  // one thread per (step, cblock, lane)
-  const int64_t total = steps * cblocks * kWave;
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; g < total; g += stride) {
-    const int lane = (int)(g % kWave);
-    const int64_t sc = g / kWave;
-    const int64_t cb = sc % cblocks;
-    const int64_t s = sc / cblocks;
-    const int64_t r = cb * 32 + (lane % 32);
-    if (mode == kModeF32) {
-      float* o = static_cast<float*>(out) + g * 8;
-#pragma unroll
-      for (int t = 0; t < 8; ++t) {
-        const int64_t j = 16 * s + 2 * t + lane / 32;
-        o[t] = (j < cols && r < R) ? (float)V[r * ldv + j] : 0.0f;
+// Bytes of one step and column block, of one operand part and of a block.
+constexpr int step_bytes(int mode) { return kWave * (mode == kModeF32 ? 32 : 16); }
+constexpr int part_bytes(int mode, int cblocks) { return kBlockSteps * cblocks * step_bytes(mode); }
+constexpr int block_bytes(int mode, int cblocks) {
+  return kMfmaSlab * 16 + part_bytes(mode, cblocks) * (mode == kModeBf16x3 ? 2 : 1);
+}
+
+__global__ __launch_bounds__(kBlock) void pack_kernel(const double* const* __restrict__ points, int dim,
+                                                      int64_t col_off, double scale, const double* __restrict__ V,
+                                                      int64_t ldv, int64_t R, int64_t cols, int64_t blocks,
+                                                      int cblocks, int mode, char* __restrict__ out) {
+  // one workgroup per block; one thread per (step, cblock, lane)
+  const int64_t bytes = kMfmaSlab * 16 + (int64_t)kBlockSteps * cblocks * step_bytes(mode) * (mode == kModeBf16x3 ? 2 : 1);
+  for (int64_t b = blockIdx.x; b < blocks; b += gridDim.x) {
+    char* image = out + b * bytes;
+    char* ops = image + kMfmaSlab * 16;
+    if (threadIdx.x < kMfmaSlab) {
+      const int64_t j = b * kMfmaSlab + threadIdx.x;
+      float4 q = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (j < cols) {
+        q.x = (float)(points[0][col_off + j] * scale);
+        if (dim > 1) q.y = (float)(points[1][col_off + j] * scale);
+        if (dim > 2) q.z = (float)(points[2][col_off + j] * scale);
+        if (dim > 3) q.w = (float)(points[3][col_off + j] * scale);
+      } else {
+        q.x = 1.0e4f;  // far away: entries of padded sources underflow to 0
       }
-    } else {
-      __bf16* hi = static_cast<__bf16*>(out) + g * 8;
-      __bf16* lo = hi + total * 8;
+      reinterpret_cast<float4*>(image)[threadIdx.x] = q;
+    }
+    for (int g = threadIdx.x; g < kBlockSteps * cblocks * kWave; g += kBlock) {
+      const int lane = g % kWave, cb = (g / kWave) % cblocks, st = g / (kWave * cblocks);
+      const int64_t r = cb * 32 + (lane % 32), j0 = b * kMfmaSlab + 16 * st;
+      if (mode == kModeF32) {
+        float* o = reinterpret_cast<float*>(ops) + g * 8;
 #pragma unroll
-      for (int t = 0; t < 8; ++t) {
-        const int64_t j = 16 * s + 8 * (lane / 32) + t;
-        const float v = (j < cols && r < R) ? (float)V[r * ldv + j] : 0.0f;
-        const __bf16 h = (__bf16)v;
-        hi[t] = h;
-        if (mode == kModeBf16x3) lo[t] = (__bf16)(v - (float)h);
+        for (int t = 0; t < 8; ++t) {
+          const int64_t j = j0 + 2 * t + lane / 32;
+          o[t] = (j < cols && r < R) ? (float)V[r * ldv + j] : 0.0f;
+        }
+      } else {
+        bf16x8 hi, lo;
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+          const int64_t j = j0 + 8 * (lane / 32) + t;
+          const float v = (j < cols && r < R) ? (float)V[r * ldv + j] : 0.0f;
+          hi[t] = (__bf16)v;
+          lo[t] = (__bf16)(v - (float)hi[t]);
+        }
+        reinterpret_cast<bf16x8*>(ops)[g] = hi;
+        if (mode == kModeBf16x3) reinterpret_cast<bf16x8*>(ops)[kBlockSteps * cblocks * kWave + g] = lo;
       }
     }
   }
@@ -220,16 +260,27 @@ __device__ __forceinline__ float dist2(const float (&p)[4], const float4& q) {
   return s;
 }
 
+// 16 bytes per lane from global memory straight into LDS (the wave's lanes at
+// consecutive 16-byte slots from `lds`), counted by vmcnt.
+__device__ __forceinline__ void load_to_lds(const char* global, char* lds) {
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)global,
+                                   (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
+}
+
+// Bound by the vector unit's entry evaluation (per entry 11 instructions, one
+// square root and one exponential for Matern BF16x3) and, in BF16x3, by the
+// matrix products, which overlap it only in part.
 template <int KIND, int MODE, int CB, int DIM>
-__global__ __launch_bounds__(kBlock) void mrhs_mfma_kernel(
-    const double* const* __restrict__ points, int dim, int64_t row_off, int64_t rows, int64_t col_off,
-    int64_t cols, int64_t slab_cols, double scale, int64_t R, const void* __restrict__ vpk, int64_t vpk_total,
-    double* __restrict__ part, const int32_t* __restrict__ skip) {
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(mfma_waves(CB), mfma_waves(CB)))) void
+mrhs_mfma_kernel(const double* const* __restrict__ points, int64_t row_off, int64_t rows, int64_t blocks,
+                 int64_t slab_blocks, double scale, int64_t R, const char* __restrict__ packed,
+                 float* __restrict__ part, const int32_t* __restrict__ skip) {
   if (skip != nullptr && *skip != 0) return;
-  __shared__ float4 lp[kChunk];  // scaled source coordinates (x, y, z, w) for dim <= 4
+  constexpr int kBytes = block_bytes(MODE, CB), kPart = part_bytes(MODE, CB);
+  __shared__ __attribute__((aligned(16))) char image[kMfmaStage * kBytes];
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
-  const int wave = tid / kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int64_t base = (int64_t)blockIdx.x * kMfmaTile + wave * kWaveTargets;
 
   // target coordinates for the two row blocks of this lane
@@ -250,57 +301,37 @@ __global__ __launch_bounds__(kBlock) void mrhs_mfma_kernel(
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[h][c][v] = 0.0f;
 
-  const int64_t c0 = (int64_t)blockIdx.y * slab_cols;
-  const int64_t c1 = (c0 + slab_cols < cols) ? c0 + slab_cols : cols;
-  for (int64_t cbase = c0; cbase < c1; cbase += kChunk) {
+  const int64_t b0 = (int64_t)blockIdx.y * slab_blocks;
+  const int64_t b1 = b0 + slab_blocks < blocks ? b0 + slab_blocks : blocks;
+  for (int64_t b = b0; b < b1; b += kMfmaStage) {
+    const int count = (int)(b1 - b < kMfmaStage ? b1 - b : kMfmaStage);
     __syncthreads();
-    {
-      const int64_t j = cbase + tid;
-      float4 q = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (j < c1) {
-        q.x = (float)(points[0][col_off + j] * scale);
-        if (DIM > 1) q.y = (float)(points[1][col_off + j] * scale);
-        if (DIM > 2) q.z = (float)(points[2][col_off + j] * scale);
-        if (DIM > 3) q.w = (float)(points[3][col_off + j] * scale);
-      } else {
-        q.x = 1.0e4f;  // far away: entries of padded sources underflow to 0
-      }
-      lp[tid] = q;
-    }
+    for (int k = wave * 1024; k < count * kBytes; k += (kBlock / kWave) * 1024)
+      load_to_lds(packed + b * kBytes + k + lane * 16, image + k);
+    // the copies of every wave are in LDS before any wave passes the barrier
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    const int64_t step0 = cbase / 16;
 #pragma unroll 1
-    for (int st = 0; st < kChunk / 16; ++st) {
-      const int64_t step = step0 + st;
+    for (int st = 0; st < count * kBlockSteps; ++st) {
+      const char* blk = image + (st / kBlockSteps) * kBytes;
+      const int s4 = st % kBlockSteps;
+      const float4* lp = reinterpret_cast<const float4*>(blk) + 16 * s4;
+      const char* ops = blk + kMfmaSlab * 16 + s4 * CB * step_bytes(MODE) + lane * (step_bytes(MODE) / kWave);
       // ---- kernel entries in A-operand layout
       float e[2][8];
-      if (MODE == kModeF32) {
 #pragma unroll
-        for (int t = 0; t < 8; ++t) {
-          const float4 q = lp[st * 16 + 2 * t + lane / 32];
+      for (int t = 0; t < 8; ++t) {
+        const float4 q = lp[MODE == kModeF32 ? 2 * t + lane / 32 : 8 * (lane / 32) + t];
 #pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            e[h][t] = kernel_entry<float, KIND>(dist2<DIM>(pa[h], q), nullptr);
-          }
-        }
-      } else {
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-          const float4 q = lp[st * 16 + 8 * (lane / 32) + t];
-#pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            e[h][t] = kernel_entry<float, KIND>(dist2<DIM>(pa[h], q), nullptr);
-          }
-        }
+        for (int h = 0; h < 2; ++h) e[h][t] = kernel_entry<float, KIND>(dist2<DIM>(pa[h], q), nullptr);
       }
       // ---- contraction with the packed V operands
       if (MODE == kModeF32) {
-        const float* vp = static_cast<const float*>(vpk);
 #pragma unroll
         for (int c = 0; c < CB; ++c) {
-          const float4* src = reinterpret_cast<const float4*>(vp + ((step * CB + c) * kWave + lane) * 8);
-          const float4 b0 = src[0], b1 = src[1];
-          const float bv[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
+          const float4* src = reinterpret_cast<const float4*>(ops + c * step_bytes(MODE));
+          const float4 b0v = src[0], b1v = src[1];
+          const float bv[8] = {b0v.x, b0v.y, b0v.z, b0v.w, b1v.x, b1v.y, b1v.z, b1v.w};
 #pragma unroll
           for (int t = 0; t < 8; ++t) {
 #pragma unroll
@@ -309,36 +340,50 @@ __global__ __launch_bounds__(kBlock) void mrhs_mfma_kernel(
           }
         }
       } else {
+        // two entries at a time: one conversion instruction per pair and part
         bf16x8 ahi[2], alo[2];
 #pragma unroll
         for (int h = 0; h < 2; ++h)
 #pragma unroll
-          for (int t = 0; t < 8; ++t) {
-            const __bf16 hb = (__bf16)e[h][t];
-            ahi[h][t] = hb;
-            if (MODE == kModeBf16x3) alo[h][t] = (__bf16)(e[h][t] - (float)hb);
-          }
-        const __bf16* vh = static_cast<const __bf16*>(vpk);
-#pragma unroll
-        for (int c = 0; c < CB; ++c) {
-          const int64_t off = ((step * CB + c) * kWave + lane) * 8;
-          const bf16x8 bhi = *reinterpret_cast<const bf16x8*>(vh + off);
-#pragma unroll
-          for (int h = 0; h < 2; ++h) acc[h][c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ahi[h], bhi, acc[h][c], 0, 0, 0);
-          if (MODE == kModeBf16x3) {
-            const bf16x8 blo = *reinterpret_cast<const bf16x8*>(vh + vpk_total * 8 + off);
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-              acc[h][c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ahi[h], blo, acc[h][c], 0, 0, 0);
-              acc[h][c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(alo[h], bhi, acc[h][c], 0, 0, 0);
+          for (int t = 0; t < 8; t += 2) {
+            const f32x2 ev = {e[h][t], e[h][t + 1]};
+            const bf16x2 hv = __builtin_convertvector(ev, bf16x2);
+            ahi[h][t] = hv[0];
+            ahi[h][t + 1] = hv[1];
+            if (MODE == kModeBf16x3) {
+              const uint32_t bits = __builtin_bit_cast(uint32_t, hv);
+              const f32x2 rv = {ev[0] - __uint_as_float(bits << 16), ev[1] - __uint_as_float(bits & 0xffff0000u)};
+              const bf16x2 lv = __builtin_convertvector(rv, bf16x2);
+              alo[h][t] = lv[0];
+              alo[h][t + 1] = lv[1];
             }
           }
+        // one product per accumulator before the next part: a product waits for
+        // the last one on its accumulator
+        bf16x8 bhi[CB], blo[CB];
+#pragma unroll
+        for (int c = 0; c < CB; ++c) {
+          bhi[c] = *reinterpret_cast<const bf16x8*>(ops + c * step_bytes(MODE));
+          if (MODE == kModeBf16x3) blo[c] = *reinterpret_cast<const bf16x8*>(ops + kPart + c * step_bytes(MODE));
+        }
+        auto contract = [&](const bf16x8(&av)[2], const bf16x8(&bv)[CB]) {
+#pragma unroll
+          for (int c = 0; c < CB; ++c)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+              acc[h][c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[h], bv[c], acc[h][c], 0, 0, 0);
+        };
+        contract(ahi, bhi);
+        if (MODE == kModeBf16x3) {
+          contract(ahi, blo);
+          contract(alo, bhi);
         }
       }
     }
   }
-  // ---- write FP64 slab partials.  32x32 accumulator layout: lane l holds
-  // column l%32 and rows 8*(v/4) + 4*(l/32) + v%4, v = 0..15.
+  // ---- slab partials, in FP32 as accumulated.  32x32 accumulator layout:
+  // lane l holds column l%32 and rows 8*(v/4) + 4*(l/32) + v%4, v = 0..15, so
+  // four consecutive rows per quarter of the accumulator.
 #pragma unroll
   for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -346,9 +391,17 @@ __global__ __launch_bounds__(kBlock) void mrhs_mfma_kernel(
       const int64_t r = c * 32 + (lane % 32);
       if (r >= R) continue;
 #pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int64_t i = base + h * 32 + 8 * (v / 4) + 4 * (lane / 32) + (v % 4);
-        if (i < rows) part[((int64_t)blockIdx.y * R + r) * rows + i] = (double)acc[h][c][v];
+      for (int u = 0; u < 4; ++u) {
+        const int64_t i = base + h * 32 + 8 * u + 4 * (lane / 32);
+        float* out = part + ((int64_t)blockIdx.y * R + r) * rows + i;
+        if (i + 4 <= rows) {
+          const f32x4u q = {acc[h][c][4 * u], acc[h][c][4 * u + 1], acc[h][c][4 * u + 2], acc[h][c][4 * u + 3]};
+          *reinterpret_cast<f32x4u*>(out) = q;
+        } else {
+#pragma unroll
+          for (int v = 0; v < 4; ++v)
+            if (i + v < rows) out[v] = acc[h][c][4 * u + v];
+        }
       }
     }
 }
@@ -474,20 +527,34 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(waves64(
     }
 }
 
-// Y[i + r ldy] = sum over slabs (slab order) + nugget * V at the global diagonal.
+// Y[i + r ldy] = sum over slabs (slab order) + nugget * V at the global
+// diagonal.  One row per thread, grid = (row blocks, columns); bound by the
+// partials' bandwidth, so kFinishBatch of them are in flight per thread.  FP32
+// accumulators leave FP32 partials: the same values as widened ones at half
+// the bytes.
+constexpr int kFinishBatch = 8;
+
+template <typename PT>
 __global__ __launch_bounds__(kBlock) void mrhs_finish_kernel(int64_t rows, int64_t R, int64_t slabs,
-                                                             const double* __restrict__ part, int64_t row_off,
+                                                             const PT* __restrict__ part, int64_t row_off,
                                                              int64_t col_off, int64_t cols, double nugget,
                                                              const double* __restrict__ V, int64_t ldv,
                                                              double* __restrict__ Y, int64_t ldy,
                                                              const int32_t* __restrict__ skip) {
   if (skip != nullptr && *skip != 0) return;
-  const int64_t total = rows * R;
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; g < total; g += stride) {
-    const int64_t i = g % rows, r = g / rows;
-    double s = part[r * rows + i];
-    for (int64_t k = 1; k < slabs; ++k) s += part[(k * R + r) * rows + i];
+  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (i >= rows) return;
+  for (int64_t r = blockIdx.y; r < R; r += gridDim.y) {
+    const PT* p = part + r * rows + i;
+    double s = (double)p[0];
+    for (int64_t k = 1; k < slabs; k += kFinishBatch) {
+      PT v[kFinishBatch];
+#pragma unroll
+      for (int u = 0; u < kFinishBatch; ++u) v[u] = k + u < slabs ? p[(k + u) * R * rows] : PT(0);
+#pragma unroll
+      for (int u = 0; u < kFinishBatch; ++u)
+        if (k + u < slabs) s += (double)v[u];
+    }
     const int64_t jd = row_off + i - col_off;
     if (nugget != 0.0 && jd >= 0 && jd < cols) s = fma(nugget, V[r * ldv + jd], s);
     Y[r * ldy + i] = s;
@@ -512,7 +579,7 @@ struct MrhsPlan {
   int64_t cblocks;
   Slabs s;
   size_t vpk_bytes, part_bytes;
-  int64_t steps;
+  int64_t blocks;  // packed source blocks
 };
 
 inline int valu_rt(int64_t R) {
@@ -528,7 +595,7 @@ inline MrhsPlan make_plan(const mplak_kernel_desc* d, int precision, int64_t R) 
   if (precision == MPLAK_PREC_F64 && R >= kMfma64MinR && d->dim <= 4) {
     p.mfma64 = true;
     p.cblocks = (R + 15) / 16;
-    p.s = balanced_slabs(d->row_count, d->col_count, kTile64, kSrc64, 256 * waves64((int)std::min<int64_t>(p.cblocks, 4)));
+    p.s = balanced_slabs(d->row_count, d->col_count, kTile64, kSrc64, waves64((int)std::min<int64_t>(p.cblocks, 4)), R);
     p.part_bytes = align_up((size_t)p.s.slabs * (size_t)R * (size_t)d->row_count * sizeof(double), 256);
     return p;
   }
@@ -538,19 +605,17 @@ inline MrhsPlan make_plan(const mplak_kernel_desc* d, int precision, int64_t R) 
   if (p.mfma) {
     p.mode = precision == MPLAK_PREC_BF16 ? kModeBf16 : (precision == MPLAK_PREC_BF16X3 ? kModeBf16x3 : kModeF32);
     p.cblocks = (R + 31) / 32;
-    p.s = slab_plan(d->row_count, d->col_count, kMfmaTile, 1);
-    const int64_t cols_pad = p.s.slabs * p.s.slab_cols;
-    p.steps = cols_pad / 16;
-    const int64_t total = p.steps * p.cblocks * kWave;
-    const size_t elem = p.mode == kModeF32 ? 4 : 2;
-    p.vpk_bytes = align_up((size_t)total * 8 * elem * (p.mode == kModeBf16x3 ? 2 : 1), 256);
+    p.s = balanced_slabs(d->row_count, d->col_count, kMfmaTile, kMfmaSlab, mfma_waves((int)p.cblocks), R);
+    p.blocks = (d->col_count + kMfmaSlab - 1) / kMfmaSlab;
+    p.vpk_bytes = align_up((size_t)p.blocks * (size_t)block_bytes(p.mode, (int)p.cblocks) + kPackAlign, 256);
   } else {
     p.rt = valu_rt(R);
     const int64_t ctiles = (R + p.rt - 1) / p.rt;
     p.s = slab_plan(d->row_count, d->col_count, kBlock, ctiles);
     p.vpk_bytes = 0;
   }
-  p.part_bytes = align_up((size_t)p.s.slabs * (size_t)R * (size_t)d->row_count * sizeof(double), 256);
+  p.part_bytes = align_up((size_t)p.s.slabs * (size_t)R * (size_t)d->row_count * (p.mfma ? sizeof(float) : sizeof(double)),
+                          256);
   return p;
 }
 
@@ -594,14 +659,12 @@ void launch_valu(const mplak_kernel_desc* d, const MrhsPlan& p, hipStream_t st, 
 
 template <int KIND, int MODE>
 void launch_mfma_mode(const mplak_kernel_desc* d, const MrhsPlan& p, hipStream_t st, double scale, int64_t R,
-                      const void* vpk, double* part, const int32_t* skip) {
+                      const char* packed, float* part, const int32_t* skip) {
   const dim3 grid((unsigned)p.s.tiles, (unsigned)p.s.slabs);
-  const int64_t total = p.steps * p.cblocks * kWave;
   auto go = [&](auto cb_tag, auto dim_tag) {
     constexpr int CBV = decltype(cb_tag)::value, DIMV = decltype(dim_tag)::value;
-    hipLaunchKernelGGL((mrhs_mfma_kernel<KIND, MODE, CBV, DIMV>), grid, dim3(kBlock), 0, st, d->points, d->dim,
-                       d->row_offset, d->row_count, d->col_offset, d->col_count, p.s.slab_cols, scale, R, vpk,
-                       total, part, skip);
+    hipLaunchKernelGGL((mrhs_mfma_kernel<KIND, MODE, CBV, DIMV>), grid, dim3(kBlock), 0, st, d->points, d->row_offset,
+                       d->row_count, p.blocks, p.s.slab_cols / kMfmaSlab, scale, R, packed, part, skip);
   };
   auto with_dim = [&](auto cb_tag) {
     switch (d->dim) {
@@ -644,13 +707,13 @@ void launch_mfma64(const mplak_kernel_desc* d, const MrhsPlan& p, hipStream_t st
 
 template <int KIND>
 void launch_mfma(const mplak_kernel_desc* d, const MrhsPlan& p, hipStream_t st, double scale, int64_t R,
-                 const void* vpk, double* part, const int32_t* skip) {
+                 const char* packed, float* part, const int32_t* skip) {
   if (p.mode == kModeBf16)
-    launch_mfma_mode<KIND, kModeBf16>(d, p, st, scale, R, vpk, part, skip);
+    launch_mfma_mode<KIND, kModeBf16>(d, p, st, scale, R, packed, part, skip);
   else if (p.mode == kModeBf16x3)
-    launch_mfma_mode<KIND, kModeBf16x3>(d, p, st, scale, R, vpk, part, skip);
+    launch_mfma_mode<KIND, kModeBf16x3>(d, p, st, scale, R, packed, part, skip);
   else
-    launch_mfma_mode<KIND, kModeF32>(d, p, st, scale, R, vpk, part, skip);
+    launch_mfma_mode<KIND, kModeF32>(d, p, st, scale, R, packed, part, skip);
 }
 
 int check_desc(const mplak_kernel_desc* d) {
@@ -710,19 +773,18 @@ int mplak_kernel_mrhs(const mplak_kernel_desc* d, int precision, int64_t nrhs, c
     const double* Vg = V + r0 * ldv;
     double* Yg = Y + r0 * ldy;
     char* w = static_cast<char*>(work);
+    char* packed = reinterpret_cast<char*>(align_up(reinterpret_cast<uintptr_t>(w), kPackAlign));
     double* part = reinterpret_cast<double*>(w + p.vpk_bytes);
+    float* part32 = reinterpret_cast<float*>(part);
     if (p.mfma) {
-      const int64_t total = p.steps * p.cblocks * kWave;
-      int64_t pb = (total + kBlock - 1) / kBlock;
-      if (pb > 8192) pb = 8192;
-      hipLaunchKernelGGL(pack_v_kernel, dim3((unsigned)pb), dim3(kBlock), 0, hs, Vg, ldv, R, d->col_count, p.steps,
-                         p.cblocks, p.mode, (void*)w);
+      hipLaunchKernelGGL(pack_kernel, dim3((unsigned)std::min<int64_t>(p.blocks, 8192)), dim3(kBlock), 0, hs, d->points,
+                         d->dim, d->col_offset, scale, Vg, ldv, R, d->col_count, p.blocks, (int)p.cblocks, p.mode, packed);
       st = launch_status();
       if (st != MPLAK_OK) return st;
       if (d->kind == MPLAK_KERNEL_GAUSSIAN)
-        launch_mfma<MPLAK_KERNEL_GAUSSIAN>(d, p, hs, scale, R, w, part, skip_if);
+        launch_mfma<MPLAK_KERNEL_GAUSSIAN>(d, p, hs, scale, R, packed, part32, skip_if);
       else
-        launch_mfma<MPLAK_KERNEL_MATERN32>(d, p, hs, scale, R, w, part, skip_if);
+        launch_mfma<MPLAK_KERNEL_MATERN32>(d, p, hs, scale, R, packed, part32, skip_if);
     } else if (p.mfma64) {
       if (d->kind == MPLAK_KERNEL_GAUSSIAN)
         launch_mfma64<MPLAK_KERNEL_GAUSSIAN>(d, p, hs, scale, R, Vg, ldv, part, skip_if);
@@ -743,10 +805,13 @@ int mplak_kernel_mrhs(const mplak_kernel_desc* d, int precision, int64_t nrhs, c
     }
     st = launch_status();
     if (st != MPLAK_OK) return st;
-    int64_t fb = (d->row_count * R + kBlock - 1) / kBlock;
-    if (fb > 8192) fb = 8192;
-    hipLaunchKernelGGL(mrhs_finish_kernel, dim3((unsigned)fb), dim3(kBlock), 0, hs, d->row_count, R, p.s.slabs, part,
-                       d->row_offset, d->col_offset, d->col_count, d->nugget, Vg, ldv, Yg, ldy, skip_if);
+    const dim3 fgrid((unsigned)((d->row_count + kBlock - 1) / kBlock), (unsigned)std::min<int64_t>(R, 65535));
+    if (p.mfma)
+      hipLaunchKernelGGL(mrhs_finish_kernel<float>, fgrid, dim3(kBlock), 0, hs, d->row_count, R, p.s.slabs, part32,
+                         d->row_offset, d->col_offset, d->col_count, d->nugget, Vg, ldv, Yg, ldy, skip_if);
+    else
+      hipLaunchKernelGGL(mrhs_finish_kernel<double>, fgrid, dim3(kBlock), 0, hs, d->row_count, R, p.s.slabs, part,
+                         d->row_offset, d->col_offset, d->col_count, d->nugget, Vg, ldv, Yg, ldy, skip_if);
     st = launch_status();
     if (st != MPLAK_OK) return st;
   }

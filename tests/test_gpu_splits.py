@@ -122,3 +122,41 @@ def test_mrhs_f64_tiles(lib, rows, cols, row_off, R, dim, kind):
     # the oracle's FP64 bar: 1e-12 of the sum of magnitudes
     assert np.all(np.abs(got[:, :rows] - V[:, :cols] @ K.T) <= 1e-12 * (np.abs(V[:, :cols]) @ K.T))
     assert np.all(got[:, rows:] == 7.0)
+
+
+# Multi-right-hand-side products on the matrix cores in lower precision: packed
+# blocks of 64 sources (a workgroup stages two at a time), 256-row tiles, one or
+# two 32-column blocks, a 64-column group with a narrow rest, several slabs.
+@pytest.mark.parametrize("rows,cols,row_off,R,dim", [
+    (1, 1, 0, 1, 1), (255, 63, 0, 16, 2), (257, 64, 2, 32, 3), (256, 65, 0, 33, 4), (100, 129, 7, 64, 3),
+    (1000, 1537, 100, 65, 3), (1500, 1500, 0, 20, 2), (5000, 4999, 0, 40, 3)])
+@pytest.mark.parametrize("prec,bar", [(1, 2e-5), (2, 2e-2), (3, 1e-4)])
+def test_mrhs_mfma_blocks(lib, rows, cols, row_off, R, dim, prec, bar):
+    import ctypes as C
+
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(rows + cols + R)
+    n = max(cols, row_off + rows)
+    P = torch.rand((dim, n), generator=g, dtype=torch.float64, device="cuda")
+    ell, nugget = 0.4, 0.7
+    ldv, ldy = cols + 3, rows + 5
+    V = torch.randn((R, ldv), generator=g, dtype=torch.float64, device="cuda")
+    s = sum((P[d, row_off:row_off + rows, None] - P[d, None, :cols]) ** 2 for d in range(dim))
+    r = (3.0 * s).sqrt() / ell
+    K = (1.0 + r) * (-r).exp()
+    ref, mag = V[:, :cols] @ K.t(), V[:, :cols].abs() @ K.t()
+    i = torch.arange(row_off, min(row_off + rows, cols), device="cuda")
+    ref[:, i - row_off] += nugget * V[:, i]
+    Y = torch.full((R, ldy), 7.0, dtype=torch.float64, device="cuda")
+    table = torch.tensor([P[d].data_ptr() for d in range(dim)], dtype=torch.int64, device="cuda")
+    desc = _native.mplak_kernel_desc(table.data_ptr(), dim, 1, ell, nugget, 0.0, row_off, rows, 0, cols)
+    wb = lib.mplak_kernel_mrhs_workspace_bytes(C.byref(desc), prec, R)
+    w = torch.empty(wb + 8, dtype=torch.uint8, device="cuda")
+    for shift in (0, 8):  # a workspace that is 8-byte aligned only
+        ck(lib.mplak_kernel_mrhs(C.byref(desc), prec, R, V.data_ptr(), ldv, Y.data_ptr(), ldy, w.data_ptr() + shift, wb,
+                                 None, stream()))
+        got = host(Y)
+        # normwise per column: FP32 entries 2e-5; BF16 operands (8 bits) 2 x 2^-8, split BF16 2^-16 with FP32 sums
+        err = np.linalg.norm(got[:, :rows] - host(ref), axis=1)
+        assert np.all(err <= bar * np.linalg.norm(host(mag), axis=1) + 1e-30)
+        assert np.all(got[:, rows:] == 7.0)
