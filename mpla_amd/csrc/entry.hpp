@@ -55,15 +55,38 @@ __device__ __forceinline__ void fill_exp2_table(double* tab) {
 // * tab[k mod 256], 2^f = sum_{n<=4} (f ln 2)^n / n!.
 __device__ __forceinline__ double exp2_neg(double s, const double* __restrict__ tab) {
   s = fmin(s, 1100.0);
-  const double k = rint(s * -256.0);
+  // adding 1.5 * 2^52 rounds -256 s to an integer (ties to even) and leaves it
+  // in the low word: the bits of rint and a conversion in two instructions
+  // instead of three
+  constexpr double kRound = 6755399441055744.0;
+  const double t = fma(s, -256.0, kRound);
+  const double k = t - kRound;
   const double f = fma(k, -1.0 / 256.0, -s);
-  const int ki = (int)k;
+  const int ki = __double2loint(t);
   // Taylor coefficients ln(2)^n / n!
   double p = fma(f, 0.0096181291076284772, 0.055504108664821580);
   p = fma(f, p, 0.24022650695910071);
   p = fma(f, p, 0.69314718055994531);
   p = fma(f, p, 1.0);
   return __builtin_amdgcn_ldexp(tab[ki & (kExp2Table - 1)] * p, ki >> 8);  // one v_ldexp_f64, any exponent
+}
+
+// sqrt(s) for s >= 0, from the hardware's 1 / sqrt (relative error 2^-24) by
+// one coupled Newton (Goldschmidt) step for the root and half its reciprocal
+// and a last residual correction (P. Markstein, "IA-64 and Elementary
+// Functions", 2000): measured within half an ulp, as sqrt() is, in 54 cycles a
+// wave against 86, which scales its argument first for the ends of the range.
+// Squared distances need neither end: 0 gives 0, and below 1e-280 the root is
+// small enough that every kernel is 1.  An infinite s gives NaN (the Matern
+// entry of one is NaN either way).
+__device__ __forceinline__ double sqrt_distance2(double s) {
+  const double y = __builtin_amdgcn_rsq(s + 1e-300);
+  double g = s * y;
+  double h = 0.5 * y;
+  const double r = fma(-h, g, 0.5);
+  g = fma(g, r, g);
+  h = fma(h, r, h);
+  return fma(fma(-g, g, s), h, g);
 }
 
 template <typename T, int KIND>
@@ -75,7 +98,7 @@ __device__ __forceinline__ double kernel_entry<double, MPLAK_KERNEL_GAUSSIAN>(do
 }
 template <>
 __device__ __forceinline__ double kernel_entry<double, MPLAK_KERNEL_MATERN32>(double s, const double* tab) {
-  const double r = sqrt(s);
+  const double r = sqrt_distance2(s);
   const double e = exp2_neg(r * kLog2e, tab);
   return fma(r, e, e);
 }

@@ -69,7 +69,8 @@ inline Slabs slab_plan(int64_t rows, int64_t cols, int tile_rows, int64_t col_ti
 // units of one workgroup's chunk on a full CU, the chunks of the busiest CU
 // plus the slabs' partials, written and read back once each.  A CU with fewer
 // than `occ` workgroups takes a chunk down to a quarter of that time.  Measured:
-// partials 4 TB/s, against 8 us for a 64-column BF16x3 chunk and 18 us for an
+// partials 4 TB/s and 0.15 us of latency a slab (n = 3000, 16 columns: 47 slabs
+// 27 us, 16 slabs 25 us), against 8 us for a 64-column BF16x3 chunk and 18 us for an
 // FP64 one (n = 20001, 64 columns in FP64: 1.44 ms in 8 slabs, five workgroups
 // on the busiest CU; 1.66 ms in 4, three).
 inline Slabs balanced_slabs(int64_t rows, int64_t cols, int tile_rows, int chunk, int occ, int64_t R) {
@@ -78,7 +79,7 @@ inline Slabs balanced_slabs(int64_t rows, int64_t cols, int tile_rows, int chunk
   p.tiles = (rows + tile_rows - 1) / tile_rows;
   const int64_t chunks = (cols + chunk - 1) / chunk;
   const int64_t most = std::min<int64_t>(chunks, std::max<int64_t>(4 * kCus * occ / p.tiles, 1));
-  const double slab_cost = 2.4e-7 * (double)rows * (double)R;
+  const double slab_cost = 0.02 + 2.4e-7 * (double)rows * (double)R;
   double best = 0.0;
   for (int64_t ks = 1; ks <= most; ++ks) {
     const int64_t per = (chunks + ks - 1) / ks;
