@@ -3,11 +3,11 @@
 // y_i = sum_j k(|p_i - p_j|) x_j (+ nugget x_i on the global diagonal,
 // + coincident_shift x_j where |p_i - p_j| < 1e-14), entries never stored.
 //
-// Tiling: a 256-thread workgroup owns a tile of 512 target points (two per
-// thread, held in registers) and one slab of source columns.  The slab is
-// streamed through LDS in chunks of 256 points (coordinates pre-scaled so the
-// kernel argument is a plain sum of squares) together with the matching x
-// values; every lane reads the same LDS word at a time (broadcast, no bank
+// Tiling of the plain product: a 256-thread workgroup owns 256 target points
+// (one per thread, in registers) and one slab of source columns.  The slab is
+// streamed through LDS in chunks of up to 256 points (coordinates pre-scaled
+// so the kernel argument is a plain sum of squares) together with the matching
+// x values; every lane reads the same LDS word at a time (broadcast, no bank
 // conflicts).  Slab partial sums go to a workspace and a second kernel adds
 // them in slab order, so the result is deterministic for a given shape.
 //
@@ -57,28 +57,34 @@ int noalloc_scratch(void** out) {
   return MPLAK_OK;
 }
 
-constexpr int kKmvTpt = 2;                     // target points per thread
-constexpr int kKmvTile = kBlock * kKmvTpt;     // 512 targets per workgroup
 constexpr int kKmvChunk = kBlock;              // sources per LDS chunk
 constexpr int kKmvMaxDim = 16;
-constexpr int kKmvTargetBlocks = 4096;
+constexpr int kKmvMinSlab = 32;                // fewest sources of a slab
+constexpr int64_t kKmvMaxSlabs = 64;
+constexpr int64_t kKmvMaxBlocks = 8192;        // bounds the partials at 16.8 MB
+constexpr int kFinishLoads = 16;               // slab partials in flight per row
 
 struct KmvPlan {
   int64_t row_tiles, slabs, slab_cols;
 };
 
+// A few thousand targets are a few workgroups, whose slab is a serial chain of
+// entries, so the slab is as short as up to 64 partials a row allow: the finish
+// takes about 1 us per 16.  Measured, FP64 Gaussian in 3-D, slabs of 256 / 128 /
+// 64 / 32 sources: n = 1000 19.6 / 12.6 / 9.5 / 8.8 us, n = 3001 21.1 / 18.6 /
+// 16.7 / 18.3 us, n = 8000 51.7 / 51.4 / 54.3 / 62.5 us.  One target a thread
+// is faster than two at every size there (n = 3001: 16.7 against 19.8 us).
 inline KmvPlan kmv_plan(int64_t rows, int64_t cols) {
   KmvPlan p;
-  p.row_tiles = (rows + kKmvTile - 1) / kKmvTile;
-  int64_t ks = (kKmvTargetBlocks + p.row_tiles - 1) / p.row_tiles;
-  int64_t max_ks = (cols + kKmvChunk - 1) / kKmvChunk;  // at least one chunk per slab
-  if (ks > max_ks) ks = max_ks;
-  if (ks < 1) ks = 1;
-  if (ks > 65535) ks = 65535;
-  // slab width is a whole number of chunks
-  int64_t chunks = (cols + kKmvChunk - 1) / kKmvChunk;
-  int64_t chunks_per_slab = (chunks + ks - 1) / ks;
-  p.slab_cols = chunks_per_slab * kKmvChunk;
+  p.row_tiles = (rows + kBlock - 1) / kBlock;
+  const int64_t most = std::max<int64_t>(std::min(kKmvMaxSlabs, kKmvMaxBlocks / p.row_tiles), 1);
+  p.slab_cols = kKmvMinSlab;
+  while (p.slab_cols < kKmvChunk && (cols + p.slab_cols - 1) / p.slab_cols > most) p.slab_cols *= 2;
+  if ((cols + p.slab_cols - 1) / p.slab_cols > most) {
+    // whole chunks
+    const int64_t chunks = (cols + kKmvChunk - 1) / kKmvChunk;
+    p.slab_cols = (chunks + most - 1) / most * kKmvChunk;
+  }
   p.slabs = (cols + p.slab_cols - 1) / p.slab_cols;
   return p;
 }
@@ -99,29 +105,21 @@ __global__ __launch_bounds__(kBlock) void kmv_partial_kernel(
   if (sizeof(T) == 8) fill_exp2_table(exp_tab);  // first read after the chunk barrier below
 
   const int tid = threadIdx.x;
-  const int64_t tile0 = (int64_t)blockIdx.x * kKmvTile;
-  const T sc = (T)scale;
   const T thr = (T)coinc_thr;
   const T shift = (T)coinc_shift;
 
   // Target coordinates in registers (rows past the end are computed on a
   // copy of the last row and never stored).
-  T pi[kKmvTpt][MD];
+  const int64_t i = (int64_t)blockIdx.x * kBlock + tid;
+  const int64_t ic = i < rows ? i : rows - 1;
+  T pi[MD];
 #pragma unroll
-  for (int t = 0; t < kKmvTpt; ++t) {
-    int64_t i = tile0 + tid + t * kBlock;
-    if (i >= rows) i = rows - 1;
-#pragma unroll
-    for (int d = 0; d < MD; ++d) pi[t][d] = d < dim ? (T)(points[d][row_off + i] * scale) : T(0);
-  }
+  for (int d = 0; d < MD; ++d) pi[d] = d < dim ? (T)(points[d][row_off + ic] * scale) : T(0);
 
   const int64_t c0 = (int64_t)blockIdx.y * slab_cols;
   const int64_t c1 = (c0 + slab_cols < cols) ? c0 + slab_cols : cols;
 
-  double acc[kKmvTpt];
-#pragma unroll
-  for (int t = 0; t < kKmvTpt; ++t) acc[t] = 0.0;
-
+  double acc = 0.0;
   for (int64_t cb = c0; cb < c1; cb += kKmvChunk) {
     __syncthreads();
     {
@@ -137,40 +135,26 @@ __global__ __launch_bounds__(kBlock) void kmv_partial_kernel(
       }
     }
     __syncthreads();
-    T cacc[kKmvTpt];
-#pragma unroll
-    for (int t = 0; t < kKmvTpt; ++t) cacc[t] = T(0);
+    T cacc = T(0);
+    // past c1 the staged values are zero: whole unrolled rounds
+    const int count = (int)(((c1 - cb < kKmvChunk ? c1 - cb : kKmvChunk) + 3) & ~int64_t(3));
 #pragma unroll 4
-    for (int jj = 0; jj < kKmvChunk; ++jj) {
-      T pj[MD];
+    for (int jj = 0; jj < count; ++jj) {
+      T s = T(0);
 #pragma unroll
-      for (int d = 0; d < MD; ++d) pj[d] = d < dim ? lp[d][jj] : T(0);
-      const T xj = lx[jj];
-#pragma unroll
-      for (int t = 0; t < kKmvTpt; ++t) {
-        T s = T(0);
-#pragma unroll
-        for (int d = 0; d < MD; ++d) {
-          if (d < dim) {
-            const T df = pi[t][d] - pj[d];
-            s = fma(df, df, s);
-          }
+      for (int d = 0; d < MD; ++d) {
+        if (d < dim) {
+          const T df = pi[d] - lp[d][jj];
+          s = fma(df, df, s);
         }
-        T k = kernel_entry<T, KIND>(s, exp_tab);
-        if (COINC) k += (s < thr) ? shift : T(0);
-        cacc[t] = fma(k, xj, cacc[t]);
       }
+      T k = kernel_entry<T, KIND>(s, exp_tab);
+      if (COINC) k += (s < thr) ? shift : T(0);
+      cacc = fma(k, lx[jj], cacc);
     }
-#pragma unroll
-    for (int t = 0; t < kKmvTpt; ++t) acc[t] += (double)cacc[t];
+    acc += (double)cacc;
   }
-  (void)sc;
-
-#pragma unroll
-  for (int t = 0; t < kKmvTpt; ++t) {
-    const int64_t i = tile0 + tid + t * kBlock;
-    if (i < rows) out[(int64_t)blockIdx.y * rows + i] = acc[t];
-  }
+  if (i < rows) out[(int64_t)blockIdx.y * rows + i] = acc;
 }
 
 // y_i = sum over slabs (slab order) + nugget * x at the global diagonal.
@@ -182,7 +166,14 @@ __global__ __launch_bounds__(kBlock) void kmv_finish_kernel(
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < rows; i += stride) {
     double s = part[i];
-    for (int64_t k = 1; k < slabs; ++k) s += part[k * rows + i];
+    for (int64_t k = 1; k < slabs; k += kFinishLoads) {
+      double v[kFinishLoads];
+#pragma unroll
+      for (int u = 0; u < kFinishLoads; ++u) v[u] = k + u < slabs ? part[(k + u) * rows + i] : 0.0;
+#pragma unroll
+      for (int u = 0; u < kFinishLoads; ++u)
+        if (k + u < slabs) s += v[u];
+    }
     const int64_t jd = row_off + i - col_off;
     if (nugget != 0.0 && jd >= 0 && jd < cols) s = fma(nugget, x[jd], s);
     y[i] = s;
@@ -275,7 +266,10 @@ __device__ __forceinline__ P* slot_row(P* part, int64_t X, int64_t partner, int3
   return part + ((X * kFinishSlices + (partner & (kFinishSlices - 1))) * pcap + slot) * kSymTile;
 }
 
-constexpr int kSymMinN = 12288;       // crossover measured on MI355X (plain kernel faster below)
+// Fewest points of the symmetric product; below, the plain product's finer
+// split is faster (FP64, 3-D Gaussian, plain / symmetric: n = 2000 11.2 / 13.3
+// us, n = 3001 16.7 / 14.2 us, n = 4000 19.6 / 19.9 us, n = 5000 29.5 / 21.2 us).
+constexpr int kSymMinN = 3000;
 
 // MPLAK_KMV_SYMMETRIC=0 turns the symmetric product off, =1 uses it for every
 // eligible block regardless of size; unset: blocks of at least kSymMinN points.
@@ -305,6 +299,21 @@ __device__ __forceinline__ double global_load(const double* ptr) {
   return *(global_ptr)ptr;
 }
 
+// A workgroup's pair (in the plan's list, if there is one), its part of the pair
+// and the bits of the source groups of that part.  SPLIT = false: whole pairs, all of it
+// constant (at n = 65536 the divisions alone cost a planned FP32 product 3 %).
+template <bool SPLIT>
+struct PairPart {
+  int64_t item;
+  int split, sub;
+  uint32_t groups;
+  __device__ __forceinline__ explicit PairPart(int s)
+      : item(SPLIT ? blockIdx.x / (unsigned)s : blockIdx.x),
+        split(SPLIT ? s : 1),
+        sub(SPLIT ? (int)(blockIdx.x % (unsigned)s) : 0),
+        groups(SPLIT ? ((1u << ((kSymTile / kWave) / s)) - 1u) << (sub * ((kSymTile / kWave) / s)) : 0xffu) {}
+};
+
 enum SymMode { kSymExact = 0, kSymScreened = 1, kSymPlanned = 2 };
 
 // One tile pair (I, J) of the symmetric product on the vector unit.
@@ -319,11 +328,14 @@ enum SymMode { kSymExact = 0, kSymScreened = 1, kSymPlanned = 2 };
 template <typename T>
 using SymSrc = typename Quad<T>::type[(sizeof(T) == 4 ? 2 : 1) * kWave];
 
-template <typename T, int KIND, int DIM, bool COINC, bool SCREEN, bool MASKED, typename P>
+// Only the 64-source groups of `groups` are worked on; SHARED_J: rows_j belongs
+// to all parts of the pair and gets this part's groups only (zeros elsewhere
+// otherwise).
+template <typename T, int KIND, int DIM, bool COINC, bool SCREEN, bool MASKED, bool SHARED_J, typename P>
 __device__ __forceinline__ void sym_valu_pair(const double* const* __restrict__ points, int64_t off, int64_t n,
                                               double scale, double coinc_thr, double coinc_shift, double drop_s,
                                               const double* __restrict__ x, P* __restrict__ rows_i,
-                                              P* __restrict__ rows_j, int64_t p, uint32_t pmask,
+                                              P* __restrict__ rows_j, int64_t p, uint32_t pmask, uint32_t groups,
                                               SymSrc<T>* src, T (*gbox)[6], T* own_red, const double* exp_tab) {
   typedef typename Quad<T>::type Q;
   constexpr int kDup = sizeof(T) == 4 ? 2 : 1;  // copies of each 64-source group
@@ -405,6 +417,7 @@ __device__ __forceinline__ void sym_valu_pair(const double* const* __restrict__ 
   }
   // true when every entry between this wave's targets and group g is dropped
   auto far_group = [&](int g) -> bool {
+    if (((groups >> g) & 1u) == 0) return true;
     if (!SCREEN) return false;
     if (MASKED) return ((wmask >> g) & 1u) == 0;
     const T d2 = box_gap2<T, DIM>(tbox, gbox[g]);
@@ -483,6 +496,7 @@ __device__ __forceinline__ void sym_valu_pair(const double* const* __restrict__ 
   if (I != J) {
     __syncthreads();
     for (int k = tid; k < kSymTile; k += kBlock) {
+      if (SHARED_J && ((groups >> (k / kWave)) & 1u) == 0) continue;
       double s = (double)red[k];
 #pragma unroll
       for (int q = 1; q < kBlock / kWave; ++q) s += (double)red[q * kSymTile + k];
@@ -492,18 +506,21 @@ __device__ __forceinline__ void sym_valu_pair(const double* const* __restrict__ 
 }
 
 // Symmetric product kernel on the vector unit: kSymExact / kSymScreened over
-// all tile pairs (workgroup p = pair p, partial rows by pair),
-// kSymPlanned over the tile pairs list[0 .. *count) of a screening plan
-// (pairs with a kept block; rows in the plan's slotted layout, which holds
-// no row for the others).
-template <typename T, int KIND, int DIM, bool COINC, int MODE>
+// all tile pairs, kSymPlanned over the tile pairs list[0 .. *count) of a
+// screening plan (pairs with a kept block; rows in the plan's slotted layout,
+// which holds no row for the others).  SPLIT: `split` workgroups share a pair,
+// each with a row set of its own for tile I.  The rows of tile J are the pair's,
+// each part writing its source groups; with a plan each part has its own (zero
+// outside its groups, so the sums are bitwise the same).
+template <typename T, int KIND, int DIM, bool COINC, int MODE, bool SPLIT>
 __global__ __launch_bounds__(kBlock) void kmv_sym_kernel(
     const double* const* __restrict__ points, int64_t off, int64_t n, double scale, double coinc_thr,
     double coinc_shift, double drop_s, const double* __restrict__ x, double* __restrict__ part_i,
     double* __restrict__ part_j, const uint32_t* __restrict__ list, const int64_t* __restrict__ count,
-    const int32_t* __restrict__ slots, int64_t pcap, const int32_t* __restrict__ skip) {
+    const int32_t* __restrict__ slots, int64_t pcap, int split, const int32_t* __restrict__ skip) {
   if (skip != nullptr && *skip != 0) return;
-  if (MODE == kSymPlanned && (int64_t)blockIdx.x >= *count) return;
+  const PairPart<SPLIT> part_of(split);
+  if (MODE == kSymPlanned && part_of.item >= *count) return;
   typedef typename Quad<T>::type Q;
   constexpr int kDup = sizeof(T) == 4 ? 2 : 1;
   constexpr int kGroups = kSymTile / kWave;
@@ -515,19 +532,20 @@ __global__ __launch_bounds__(kBlock) void kmv_sym_kernel(
   __shared__ T own_red[kHoldSums ? 1 : (kBlock / kWave) * kSymTile];
   __shared__ double exp_tab[Exp2Lds<T>::size];
   if (sizeof(T) == 8) fill_exp2_table(exp_tab);  // first read after the staging barrier
-  const int64_t p = MODE == kSymPlanned ? (int64_t)list[blockIdx.x] : (int64_t)blockIdx.x;
+  const int64_t p = MODE == kSymPlanned ? (int64_t)list[part_of.item] : part_of.item;
   // partial rows: by pair (part_i for tile I, part_j for tile J), or with a
   // plan in its slotted layout (part_i)
-  double* rows_i = part_i + p * kSymTile;
+  double* rows_i = part_i + (p * part_of.split + part_of.sub) * kSymTile;
   double* rows_j = part_j + p * kSymTile;
   if (MODE == kSymPlanned) {
     int64_t I, J;
     decode_pair(p, I, J);
-    rows_i = slot_row(part_i, I, J, slots[2 * p], pcap);
-    rows_j = I != J ? slot_row(part_i, J, I, slots[2 * p + 1], pcap) : rows_i;
+    const int64_t rows = pcap * part_of.split;
+    rows_i = slot_row(part_i, I, J, slots[2 * p] * part_of.split + part_of.sub, rows);
+    rows_j = I != J ? slot_row(part_i, J, I, slots[2 * p + 1] * part_of.split + part_of.sub, rows) : rows_i;
   }
-  sym_valu_pair<T, KIND, DIM, COINC, MODE != kSymExact, false, double>(
-      points, off, n, scale, coinc_thr, coinc_shift, drop_s, x, rows_i, rows_j, p, 0u,
+  sym_valu_pair<T, KIND, DIM, COINC, MODE != kSymExact, false, SPLIT && MODE != kSymPlanned, double>(
+      points, off, n, scale, coinc_thr, coinc_shift, drop_s, x, rows_i, rows_j, p, 0u, part_of.groups,
       reinterpret_cast<SymSrc<T>*>(&src[0][0]), gbox, own_red, exp_tab);
 }
 
@@ -879,21 +897,6 @@ struct PlanLevels {
   int split;  // 1, 2, 4 or 8
 };
 
-// A workgroup's pair in the plan's list, its part of the pair and the bits of
-// the source groups of that part.  SPLIT = false: whole pairs, all of it
-// constant (at n = 65536 the divisions alone cost a planned FP32 product 3 %).
-template <bool SPLIT>
-struct PairPart {
-  int64_t item;
-  int split, sub;
-  uint32_t groups;
-  __device__ __forceinline__ explicit PairPart(int s)
-      : item(SPLIT ? blockIdx.x / (unsigned)s : blockIdx.x),
-        split(SPLIT ? s : 1),
-        sub(SPLIT ? (int)(blockIdx.x % (unsigned)s) : 0),
-        groups(SPLIT ? ((1u << (kSymGroups / s)) - 1u) << (sub * (kSymGroups / s)) : 0xffu) {}
-};
-
 
 // Element l of a kernel-argument array by selects (no dynamic indexing, so
 // the array stays in the argument segment).
@@ -937,10 +940,9 @@ __global__ __launch_bounds__(kBlock) void kmv_sym_planned_kernel(
   if (centre.w != 0.0f) {
     sym_mfma_pair<KIND, DIM, float>(points, off, n, scale, x, rows_i, rows_j, p, I, J, centre, tmask, part_of.groups, mf);
   } else {
-    sym_valu_pair<float, KIND, DIM, false, true, true, float>(points, off, n, scale, 0.0, 0.0, 0.0, x, rows_i, rows_j, p,
-                                                       bmask[p] & (0x01010101u * part_of.groups),
-                                                       reinterpret_cast<SymSrc<float>*>(mf), nullptr,
-                                                       nullptr, nullptr);
+    sym_valu_pair<float, KIND, DIM, false, true, true, false, float>(
+        points, off, n, scale, 0.0, 0.0, 0.0, x, rows_i, rows_j, p, bmask[p], part_of.groups,
+        reinterpret_cast<SymSrc<float>*>(mf), nullptr, nullptr, nullptr);
   }
 }
 
@@ -1359,12 +1361,6 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 4))) 
 // of <x,x> and <x,y> over its rows (wave butterfly, so a fixed order):
 // dots[b] and dots[gridDim.x + b].
 
-template <typename PT>
-__device__ __forceinline__ double sym_partial(const PT* __restrict__ part_i, const PT* __restrict__ part_j,
-                                              int64_t X, int64_t P, int64_t t) {
-  return P < X ? (double)part_j[sym_pair_index(P, X) * kSymTile + t] : (double)part_i[sym_pair_index(X, P) * kSymTile + t];
-}
-
 // Partials in FP64, or in FP32 where the tile sums are FP32 sums anyway (the
 // planned FP32 kernel); the finish adds them in FP64 either way.
 template <bool LIST, typename PT>
@@ -1413,7 +1409,15 @@ __global__ __launch_bounds__(kBlock) void kmv_sym_finish_kernel(
         for (int u = 0; u < kFinishBatch; ++u) s += v[u];
       }
     } else {
-      for (int64_t P = k; P < ntiles; P += kFinishSlices) s += sym_partial(part_i, part_j, X, P, t);
+      // partners P < X: the pair's row of its tile J; P >= X: a row per part
+      int64_t P = k;
+#pragma unroll 4
+      for (; P < X; P += kFinishSlices) s += (double)part_j[sym_pair_index(P, X) * kSymTile + t];
+      for (; P < ntiles; P += kFinishSlices) {
+        const PT* pi = part_i + sym_pair_index(X, P) * lv.split * kSymTile + t;
+#pragma unroll 8
+        for (int q = 0; q < lv.split; ++q) s += (double)pi[q * kSymTile];
+      }
     }
     __syncthreads();
     red[k][r] = s;
@@ -1463,6 +1467,7 @@ struct SymArgs {
   const int64_t* count;
   const int32_t* slots;  // planned: the plan's slotted partial rows (level 0)
   int64_t pcap;
+  int split;  // workgroups per pair
   // planned FP32 without coincidence shift: the plans' tile data, for the
   // planned kernel (matrix-core form on compact target tiles); null otherwise
   const PlanLevels* lv;
@@ -1472,8 +1477,7 @@ struct SymArgs {
 template <typename T, int KIND, int DIM, int MODE>
 void launch_sym_dim(hipStream_t st, bool coinc, const mplak_kernel_desc* d, const SymArgs& a) {
   const int64_t nt = sym_tiles(d->row_count);
-  const dim3 grid((unsigned)(nt * (nt + 1) / 2));
-  const dim3 parts((unsigned)(nt * (nt + 1) / 2 * (a.lv != nullptr ? a.lv->split : 1)));
+  const dim3 parts((unsigned)(nt * (nt + 1) / 2 * a.split));
   if constexpr (MODE == kSymPlanned && sizeof(T) == 8) {
     if (a.lv != nullptr && !coinc) {
       auto kern = a.lv->split > 1 ? kmv_sym_planned64_kernel<KIND, DIM, true> : kmv_sym_planned64_kernel<KIND, DIM, false>;
@@ -1491,14 +1495,15 @@ void launch_sym_dim(hipStream_t st, bool coinc, const mplak_kernel_desc* d, cons
       return;
     }
   }
-  if (coinc)
-    hipLaunchKernelGGL((kmv_sym_kernel<T, KIND, DIM, true, MODE>), grid, dim3(kBlock), 0, st, d->points,
-                       d->row_offset, d->row_count, a.scale, a.thr, d->coincident_shift, a.drop_s, a.x, a.pi, a.pj,
-                       a.list, a.count, a.slots, a.pcap, a.skip);
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, parts, dim3(kBlock), 0, st, d->points, d->row_offset, d->row_count, a.scale, a.thr,
+                       d->coincident_shift, a.drop_s, a.x, a.pi, a.pj, a.list, a.count, a.slots, a.pcap, a.split,
+                       a.skip);
+  };
+  if (a.split > 1)
+    go(coinc ? kmv_sym_kernel<T, KIND, DIM, true, MODE, true> : kmv_sym_kernel<T, KIND, DIM, false, MODE, true>);
   else
-    hipLaunchKernelGGL((kmv_sym_kernel<T, KIND, DIM, false, MODE>), grid, dim3(kBlock), 0, st, d->points,
-                       d->row_offset, d->row_count, a.scale, a.thr, d->coincident_shift, a.drop_s, a.x, a.pi, a.pj,
-                       a.list, a.count, a.slots, a.pcap, a.skip);
+    go(coinc ? kmv_sym_kernel<T, KIND, DIM, true, MODE, false> : kmv_sym_kernel<T, KIND, DIM, false, MODE, false>);
 }
 
 template <typename T, int KIND, int MODE>
@@ -1531,7 +1536,7 @@ bool sym_eligible(const mplak_kernel_desc* d) {
          sym_tiles(d->row_count) < 65536;  // pair count fits a 1-D grid
 }
 
-// Workgroups per listed pair of a planned product: the largest power of two
+// Workgroups per listed pair of a planned product on 16 x 16 tiles: the largest power of two
 // up to 8 that keeps tile pairs times workgroups below 2400.  A workgroup
 // walks its pair's 16 x 16 tiles one after the other, so with few pairs the
 // launch takes as long as one whole pair (33 us at n = 4096, 36 pairs) on a
@@ -1541,16 +1546,34 @@ bool sym_eligible(const mplak_kernel_desc* d) {
 // n = 24576 35.2 / 33.0 / 36.6 / 47.3 us; from 2400 pairs on (n > 35000) the
 // extra staging and row sets cost more than the balance gives (n = 49152 50.6
 // / 55.8 us).
-inline int sym_split(int64_t nt) {
+inline int planned_split(int64_t nt) {
   const int64_t np = nt * (nt + 1) / 2;
   int k = 1;
   while (k < kSymGroups && np * (2 * k) < 2400) k *= 2;
   return k;
 }
 
+// Workgroups per pair of the vector unit's symmetric products (exact, screened
+// and, with a coincidence shift, planned, whose sums are bitwise the same): the
+// largest power of two up to 8 that keeps pairs times workgroups within 7000, below 820 pairs (n =
+// 20000).  Few whole pairs leave CUs idle or their last round nearly empty.
+// FP64, 3-D Gaussian, at 1 / 2 / 4 / 8 workgroups a pair: n = 5000 60.8 / 35.0 /
+// 24.2 / 21.2 us, n = 16000 140 / 118 / 114 / 110 us.  From 820 pairs on the
+// workspace stays at two row sets a pair, its documented size; there the gain
+// falls from 12 % (n = 20000, 183 / 165 / 162 / 161 us) to nothing (n = 30000,
+// 318 / 322 / 335 / 336 us).
+inline int sym_split(int64_t nt) {
+  const int64_t np = nt * (nt + 1) / 2;
+  int k = 1;
+  if (np < 820)
+    while (k < kSymGroups && np * (2 * k) <= 7000) k *= 2;
+  return k;
+}
+
+// A row set per part for tile I of every pair and one for tile J.
 size_t sym_workspace_bytes(int64_t n) {
   const int64_t nt = sym_tiles(n);
-  return (size_t)2 * (size_t)(nt * (nt + 1) / 2) * kSymTile * sizeof(double);
+  return (size_t)(sym_split(nt) + 1) * (size_t)(nt * (nt + 1) / 2) * kSymTile * sizeof(double);
 }
 
 // Symmetric product: tile-pair kernel (exact, screened or planned) and the
@@ -1561,8 +1584,9 @@ int run_sym(const mplak_kernel_desc* d, int precision, int mode, double drop_s, 
             double* dots = nullptr) {
   SymArgs a;
   const bool coinc = d->coincident_shift != 0.0;
-  // the vector-unit kernel a coincidence shift takes works on whole pairs
-  if (lv != nullptr) lv->split = coinc ? 1 : sym_split(sym_tiles(d->row_count));
+  const int64_t nt = sym_tiles(d->row_count);
+  a.split = mode == kSymPlanned && !coinc ? planned_split(nt) : sym_split(nt);
+  if (lv != nullptr) lv->split = a.split;
   // planned FP32 without coincidence shift: the planned kernel, FP32 partials
   const bool tiles = mode == kSymPlanned && precision == MPLAK_PREC_F32 && lv != nullptr && !coinc;
   // planned FP64 without coincidence shift: the FP64 tile form
@@ -1579,9 +1603,8 @@ int run_sym(const mplak_kernel_desc* d, int precision, int mode, double drop_s, 
   a.slots = lv != nullptr ? lv->slots[0] : nullptr;
   a.pcap = lv != nullptr ? lv->pcap : 0;
   a.skip = skip_if;
-  const int64_t nt = sym_tiles(d->row_count);
   a.pi = static_cast<double*>(work);
-  a.pj = a.pi + (size_t)(nt * (nt + 1) / 2) * kSymTile;
+  a.pj = a.pi + (size_t)(nt * (nt + 1) / 2 * a.split) * kSymTile;
   double* pi = a.pi;
   double* pj = a.pj;
   hipStream_t hs = as_stream(s);
@@ -1603,7 +1626,8 @@ int run_sym(const mplak_kernel_desc* d, int precision, int mode, double drop_s, 
     hipLaunchKernelGGL((kmv_sym_finish_kernel<true, double>), dim3((unsigned)fb), dim3(kBlock), 0, hs, d->row_count,
                        nt, pi, pj, d->nugget, x, y, *lv, pcap, skip_if, dots);
   } else {
-    const PlanLevels none{};
+    PlanLevels none{};
+    none.split = a.split;
     hipLaunchKernelGGL((kmv_sym_finish_kernel<false, double>), dim3((unsigned)fb), dim3(kBlock), 0, hs,
                        d->row_count, nt, pi, pj, d->nugget, x, y, none, 0, skip_if, dots);
   }
@@ -1663,7 +1687,8 @@ PlanLayout plan_layout(int64_t n) {
   L.slots = L.pcount + align_up(sizeof(int32_t) * kFinishSlices * (size_t)nt, 256);
   L.part = L.slots + align_up(sizeof(int32_t) * 2 * np, 256);
   // partial rows: by pair (2 per pair) without a plan, slotted with one
-  const size_t rows = std::max((size_t)2 * np, (size_t)nt * kFinishSlices * (size_t)(L.pcap * sym_split(nt)));
+  const int split = std::max(planned_split(nt), sym_split(nt));
+  const size_t rows = std::max((size_t)2 * np, (size_t)nt * kFinishSlices * (size_t)(L.pcap * split));
   L.total = L.part + rows * kSymTile * sizeof(double);
   return L;
 }

@@ -160,3 +160,44 @@ def test_mrhs_mfma_blocks(lib, rows, cols, row_off, R, dim, prec, bar):
         err = np.linalg.norm(got[:, :rows] - host(ref), axis=1)
         assert np.all(err <= bar * np.linalg.norm(host(mag), axis=1) + 1e-30)
         assert np.all(got[:, rows:] == 7.0)
+
+
+# Exact products around the slab and tile edges of the plain product (square up
+# to 2999 points, rectangular blocks, more than 3 dimensions) and of the
+# symmetric one, whose tile pairs 8, 4, 2 or 1 workgroups share.
+@pytest.mark.parametrize("rows,cols,row_off,dim", [
+    (1, 1, 0, 1), (255, 31, 0, 2), (257, 33, 5, 3), (1000, 2049, 7, 3), (2999, 2999, 0, 2), (700, 17000, 0, 3),
+    (3000, 3000, 0, 5), (3000, 3000, 0, 1), (3073, 3073, 0, 3), (12289, 12289, 0, 2), (20993, 20993, 0, 3),
+    (21505, 21505, 0, 2), (30209, 30209, 0, 3), (42497, 42497, 0, 3)])
+@pytest.mark.parametrize("kind,prec,bar", [(0, 0, 1e-12), (1, 0, 1e-12), (1, 1, 2e-5)])
+@pytest.mark.parametrize("shift", [0.0, 1e-3])
+def test_exact_product_splits(lib, rows, cols, row_off, dim, kind, prec, bar, shift):
+    import ctypes as C
+
+    import torch
+    if shift and rows > 13000:
+        pytest.skip("the coincidence shift takes the same splits; covered at the smaller sizes")
+    g = torch.Generator(device="cuda").manual_seed(rows + cols)
+    n = max(cols, row_off + rows)
+    P = torch.rand((dim, n), generator=g, dtype=torch.float64, device="cuda")
+    x = torch.rand(cols, generator=g, dtype=torch.float64, device="cuda") - 0.5
+    ell, nugget = 0.3, 0.7
+    ref = torch.empty(rows, dtype=torch.float64, device="cuda")
+    mag = torch.empty_like(ref)
+    for i in range(0, rows, 4096):
+        sl = slice(row_off + i, row_off + min(i + 4096, rows))
+        s = sum((P[d, sl, None] - P[d][None, :cols]) ** 2 for d in range(dim))
+        r = (3.0 * s).sqrt() / ell
+        k = (-0.5 * s / ell ** 2).exp() if kind == 0 else (1.0 + r) * (-r).exp()
+        k += shift * (s < 1e-28).double()
+        k[torch.arange(sl.start, sl.stop, device="cuda")[:, None] == torch.arange(cols, device="cuda")[None]] += nugget
+        ref[i:i + 4096], mag[i:i + 4096] = k @ x, k @ x.abs()
+    y = torch.full((rows + 1,), 7.0, dtype=torch.float64, device="cuda")
+    table = torch.tensor([P[d].data_ptr() for d in range(dim)], dtype=torch.int64, device="cuda")
+    desc = _native.mplak_kernel_desc(table.data_ptr(), dim, kind, ell, nugget, shift, row_off, rows, 0, cols)
+    wb = lib.mplak_kernel_matvec_workspace_bytes(C.byref(desc))
+    w = torch.empty(wb, dtype=torch.uint8, device="cuda")
+    ck(lib.mplak_kernel_matvec(C.byref(desc), prec, x.data_ptr(), y.data_ptr(), w.data_ptr(), wb, None, stream()))
+    got = host(y)
+    assert np.all(np.abs(got[:rows] - host(ref)) <= bar * host(mag))
+    assert got[rows] == 7.0
