@@ -351,6 +351,29 @@ int mplak_hm_apply_pairs(const mplak_hm_chunk* chunks, int64_t nchunks, const in
                          const int32_t* rank, int32_t kmax, const double* U, const double* t, double* ys,
                          mplak_stream_t stream);
 
+/* The symmetric product in three launches that each use the memory system
+ * and the vector unit at once: mplak_hm_far_near is mplak_hm_far_partials (into
+ * fpart) beside mplak_hm_near_pairs of some of the pairs; mplak_hm_rows_near
+ * writes ys[row] = sum over the row leaf's admissible blocks of U_b(row, :) t_b
+ * beside more pairs; mplak_hm_pairs_finish adds the near partials (as
+ * mplak_hm_apply_pairs) and, with perm, the nugget and the caller's row order (as
+ * mplak_hm_scatter_nugget), otherwise the sums are left in ys.  npairs or the
+ * other part may be 0.  stream_factors: nonzero reads the factors
+ * nontemporally, for factors that exceed the 256 MiB Infinity Cache. */
+int mplak_hm_far_near(const mplak_hm_points* pts, const mplak_hm_block* blocks, const mplak_hm_item* items,
+                      int64_t nitems, const int32_t* rank, int32_t kmax, const double* V, const double* xs,
+                      double* fpart, const mplak_hm_pair* pairs, int64_t npairs, double* part, int32_t stream_factors,
+                      mplak_stream_t stream);
+int mplak_hm_rows_near(const mplak_hm_points* pts, const mplak_hm_chunk* chunks, int64_t nchunks,
+                       const int64_t* far_ptr, const int32_t* far_blk, const mplak_hm_block* blocks,
+                       const int32_t* rank, int32_t kmax, const double* U, const double* t, double* ys,
+                       const double* xs, const mplak_hm_pair* pairs, int64_t npairs, double* part,
+                       int32_t stream_factors, mplak_stream_t stream);
+int mplak_hm_pairs_finish(const mplak_hm_chunk* chunks, int64_t nchunks, const int64_t* chunk_near,
+                          const int64_t* near_start, const int64_t* ent_ptr, const int64_t* ent, const double* part,
+                          double* ys, const int64_t* perm, double nugget, const double* x, int64_t shift,
+                          int64_t x_count, double* y, mplak_stream_t stream);
+
 /* The apply of mplak_hm_apply with the inadmissible blocks' entries read
  * from `stored` instead of evaluated: near range k (CSR order) of leaf l
  * holds entry (i, j) at stored[near_off[k] + (i - lo_l) + j m_l], with

@@ -192,26 +192,47 @@ __global__ __launch_bounds__(kHmThreads) void aca_kernel(E e, const mplak_hm_blo
   aca_block(e, B, kmax, eps, U, V, rank + blockIdx.x, tab);
 }
 
+// Factors are read once per product: nontemporally where the two together
+// exceed the 256 MiB Infinity Cache (STREAM), so that they do not churn it.
+template <bool STREAM>
+__device__ __forceinline__ double factor_load(const double* p) {
+  if constexpr (STREAM) return __builtin_nontemporal_load(p);
+  else return *p;
+}
+
 // Far field for the rows of an apply item: sum over the leaf's admissible
-// blocks b (those of part `part` of kHmParts) of U_b(row - r0_b, :) t_b.
+// blocks b (those of part `part` of `parts`, wave-uniform) of
+// U_b(row - r0_b, :) t_b, kHmTerms terms of both rows in flight at a time.
+constexpr int kHmTerms = 8;
+
+template <bool STREAM>
 __device__ __forceinline__ void far_rows(const int64_t (&row)[kHmLaneRows], const bool (&valid)[kHmLaneRows],
                                          const int64_t* __restrict__ far_ptr, const int32_t* __restrict__ far_blk,
                                          int32_t leaf, const mplak_hm_block* __restrict__ blocks,
                                          const int32_t* __restrict__ rank, int kmax, const double* __restrict__ U,
-                                         const double* __restrict__ t, int part, double (&acc)[kHmLaneRows]) {
+                                         const double* __restrict__ t, int part, int parts,
+                                         double (&acc)[kHmLaneRows]) {
   const int64_t f0 = far_ptr[leaf], f1 = far_ptr[leaf + 1];
-  for (int64_t f = f0 + part; f < f1; f += kHmParts) {
-    const int32_t b = far_blk[f];
+  for (int64_t f = f0 + part; f < f1; f += parts) {
+    const int32_t b = __builtin_amdgcn_readfirstlane(far_blk[f]);
     const mplak_hm_block B = blocks[b];
     const int rb = rank[b];
     const double* tb = t + (int64_t)b * kmax;
+    const double* u[kHmLaneRows];
 #pragma unroll
-    for (int h = 0; h < kHmLaneRows; ++h) {
-      if (!valid[h]) continue;
-      const double* u = U + B.uoff + (row[h] - B.r0);
-      double a = acc[h];
-      for (int q = 0; q < rb; ++q) a = fma(u[q * B.m], tb[q], a);
-      acc[h] = a;
+    for (int h = 0; h < kHmLaneRows; ++h) u[h] = U + B.uoff + (row[h] - B.r0);  // rows past the item: its first
+    for (int q0 = 0; q0 < rb; q0 += kHmTerms) {
+      double v[kHmLaneRows][kHmTerms];
+#pragma unroll
+      for (int q = 0; q < kHmTerms; ++q)
+#pragma unroll
+        for (int h = 0; h < kHmLaneRows; ++h)
+          if (q0 + q < rb) v[h][q] = factor_load<STREAM>(u[h] + (q0 + q) * B.m);
+#pragma unroll
+      for (int q = 0; q < kHmTerms; ++q)
+#pragma unroll
+        for (int h = 0; h < kHmLaneRows; ++h)
+          if (q0 + q < rb) acc[h] = valid[h] ? fma(v[h][q], tb[q0 + q], acc[h]) : acc[h];
     }
   }
 }
@@ -267,7 +288,7 @@ __global__ __launch_bounds__(kHmApplyThreads) void apply_kernel(
   const int dim = DIM > 0 ? DIM : e.dim;
   fill_exp2_table(tab);
   const mplak_hm_chunk c = chunks[blockIdx.x];
-  const int part = threadIdx.x / kWave;
+  const int part = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   int64_t row[kHmLaneRows];
   bool valid[kHmLaneRows];
   item_rows(c, row, valid);
@@ -312,7 +333,7 @@ __global__ __launch_bounds__(kHmApplyThreads) void apply_kernel(
       }
     }
   }
-  far_rows(row, valid, far_ptr, far_blk, c.leaf, blocks, rank, kmax, U, t, part, acc);
+  far_rows<false>(row, valid, far_ptr, far_blk, c.leaf, blocks, rank, kmax, U, t, part, kHmParts, acc);
   finish_rows(acc, row, valid, ys, red);
 }
 
@@ -332,7 +353,7 @@ __global__ __launch_bounds__(kHmApplyThreads) void apply_generic_kernel(
     __syncthreads();
   }
   const mplak_hm_chunk c = chunks[blockIdx.x];
-  const int part = threadIdx.x / kWave;
+  const int part = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   int64_t row[kHmLaneRows];
   bool valid[kHmLaneRows];
   item_rows(c, row, valid);
@@ -347,7 +368,7 @@ __global__ __launch_bounds__(kHmApplyThreads) void apply_generic_kernel(
       for (int64_t s = part; s < cn; s += kHmParts) acc[h] = fma(e(row[h], c0 + s, tab), xs[c0 + s], acc[h]);
     }
   }
-  far_rows(row, valid, far_ptr, far_blk, c.leaf, blocks, rank, kmax, U, t, part, acc);
+  far_rows<false>(row, valid, far_ptr, far_blk, c.leaf, blocks, rank, kmax, U, t, part, kHmParts, acc);
   finish_rows(acc, row, valid, ys, red);
 }
 
@@ -386,7 +407,7 @@ __global__ __launch_bounds__(kHmApplyThreads) void apply_stored_kernel(
     double* __restrict__ ys) {
   __shared__ double red[kHmParts][kHmRows];
   const mplak_hm_chunk c = chunks[blockIdx.x];
-  const int part = threadIdx.x / kWave;
+  const int part = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   int64_t row[kHmLaneRows];
   bool valid[kHmLaneRows];
   item_rows(c, row, valid);
@@ -405,7 +426,7 @@ __global__ __launch_bounds__(kHmApplyThreads) void apply_stored_kernel(
         if (valid[h]) acc[h] = fma(a[(row[h] - lo) + s * m], xv, acc[h]);
     }
   }
-  far_rows(row, valid, far_ptr, far_blk, c.leaf, blocks, rank, kmax, U, t, part, acc);
+  far_rows<false>(row, valid, far_ptr, far_blk, c.leaf, blocks, rank, kmax, U, t, part, kHmParts, acc);
   finish_rows(acc, row, valid, ys, red);
 }
 

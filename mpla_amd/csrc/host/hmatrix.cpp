@@ -186,6 +186,7 @@ struct HMatrix {
   double* near_st = nullptr;
   int64_t *near_off = nullptr, *leaf_range = nullptr;
   int64_t nblocks = 0, nitems = 0, nchunks = 0;
+  int32_t stream_factors = 0;  // the factors exceed the Infinity Cache
   double** coords_host[2] = {nullptr, nullptr};  // the h_matrix_data coords_d arrays
 };
 
@@ -404,6 +405,7 @@ void setup(mpla_generic_matrix* A, h_matrix_data* data, HMatrix* h, const std::v
              factor_bytes / 1e9, (double)free_b / 1e9);
     fail(what, msg);
   }
+  h->stream_factors = factor_bytes > (double)(int64_t(256) << 20);
   h->perm_r = upload(h, rt.perm, s);
   h->perm_c = upload(h, ct.perm, s);
   std::vector<int64_t> g(h->nr);
@@ -570,6 +572,24 @@ void apply(HMatrix* h, bool full, const double* x, double* y, mpla_instance* ins
   if (h->nr == 0) return;
   if (h->nc > 0) ck(mplak_gather_f64(h->xs, x, h->perm_c, h->nc, s), what);
   const bool far = !full && h->nblocks > 0;
+  if (h->closed_form && !full && h->npairs > 0) {
+    // half of the near pairs beside each of the far field's two launches
+    const mplak_hm_points p = points_of(h);
+    const int64_t first = far ? h->npairs / 2 : h->npairs, rest = h->npairs - first;
+    const int64_t nitems = far ? h->nitems : 0;
+    ck(mplak_hm_far_near(&p, h->blocks, h->items, nitems, h->rank, h->kmax, h->V, h->xs, h->fpart, h->pairs, first,
+                         h->pair_part, h->stream_factors, s),
+       what);
+    if (far) ck(mplak_hm_far_sum(h->first_item, h->nblocks, h->rank, h->kmax, h->fpart, h->t, s), what);
+    ck(mplak_hm_rows_near(&p, h->chunks, h->nchunks, far ? h->far_ptr : h->nofar_ptr, h->far_blk, h->blocks, h->rank,
+                          h->kmax, h->U, h->t, h->ys, h->xs, h->pairs + first, rest,
+                          h->pair_part + 2 * first * kNearChunk, h->stream_factors, s),
+       what);
+    ck(mplak_hm_pairs_finish(h->chunks, h->nchunks, h->chunk_near, h->near_start, h->ent_ptr, h->ent, h->pair_part,
+                             h->ys, h->perm_r, h->nugget, x, h->row_off - h->col_off, h->nc, y, s),
+       what);
+    return;
+  }
   if (far) {
     ck(mplak_hm_far_partials(h->blocks, h->items, h->nitems, h->rank, h->kmax, h->V, h->xs, h->fpart, s), what);
     ck(mplak_hm_far_sum(h->first_item, h->nblocks, h->rank, h->kmax, h->fpart, h->t, s), what);
@@ -577,13 +597,7 @@ void apply(HMatrix* h, bool full, const double* x, double* y, mpla_instance* ins
   const int64_t* np = full ? h->full_ptr : h->near_ptr;
   const int64_t* nc = full ? h->full_cols : h->near_cols;
   const int64_t* fp = far ? h->far_ptr : h->nofar_ptr;
-  if (h->closed_form && !full && h->npairs > 0) {
-    const mplak_hm_points p = points_of(h);
-    ck(mplak_hm_near_pairs(&p, h->pairs, h->npairs, h->xs, h->pair_part, s), what);
-    ck(mplak_hm_apply_pairs(h->chunks, h->nchunks, h->chunk_near, h->near_start, h->ent_ptr, h->ent, h->pair_part,
-                            fp, h->far_blk, h->blocks, h->rank, h->kmax, h->U, h->t, h->ys, s),
-       what);
-  } else if (h->closed_form) {
+  if (h->closed_form) {
     const mplak_hm_points p = points_of(h);
     ck(mplak_hm_apply(&p, h->chunks, h->nchunks, np, nc, fp, h->far_blk, h->blocks, h->rank, h->kmax, h->U, h->t,
                       h->xs, h->ys, s),

@@ -201,3 +201,49 @@ def test_exact_product_splits(lib, rows, cols, row_off, dim, kind, prec, bar, sh
     got = host(y)
     assert np.all(np.abs(got[:rows] - host(ref)) <= bar * host(mag))
     assert got[rows] == 7.0
+
+
+# Near pairs: chunks around the 64-point groups and 128-row blocks, diagonal pairs
+# (symmetric inside), alone and beside far-field items of 1 to 32 terms whose
+# columns end inside a wave's pairs of columns.
+@pytest.mark.parametrize("am,bm,terms,cols", [(1, 1, 1, 1), (63, 65, 4, 127), (64, 128, 5, 128), (129, 300, 16, 129),
+                                              (312, 313, 20, 511), (512, 511, 21, 1025), (500, 512, 32, 300)])
+@pytest.mark.parametrize("kind,dim", [(0, 1), (1, 2), (0, 3), (1, 4)])
+def test_hmatrix_near_pairs_and_far_items(lib, am, bm, terms, cols, kind, dim):
+    import ctypes as C
+
+    import torch
+    rng = np.random.default_rng(am * 7 + bm + terms)
+    n = max(am + bm, cols + 3)
+    P, x = rng.random((dim, n)) * 3.0, rng.standard_normal(n)  # coordinates already scaled
+    s = sum((P[d, :, None] - P[d, None, :]) ** 2 for d in range(dim))
+    K = np.exp2(-s) if kind == 0 else (1.0 + np.sqrt(s)) * np.exp(-np.sqrt(s))
+    V = rng.standard_normal((terms, cols))
+    pairs = np.array([[0, am, am, bm], [0, am, 0, am], [am, bm, am, bm]], dtype=np.int64)
+    block = np.array([[0, 1, 3, cols, 0, 0]], dtype=np.int64)
+    half = cols // 2
+    items = np.array([[0, 0, half], [0, half, cols - half]], dtype=np.int64)
+    P_dev, x_dev, V_dev = dev(P), dev(x), dev(V)
+    pairs_dev, block_dev, items_dev = (torch.as_tensor(v, device="cuda") for v in (pairs, block, items))
+    rank = torch.full((1,), terms, dtype=torch.int32, device="cuda")
+    part = torch.full((3, 2, 512), 7.0, dtype=torch.float64, device="cuda")
+    fpart = torch.full((2, 32), 7.0, dtype=torch.float64, device="cuda")
+
+    class Points(C.Structure):
+        _fields_ = [("rows", C.c_void_p), ("cols", C.c_void_p), ("row_ld", C.c_int64), ("col_ld", C.c_int64),
+                    ("dim", C.c_int32), ("kind", C.c_int32)]
+
+    pts = Points(P_dev.data_ptr(), P_dev.data_ptr(), n, n, dim, kind)
+    for stream_factors in (0, 1):
+        ck(lib.mplak_hm_far_near(C.byref(pts), block_dev.data_ptr(), items_dev.data_ptr(), 2, rank.data_ptr(), 32,
+                                 V_dev.data_ptr(), x_dev.data_ptr(), fpart.data_ptr(), pairs_dev.data_ptr(), 3,
+                                 part.data_ptr(), stream_factors, stream()))
+        got, far = host(part), host(fpart)
+        a, b = slice(0, am), slice(am, am + bm)
+        for k, side, rows, src in ((0, 0, a, b), (0, 1, b, a), (1, 0, a, a), (2, 0, b, b)):
+            y, m = K[rows, src] @ x[src], np.abs(K[rows, src]) @ np.abs(x[src])
+            assert np.all(np.abs(got[k, side, :y.size] - y) <= 1e-12 * m)  # the oracle's FP64 bar
+        for i, cs in enumerate((slice(0, half), slice(half, cols))):
+            t, m = V[:, cs] @ x[3:][cs], np.abs(V[:, cs]) @ np.abs(x[3:][cs])
+            assert np.all(np.abs(far[i, :terms] - t) <= (cols + 8) * EPS * m)
+            assert np.all(far[i, terms:] == 7.0)
