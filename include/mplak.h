@@ -545,7 +545,7 @@ typedef struct mplak_ragged_system {
                             reference counterpart); 0: exact product */
   double drop_s;         /* planned */
   int32_t scheme;        /* planned: MPLAK_RAGGED_SLABS or MPLAK_RAGGED_PAIRS */
-  int32_t reserved;
+  int32_t reserved;      /* planned: workgroups per tile pair (0 and 1: one) */
 } mplak_ragged_system;
 
 /* Work split of a ragged product.
@@ -572,6 +572,12 @@ typedef struct mplak_ragged_item {
  * needs. */
 size_t mplak_ragged_plan(mplak_ragged_system* s);
 
+/* Host only: the same for mplak_ragged_product_mixed (FP32) and, by class, FP64
+ * products of the same system: pairs from n = 2048, shared by up to 8 workgroups
+ * each (`reserved`; the item's slab field is the part), shorter slabs, and FP32
+ * column tiles of min(nrhs, 8). */
+size_t mplak_ragged_plan_mixed(mplak_ragged_system* s);
+
 /* Host only: number of product / finish work items of a planned system; when
  * `out` is non-NULL also writes them (sys field = sys_index). */
 int64_t mplak_ragged_product_items(const mplak_ragged_system* s, mplak_ragged_item* out, int32_t sys_index);
@@ -585,6 +591,10 @@ int64_t mplak_ragged_finish_items(const mplak_ragged_system* s, mplak_ragged_ite
  * are left undone), 0 for any mix of dimensions (SLABS only). */
 int mplak_ragged_product(const mplak_ragged_system* systems, const mplak_ragged_item* items, int64_t count, int rt,
                          int dim, int precision, int scheme, mplak_stream_t stream);
+/* FP32 product partials for the items of any mix of systems planned by
+ * mplak_ragged_plan_mixed, in one launch. */
+int mplak_ragged_product_mixed(const mplak_ragged_system* systems, const mplak_ragged_item* items, int64_t count,
+                               mplak_stream_t stream);
 int mplak_ragged_finish(const mplak_ragged_system* systems, const mplak_ragged_item* items, int64_t count,
                         mplak_stream_t stream);
 

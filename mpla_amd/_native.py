@@ -201,6 +201,8 @@ MPLAK_SIGNATURES = {
     "mplak_bcg_iterate": (C.c_int, [_i64, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
     "mplak_bcg_copy_states": (C.c_int, [_vp, _vp, _i64, _vp, _vp]),
     "mplak_ragged_plan": (_sz, [_vp]),
+    "mplak_ragged_plan_mixed": (_sz, [_vp]),
+    "mplak_ragged_product_mixed": (C.c_int, [_vp, _vp, _i64, _vp]),
     "mplak_ragged_product_items": (_i64, [_vp, _vp, _i32]),
     "mplak_ragged_finish_items": (_i64, [_vp, _vp, _i32]),
     "mplak_ragged_product": (C.c_int, [_vp, _vp, _i64, C.c_int, C.c_int, C.c_int, C.c_int, _vp]),

@@ -90,7 +90,7 @@ Layout layout_for(int64_t n, int dim, int nrhs) {
   s.kind = MPLAK_KERNEL_GAUSSIAN;
   s.length_scale = 1.0;
   s.precision = MPLAK_PREC_F64;
-  L.part = align256(mplak_ragged_plan(&s));
+  L.part = align256(mplak_ragged_plan_mixed(&s));
   L.cgpart = align256(mplak_ragged_cg_part_bytes(n, nrhs));
   L.perm = align256(sizeof(int64_t) * (size_t)n);
   L.total = L.points + 6 * L.vec + L.part + L.cgpart + L.perm;  // points, B, X, R, D, Z, E, spatial order
@@ -122,7 +122,7 @@ struct Upload {
   std::vector<mplak_ragged_cg> csys;
   std::vector<mplak_ragged_item> items;
   struct Launch {
-    int kind;  // 0 product, 1 finish, 2 cg op
+    int kind;  // 0 product of one class, 1 finish, 2 cg op, 3 FP32 product of any mix
     int op;    // cg op; for a product, the systems' dimension
     int rt, precision, parity;
     double value;
@@ -204,6 +204,8 @@ void submit_upload(mpla_server* s, Upload& u) {
     const mplak_ragged_item* it = dit + L.first;
     if (L.kind == 0)
       ck(mplak_ragged_product(dps, it, L.count, L.rt, L.op, L.precision, L.scheme, s->stream), "server product");
+    else if (L.kind == 3)
+      ck(mplak_ragged_product_mixed(dps, it, L.count, s->stream), "server product");
     else if (L.kind == 1)
       ck(mplak_ragged_finish(dps, it, L.count, s->stream), "server finish");
     else
@@ -229,7 +231,7 @@ mplak_ragged_system product_system(const Request& r, int precision, const double
   sy.kind = r.req.kind;
   sy.nrhs = r.req.nrhs;
   sy.precision = precision;
-  mplak_ragged_plan(&sy);
+  mplak_ragged_plan_mixed(&sy);
   return sy;
 }
 
@@ -251,11 +253,26 @@ mplak_ragged_cg cg_system(mpla_server* s, const Request& r, double* X, double* X
   return c;
 }
 
-// Adds product launches (grouped by rt) and the finish launch for `systems`.
+// Adds the product launches and the finish launch for `systems`.
 void add_products(Upload& u, const std::vector<mplak_ragged_system>& systems, int precision) {
   if (systems.empty()) return;
   const size_t base = u.psys.size();
   for (const auto& sy : systems) u.psys.push_back(sy);
+  auto add_items = [&](size_t k) {
+    const int64_t c = mplak_ragged_product_items(&systems[k], nullptr, 0);
+    const size_t at = u.items.size();
+    u.items.resize(at + (size_t)c);
+    mplak_ragged_product_items(&systems[k], u.items.data() + at, (int32_t)(base + k));
+  };
+  if (precision == MPLAK_PREC_F32) {
+    // one launch for every system, the largest first
+    std::vector<size_t> order(systems.size());
+    for (size_t k = 0; k < order.size(); ++k) order[k] = k;
+    std::stable_sort(order.begin(), order.end(), [&](size_t a, size_t b) { return systems[a].n > systems[b].n; });
+    const size_t first = u.items.size();
+    for (size_t k : order) add_items(k);
+    u.launches.push_back({3, 0, 0, precision, 0, 0.0, first, (int64_t)(u.items.size() - first)});
+  } else
   // one launch per (scheme, rt, dim) class: kernels specialised for each;
   // the pair scheme (large systems, heavier items) first
   for (int scheme : {MPLAK_RAGGED_PAIRS, MPLAK_RAGGED_SLABS})
@@ -263,11 +280,7 @@ void add_products(Upload& u, const std::vector<mplak_ragged_system>& systems, in
       for (int dim = 1; dim <= MPLA_SERVER_MAX_DIM; ++dim) {
         const size_t first = u.items.size();
         for (size_t k = 0; k < systems.size(); ++k) {
-          if (systems[k].scheme != scheme || systems[k].rt != rt || systems[k].dim != dim) continue;
-          const int64_t c = mplak_ragged_product_items(&systems[k], nullptr, 0);
-          const size_t at = u.items.size();
-          u.items.resize(at + (size_t)c);
-          mplak_ragged_product_items(&systems[k], u.items.data() + at, (int32_t)(base + k));
+          if (systems[k].scheme == scheme && systems[k].rt == rt && systems[k].dim == dim) add_items(k);
         }
         const int64_t count = (int64_t)(u.items.size() - first);
         if (count > 0) u.launches.push_back({0, dim, rt, precision, 0, 0.0, first, count, scheme});

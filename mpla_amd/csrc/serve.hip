@@ -21,6 +21,7 @@
 #include <math.h>
 #include <stdlib.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "common.hpp"
@@ -42,19 +43,23 @@ inline int vec_blocks_r(int64_t n) {
 
 inline int rt_class(int64_t R) { return R <= 1 ? 1 : (R <= 2 ? 2 : (R <= 4 ? 4 : 8)); }
 
-// DIM > 0: every system of the launch has that dimension; DIM == 0: any
-// dimension <= kMaxRaggedDim (coordinates past it are zero).
+// LDS of the product of a slab item: sources, values, chunk boxes and the
+// FP64 exponential's table.
+template <typename T, int RT, int MD>
+struct SlabLds {
+  T lp[MD][kChunk];
+  T lv[RT][kChunk];
+  T cbox[kBlock / kWave][2 * MD];
+  double exp_tab[Exp2Lds<T>::size];
+};
+
+// DIM > 0: the system has that dimension; DIM == 0: any dimension <=
+// kMaxRaggedDim (coordinates past it are zero).
 template <typename T, int RT, int DIM>
-__global__ __launch_bounds__(kBlock) void ragged_product_kernel(const mplak_ragged_system* __restrict__ systems,
-                                                                const mplak_ragged_item* __restrict__ items) {
+__device__ __forceinline__ void slab_item(const mplak_ragged_item& it, const mplak_ragged_system& S, void* lds_raw) {
   constexpr int MD = DIM > 0 ? DIM : kMaxRaggedDim;
-  const mplak_ragged_item it = items[blockIdx.x];
-  const mplak_ragged_system S = systems[it.sys];
-  if (S.skip != nullptr && *S.skip != 0) return;
-  __shared__ T lp[MD][kChunk];
-  __shared__ T lv[RT][kChunk];
-  __shared__ double exp_tab[Exp2Lds<T>::size];
-  if (sizeof(T) == 8) fill_exp2_table(exp_tab);  // first read after the chunk barrier below
+  auto& lds = *static_cast<SlabLds<T, RT, MD>*>(lds_raw);
+  if (sizeof(T) == 8) fill_exp2_table(lds.exp_tab);  // first read after the chunk barrier below
   const int tid = threadIdx.x;
   const int64_t n = S.n;
   const int dim = S.dim;
@@ -74,7 +79,6 @@ __global__ __launch_bounds__(kBlock) void ragged_product_kernel(const mplak_ragg
   // within a kept chunk each 64-source part whose box is that far.
   const bool screen = S.drop_s > 0.0;
   const int lane = tid & (kWave - 1), w = tid / kWave;
-  __shared__ T cbox[kBlock / kWave][2 * MD];
   T tbox[2 * MD];
   if (screen) {
 #pragma unroll
@@ -90,17 +94,17 @@ __global__ __launch_bounds__(kBlock) void ragged_product_kernel(const mplak_ragg
     __syncthreads();
     const int64_t j = cb + tid;
 #pragma unroll
-    for (int d = 0; d < MD; ++d) lp[d][tid] = (j < c1 && d < dim) ? (T)(S.points[d * n + j] * S.scale) : T(0);
+    for (int d = 0; d < MD; ++d) lds.lp[d][tid] = (j < c1 && d < dim) ? (T)(S.points[d * n + j] * S.scale) : T(0);
 #pragma unroll
-    for (int q = 0; q < RT; ++q) lv[q][tid] = (j < c1 && r0 + q < R) ? (T)S.V[(r0 + q) * n + j] : T(0);
+    for (int q = 0; q < RT; ++q) lds.lv[q][tid] = (j < c1 && r0 + q < R) ? (T)S.V[(r0 + q) * n + j] : T(0);
     if (screen) {  // this wave's part of the chunk box; sources past the slab do not count
 #pragma unroll
       for (int d = 0; d < MD; ++d) {
-        const T lo = wave_min(j < c1 ? lp[d][tid] : (T)INFINITY);
-        const T hi = wave_max(j < c1 ? lp[d][tid] : (T)-INFINITY);
+        const T lo = wave_min(j < c1 ? lds.lp[d][tid] : (T)INFINITY);
+        const T hi = wave_max(j < c1 ? lds.lp[d][tid] : (T)-INFINITY);
         if (lane == 0) {
-          cbox[w][d] = lo;
-          cbox[w][MD + d] = hi;
+          lds.cbox[w][d] = lo;
+          lds.cbox[w][MD + d] = hi;
         }
       }
     }
@@ -109,11 +113,11 @@ __global__ __launch_bounds__(kBlock) void ragged_product_kernel(const mplak_ragg
       T d2 = T(0);
 #pragma unroll
       for (int d = 0; d < MD; ++d) {
-        T lo = cbox[0][d], hi = cbox[0][MD + d];
+        T lo = lds.cbox[0][d], hi = lds.cbox[0][MD + d];
 #pragma unroll
         for (int q = 1; q < kBlock / kWave; ++q) {
-          lo = fmin(lo, cbox[q][d]);
-          hi = fmax(hi, cbox[q][MD + d]);
+          lo = fmin(lo, lds.cbox[q][d]);
+          hi = fmax(hi, lds.cbox[q][MD + d]);
         }
         const T gap = fmax(T(0), fmax(lo - tbox[MD + d], tbox[d] - hi));
         d2 = fma(gap, gap, d2);
@@ -121,15 +125,17 @@ __global__ __launch_bounds__(kBlock) void ragged_product_kernel(const mplak_ragg
       if (__builtin_amdgcn_readfirstlane((int)(d2 > (T)S.drop_s)) != 0) continue;
     }
     // then per 64-source part of the chunk (wave q staged part q and its box):
-    // the wave skips the parts whose box is too far from its targets
-    uint32_t far_parts = 0;
+    // the wave skips the parts whose box is too far from its targets, and those
+    // past the slab
+    const int parts = (int)((std::min<int64_t>(c1 - cb, kChunk) + kWave - 1) / kWave);
+    uint32_t far_parts = ~0u << parts;
     if (screen) {
 #pragma unroll
       for (int q = 0; q < kBlock / kWave; ++q) {
         T d2 = T(0);
 #pragma unroll
         for (int d = 0; d < MD; ++d) {
-          const T gap = fmax(T(0), fmax(cbox[q][d] - tbox[MD + d], tbox[d] - cbox[q][MD + d]));
+          const T gap = fmax(T(0), fmax(lds.cbox[q][d] - tbox[MD + d], tbox[d] - lds.cbox[q][MD + d]));
           d2 = fma(gap, gap, d2);
         }
         if (__builtin_amdgcn_readfirstlane((int)(d2 > (T)S.drop_s)) != 0) far_parts |= 1u << q;
@@ -138,21 +144,30 @@ __global__ __launch_bounds__(kBlock) void ragged_product_kernel(const mplak_ragg
     T cacc[RT];
 #pragma unroll
     for (int q = 0; q < RT; ++q) cacc[q] = T(0);
+    // specialised per kernel function (uniform over the workgroup)
+    auto run = [&](auto kind_c) {
+      constexpr int KIND = decltype(kind_c)::value;
 #pragma unroll 1
-    for (int part = 0; part < kBlock / kWave; ++part) {
-      if ((far_parts >> part) & 1u) continue;
-      for (int jj = part * kWave; jj < (part + 1) * kWave; ++jj) {
-        T s = T(0);
+      for (int part = 0; part < kBlock / kWave; ++part) {
+        if ((far_parts >> part) & 1u) continue;
+#pragma unroll 2
+        for (int jj = part * kWave; jj < (part + 1) * kWave; ++jj) {
+          T s = T(0);
 #pragma unroll
-        for (int d = 0; d < MD; ++d) {
-          const T df = pi[d] - lp[d][jj];
-          s = fma(df, df, s);
+          for (int d = 0; d < MD; ++d) {
+            const T df = pi[d] - lds.lp[d][jj];
+            s = fma(df, df, s);
+          }
+          const T k = kernel_entry<T, KIND>(s, lds.exp_tab);
+#pragma unroll
+          for (int q = 0; q < RT; ++q) cacc[q] = fma(k, lds.lv[q][jj], cacc[q]);
         }
-        const T k = kernel_entry_rt<T>(S.kind, s, exp_tab);
-#pragma unroll
-        for (int q = 0; q < RT; ++q) cacc[q] = fma(k, lv[q][jj], cacc[q]);
       }
-    }
+    };
+    if (S.kind == MPLAK_KERNEL_GAUSSIAN)
+      run(std::integral_constant<int, MPLAK_KERNEL_GAUSSIAN>{});
+    else
+      run(std::integral_constant<int, MPLAK_KERNEL_MATERN32>{});
 #pragma unroll
     for (int q = 0; q < RT; ++q) acc[q] += (double)cacc[q];
   }
@@ -161,6 +176,16 @@ __global__ __launch_bounds__(kBlock) void ragged_product_kernel(const mplak_ragg
     for (int q = 0; q < RT; ++q)
       if (r0 + q < R) S.part[((int64_t)it.slab * R + r0 + q) * n + i] = acc[q];
   }
+}
+
+template <typename T, int RT, int DIM>
+__global__ __launch_bounds__(kBlock) void ragged_product_kernel(const mplak_ragged_system* __restrict__ systems,
+                                                                const mplak_ragged_item* __restrict__ items) {
+  const mplak_ragged_item it = items[blockIdx.x];
+  const mplak_ragged_system S = systems[it.sys];
+  if (S.skip != nullptr && *S.skip != 0) return;
+  __shared__ SlabLds<T, RT, (DIM > 0 ? DIM : kMaxRaggedDim)> lds;
+  slab_item<T, RT, DIM>(it, S, &lds);
 }
 
 // ---- pair scheme ------------------------------------------------------------
@@ -175,15 +200,24 @@ __global__ __launch_bounds__(kBlock) void ragged_product_kernel(const mplak_ragg
 // The four waves' column sums of a group are added in wave order (FP64) and
 // stored; the diagonal pair evaluates its whole block for the row sums.
 //
-// Partials (entry precision T): rows of I at part_i[(p R + r) 512 + k], rows
-// of J at part_j[...] (same shape, after part_i), one flag per pair after
-// both: 0 when every 128 x 64 block of the pair is screened out (nothing else
-// written), 1 otherwise.  The finish adds, for a row of tile X, the pairs
-// (X, P) over P = 0 .. tiles - 1 in order.
+// A system planned for mixed launches may split its pairs: part u of `split`
+// works on source groups u 8 / split .. of tile J (the item's slab field).
+//
+// Partials (entry precision T): rows of I at part_i[((p split + u) R + r) 512 +
+// k], rows of J at part_j[(p R + r) 512 + k] (after part_i; each part writes its
+// groups), one flag per pair and part after both: 0 when every 128 x 64 block of
+// it is screened out (nothing else written), 1 otherwise.  The finish adds, for
+// a row of tile X, the pairs (X, P) over P = 0 .. tiles - 1 in order and their
+// parts in order.
 
 constexpr int kPairTile = 2 * kBlock;
 constexpr int kPairGroups = kPairTile / kWave;
 constexpr int64_t kRagPairMinN = 8192;
+// In mixed launches, where pairs are split and the chip is shared, evaluating
+// an entry once for both of its rows pays from fewer points (alone, an FP32
+// product of 2000 points takes 9.3 us either way, one of 4000 11.9 us in pairs
+// and 12.1 us in slabs).
+constexpr int64_t kMixedPairMinN = 2048;
 
 __host__ __device__ inline int64_t pair_count(int64_t tiles) { return tiles * (tiles + 1) / 2; }
 
@@ -191,32 +225,45 @@ template <typename T>
 __device__ __forceinline__ T* pair_rows(const mplak_ragged_system& S) {
   return reinterpret_cast<T*>(S.part);
 }
+__host__ __device__ inline int pair_split(const mplak_ragged_system& S) { return S.reserved > 1 ? S.reserved : 1; }
 template <typename T>
 __device__ __forceinline__ int32_t* pair_flags(const mplak_ragged_system& S) {
-  const int64_t bytes = 2 * pair_count(S.tiles) * (int64_t)S.nrhs * kPairTile * (int64_t)sizeof(T);
+  const int64_t bytes =
+      (pair_split(S) + 1) * pair_count(S.tiles) * (int64_t)S.nrhs * kPairTile * (int64_t)sizeof(T);
   return reinterpret_cast<int32_t*>(reinterpret_cast<char*>(S.part) + (bytes + 255) / 256 * 256);
 }
 
+// LDS of a pair item.  The values of a source are padded to an even count, so
+// that the rotated reads stay 8-byte aligned.
 template <typename T, int RT, int DIM>
-__global__ __launch_bounds__(kBlock) void ragged_pair_kernel(const mplak_ragged_system* __restrict__ systems,
-                                                             const mplak_ragged_item* __restrict__ items) {
+struct PairLds {
+  static constexpr int kVals = RT > 1 ? (RT + 1) / 2 * 2 : 1;
+  typename Quad<T>::type src[kPairTile];              // scaled source coordinates
+  __attribute__((aligned(16))) T sval[kPairTile][kVals];  // source values, column tile
+  T gbox[kPairGroups][2 * DIM];
+  T red[kBlock / kWave][RT][kWave];
+  uint32_t wkeep[kBlock / kWave];
+  double exp_tab[Exp2Lds<T>::size];
+};
+
+template <typename T, int RT, int DIM>
+__device__ __forceinline__ void pair_item(const mplak_ragged_item& it, const mplak_ragged_system& S, void* lds_raw) {
   typedef typename Quad<T>::type Q;
-  const mplak_ragged_item it = items[blockIdx.x];
-  const mplak_ragged_system S = systems[it.sys];
-  // a launch specialised for DIM reads DIM coordinates: other systems are not its items
-  if ((S.skip != nullptr && *S.skip != 0) || S.dim != DIM) return;
-  __shared__ Q src[kPairTile];       // scaled source coordinates
-  __shared__ T sval[kPairTile][RT];  // source values, column tile
-  __shared__ T gbox[kPairGroups][2 * DIM];
-  __shared__ T red[kBlock / kWave][RT][kWave];
-  __shared__ uint32_t wkeep[kBlock / kWave];
-  __shared__ double exp_tab[Exp2Lds<T>::size];
+  auto& lds = *static_cast<PairLds<T, RT, DIM>*>(lds_raw);
+  auto& src = lds.src;
+  auto& sval = lds.sval;
+  auto& gbox = lds.gbox;
+  auto& red = lds.red;
+  auto& wkeep = lds.wkeep;
+  auto& exp_tab = lds.exp_tab;
   if (sizeof(T) == 8) fill_exp2_table(exp_tab);  // first read after the staging barrier
 
   const int64_t n = S.n, R = S.nrhs;
   const int64_t p = it.tile;
   int64_t I, J;
   decode_pair(p, I, J);
+  const int split = pair_split(S), part = it.slab;
+  const int g0 = part * (kPairGroups / split), g1 = g0 + kPairGroups / split;
   const int64_t r0 = (int64_t)it.ctile * RT;
   const int tid = threadIdx.x, lane = tid & (kWave - 1), w = tid / kWave;
   const double scale = S.scale;
@@ -282,7 +329,8 @@ __global__ __launch_bounds__(kBlock) void ragged_pair_kernel(const mplak_ragged_
   }
   __syncthreads();
   // groups this wave keeps (bit g); a pair nobody keeps writes only its flag
-  uint32_t keep = (1u << kPairGroups) - 1u;
+  const uint32_t mine = (1u << g1) - (1u << g0);
+  uint32_t keep = mine;
   if (screen) {
     keep = 0u;
 #pragma unroll
@@ -295,18 +343,19 @@ __global__ __launch_bounds__(kBlock) void ragged_pair_kernel(const mplak_ragged_
       }
       if (__builtin_amdgcn_readfirstlane((int)(d2 > (T)S.drop_s)) == 0) keep |= 1u << g;
     }
+    keep &= mine;
     if (lane == 0) wkeep[w] = keep;
     __syncthreads();
     const uint32_t any = wkeep[0] | wkeep[1] | wkeep[2] | wkeep[3];
     if (any == 0u) {
-      if (tid == 0) pair_flags<T>(S)[p] = 0;
+      if (tid == 0) pair_flags<T>(S)[p * split + part] = 0;
       return;
     }
   }
-  if (tid == 0) pair_flags<T>(S)[p] = 1;
+  if (tid == 0) pair_flags<T>(S)[p * split + part] = 1;
 
   T* part_i = pair_rows<T>(S);
-  T* part_j = part_i + pair_count(S.tiles) * R * kPairTile;
+  T* part_j = part_i + split * pair_count(S.tiles) * R * kPairTile;
   // the compute loop specialised per kernel function (the kind is uniform
   // over the workgroup: no per-entry branch)
   auto run = [&](auto kind_c) {
@@ -339,7 +388,7 @@ __global__ __launch_bounds__(kBlock) void ragged_pair_kernel(const mplak_ragged_
 
     if (I == J) {
 #pragma unroll 1
-      for (int g = 0; g < kPairGroups; ++g) {
+      for (int g = g0; g < g1; ++g) {
         if (((keep >> g) & 1u) == 0u) continue;
 #pragma unroll 2
         for (int s = 0; s < kWave; ++s) {
@@ -356,7 +405,7 @@ __global__ __launch_bounds__(kBlock) void ragged_pair_kernel(const mplak_ragged_
       }
     } else {
 #pragma unroll 1
-      for (int g = 0; g < kPairGroups; ++g) {
+      for (int g = g0; g < g1; ++g) {
         T t[RT];
 #pragma unroll
         for (int q = 0; q < RT; ++q) t[q] = T(0);
@@ -393,7 +442,8 @@ __global__ __launch_bounds__(kBlock) void ragged_pair_kernel(const mplak_ragged_
     for (int h = 0; h < 2; ++h)
 #pragma unroll
       for (int q = 0; q < RT; ++q)
-        if (r0 + q < R) part_i[(p * R + r0 + q) * kPairTile + w * 2 * kWave + h * kWave + lane] = acc[h][q];
+        if (r0 + q < R)
+          part_i[((p * split + part) * R + r0 + q) * kPairTile + w * 2 * kWave + h * kWave + lane] = acc[h][q];
   };
   if (S.kind == MPLAK_KERNEL_GAUSSIAN)
     run(std::integral_constant<int, MPLAK_KERNEL_GAUSSIAN>{});
@@ -401,55 +451,136 @@ __global__ __launch_bounds__(kBlock) void ragged_pair_kernel(const mplak_ragged_
     run(std::integral_constant<int, MPLAK_KERNEL_MATERN32>{});
 }
 
+template <typename T, int RT, int DIM>
+__global__ __launch_bounds__(kBlock) void ragged_pair_kernel(const mplak_ragged_system* __restrict__ systems,
+                                                             const mplak_ragged_item* __restrict__ items) {
+  const mplak_ragged_item it = items[blockIdx.x];
+  const mplak_ragged_system S = systems[it.sys];
+  // a launch specialised for DIM reads DIM coordinates: other systems are not its items
+  if ((S.skip != nullptr && *S.skip != 0) || S.dim != DIM) return;
+  __shared__ PairLds<T, RT, DIM> lds;
+  pair_item<T, RT, DIM>(it, S, &lds);
+}
+
+// Items of every scheme, dimension (<= 4) and column tile in one launch, for
+// systems planned by mplak_ragged_plan_mixed: a column tile is min(nrhs, 8)
+// wide, and work that a launch per class would queue behind the largest system
+// runs beside it.  Bound by the vector unit (FP32 entries and, per right-hand
+// side, four FMAs and a rotation for each pair of entries).
 template <typename T>
-__device__ __forceinline__ double pair_finish_row(const mplak_ragged_system& S, int64_t i, int64_t r) {
-  const int64_t X = i / kPairTile, t = i % kPairTile, R = S.nrhs;
-  const T* part_i = pair_rows<T>(S);
-  const T* part_j = part_i + pair_count(S.tiles) * R * kPairTile;
-  const int32_t* flags = pair_flags<T>(S);
-  // the partial of pair (X, P), or 0 for a pair whose flag says it wrote
-  // nothing (its block is then never used, whatever the memory holds)
-  auto term = [&](int64_t P) -> double {
-    const int64_t p = X <= P ? sym_pair_index(X, P) : sym_pair_index(P, X);
-    const T v = (X <= P ? part_i : part_j)[(p * R + r) * kPairTile + t];
-    return flags[p] != 0 ? (double)v : 0.0;
+__global__ __launch_bounds__(kBlock) void ragged_mixed_kernel(const mplak_ragged_system* __restrict__ systems,
+                                                              const mplak_ragged_item* __restrict__ items) {
+  const mplak_ragged_item it = items[blockIdx.x];
+  const mplak_ragged_system S = systems[it.sys];
+  if (S.skip != nullptr && *S.skip != 0) return;
+  constexpr size_t kLds = std::max(sizeof(PairLds<T, 8, 4>), sizeof(SlabLds<T, 8, kMaxRaggedDim>));
+  __shared__ __attribute__((aligned(16))) char lds[kLds];
+  auto columns = [&](auto rt_c) {
+    constexpr int RT = decltype(rt_c)::value;
+    if (S.scheme == MPLAK_RAGGED_SLABS) {
+      slab_item<T, RT, 0>(it, S, lds);
+      return;
+    }
+    switch (S.dim) {
+      case 1: pair_item<T, RT, 1>(it, S, lds); break;
+      case 2: pair_item<T, RT, 2>(it, S, lds); break;
+      case 3: pair_item<T, RT, 3>(it, S, lds); break;
+      default: pair_item<T, RT, 4>(it, S, lds); break;
+    }
   };
-  // loads batched ahead of the additions, which stay in tile order; the
-  // last batch adds +0.0 past the last tile, which leaves a sum that started
-  // at +0.0 unchanged, so the bits are those of adding tile by tile
-  constexpr int kBatch = 8;
+  switch (S.rt) {
+    case 1: columns(std::integral_constant<int, 1>{}); break;
+    case 2: columns(std::integral_constant<int, 2>{}); break;
+    case 3: columns(std::integral_constant<int, 3>{}); break;
+    case 4: columns(std::integral_constant<int, 4>{}); break;
+    case 5: columns(std::integral_constant<int, 5>{}); break;
+    case 6: columns(std::integral_constant<int, 6>{}); break;
+    case 7: columns(std::integral_constant<int, 7>{}); break;
+    default: columns(std::integral_constant<int, 8>{}); break;
+  }
+}
+
+// The finish: 64 entries of Y per workgroup, each wave a slice of their terms
+// (every fourth), the slices added in order.  Bound by the latency of the
+// partials, which other dies' caches have just written: with one thread per
+// entry walking all of its 40 or so terms a twelve-request batch took 27 us,
+// with four slices and kFinishLoads terms of each in flight 11 us.
+constexpr int kFinishLoads = 8;
+constexpr int kFinishSlices = kBlock / kWave;
+
+// Slice k of the partials of row i, right-hand side r: the pairs (X, P) of the
+// row's tile X over P = 0 .. tiles - 1, from P = X on one term per part.  A
+// partial counts only if its flag says that it was written (it is then never
+// used, whatever the memory holds).  A batch past the end adds +0.0, which
+// leaves a sum that started at +0.0 unchanged.
+template <typename T>
+__device__ __forceinline__ double pair_finish_row(const mplak_ragged_system& S, int64_t i, int64_t r, int k) {
+  // pair indices and parts fit 32 bits (use_pairs, plan_split); the split is a
+  // power of two, so there is no division in the loop
+  const uint32_t X = (uint32_t)(i / kPairTile), t = (uint32_t)(i % kPairTile), tiles = (uint32_t)S.tiles;
+  const uint32_t split = (uint32_t)pair_split(S), shift = (uint32_t)__builtin_ctz(split);
+  const int64_t stride = S.nrhs * (int64_t)kPairTile;  // of a pair's rows
+  const T* part_i = pair_rows<T>(S) + r * kPairTile + t;
+  const T* part_j = part_i + split * pair_count(S.tiles) * stride;
+  const int32_t* flags = pair_flags<T>(S);
+  auto pair = [](uint32_t I, uint32_t J) { return J * (J + 1) / 2 + I; };
+  const uint32_t own = (t / kWave) >> (3 - shift);  // the part of t's group, in pairs whose tile J is X
+  const uint32_t terms = X + ((tiles - X) << shift);
   double s = 0.0;
-  for (int64_t P = 0; P < S.tiles; P += kBatch) {
-    double v[kBatch];
+  for (uint32_t m0 = k; m0 < terms; m0 += kFinishLoads * kFinishSlices) {
+    double v[kFinishLoads];
 #pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-      const int64_t Q = P + u < S.tiles ? P + u : S.tiles - 1;
-      const double t = term(Q);
-      v[u] = P + u < S.tiles ? t : 0.0;
+    for (uint32_t u = 0; u < kFinishLoads; ++u) {
+      const uint32_t m = m0 + u * kFinishSlices < terms ? m0 + u * kFinishSlices : m0;
+      const uint32_t q = m - X;  // only used for m >= X
+      const uint32_t p = m < X ? pair(m, X) : pair(X, X + (q >> shift));
+      const uint32_t f = (p << shift) + (m < X ? own : (q & (split - 1)));
+      const T w = *(m < X ? part_j + p * stride : part_i + f * stride);
+      v[u] = m0 + u * kFinishSlices < terms && flags[f] != 0 ? (double)w : 0.0;
     }
 #pragma unroll
-    for (int u = 0; u < kBatch; ++u) s += v[u];
+    for (uint32_t u = 0; u < kFinishLoads; ++u) s += v[u];
   }
   return s;
 }
 
-// items: (system, block) over n * nrhs entries of Y, 256 per block
+// items: (system, block) over n * nrhs entries of Y, 256 per item in four
+// workgroups
 __global__ __launch_bounds__(kBlock) void ragged_finish_kernel(const mplak_ragged_system* __restrict__ systems,
                                                                const mplak_ragged_item* __restrict__ items) {
-  const mplak_ragged_item it = items[blockIdx.x];
+  __shared__ double red[kFinishSlices][kWave];
+  const mplak_ragged_item it = items[blockIdx.x / (kBlock / kWave)];
   const mplak_ragged_system S = systems[it.sys];
   if (S.skip != nullptr && *S.skip != 0) return;
-  const int64_t g = (int64_t)it.tile * kBlock + threadIdx.x;
+  const int lane = threadIdx.x % kWave, k = threadIdx.x / kWave;
+  const int64_t g = (int64_t)it.tile * kBlock + (blockIdx.x % (kBlock / kWave)) * kWave + lane;
   const int64_t n = S.n, R = S.nrhs;
-  if (g >= n * R) return;
-  const int64_t i = g % n, r = g / n;
-  double s;
-  if (S.scheme == MPLAK_RAGGED_PAIRS) {
-    s = S.precision == MPLAK_PREC_F64 ? pair_finish_row<double>(S, i, r) : pair_finish_row<float>(S, i, r);
-  } else {
-    s = S.part[r * n + i];
-    for (int64_t k = 1; k < S.slabs; ++k) s += S.part[(k * R + r) * n + i];
+  const bool active = g < n * R;
+  const bool narrow = n * R <= 0xffffffffll;
+  const int64_t r = narrow ? (int64_t)((uint32_t)g / (uint32_t)n) : g / n, i = g - r * n;
+  double s = 0.0;
+  if (active) {
+    if (S.scheme == MPLAK_RAGGED_PAIRS) {
+      s = S.precision == MPLAK_PREC_F64 ? pair_finish_row<double>(S, i, r, k) : pair_finish_row<float>(S, i, r, k);
+    } else {
+      const double* p = S.part + r * n + i;
+      for (int64_t m0 = k; m0 < S.slabs; m0 += kFinishLoads * kFinishSlices) {
+        double v[kFinishLoads];
+#pragma unroll
+        for (int u = 0; u < kFinishLoads; ++u) {
+          const int64_t m = m0 + u * kFinishSlices;
+          v[u] = m < S.slabs ? p[m * R * n] : 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < kFinishLoads; ++u) s += v[u];
+      }
+    }
   }
+  red[k][lane] = s;
+  __syncthreads();
+  if (k != 0 || !active) return;
+#pragma unroll
+  for (int q = 1; q < kFinishSlices; ++q) s += red[q][lane];
   if (S.nugget != 0.0) s = fma(S.nugget, S.V[r * n + i], s);
   S.Y[r * n + i] = s;
 }
@@ -671,16 +802,62 @@ void launch_pairs(int rt, int dim, const mplak_ragged_system* sys, const mplak_r
   }
 }
 
-// PAIRS for n >= kRagPairMinN unless MPLAK_RAGGED_PAIRS says otherwise
-// (0: never, 1: every n); the pair index must fit an item's 32-bit field.
-bool use_pairs(int64_t n) {
+// PAIRS for n >= least unless MPLAK_RAGGED_PAIRS says otherwise (0: never, 1:
+// every n); the pair index must fit an item's 32-bit field.
+bool use_pairs(int64_t n, int64_t least) {
   const char* v = getenv("MPLAK_RAGGED_PAIRS");
-  bool on = n >= kRagPairMinN;
+  bool on = n >= least;
   if (v != nullptr && *v != '\0') on = atoi(v) != 0;
   const int64_t tiles = (n + kPairTile - 1) / kPairTile;
   return on && pair_count(tiles) <= 0x7fffffff;
 }
 
+static_assert(kPairGroups == 8, "pair_finish_row: parts of 8 groups");
+
+// Work split of a system whose column tiles are `rt` wide: tile pairs from
+// `pairs_from` points on, shared by `parts` workgroups each, and slabs of at
+// least `unit` sources otherwise.
+size_t plan_split(mplak_ragged_system* s, int rt, int64_t pairs_from, int64_t unit, int parts) {
+  if (s == nullptr || s->n <= 0 || s->nrhs <= 0 || s->dim < 1 || s->dim > kMaxRaggedDim) return 0;
+  s->rt = rt;
+  s->ctiles = (s->nrhs + s->rt - 1) / s->rt;
+  s->tiles = (int32_t)((s->n + kBlock - 1) / kBlock);
+  int64_t ks = (kRagTargetBlocks + (int64_t)s->tiles * s->ctiles - 1) / ((int64_t)s->tiles * s->ctiles);
+  const int64_t units = (s->n + unit - 1) / unit;
+  if (ks > units) ks = units;
+  if (ks < 1) ks = 1;
+  const int64_t per = (units + ks - 1) / ks;
+  s->slab_cols = per * unit;
+  s->slabs = (int32_t)((s->n + s->slab_cols - 1) / s->slab_cols);
+  s->scale = coord_scale(s->kind, s->length_scale);
+  s->drop_s = s->drop_log2 > 0.0 ? drop_distance2(s->kind, s->drop_log2) : 0.0;
+  s->reserved = 0;
+  if (use_pairs(s->n, pairs_from)) {
+    s->scheme = MPLAK_RAGGED_PAIRS;
+    s->tiles = (int32_t)((s->n + kPairTile - 1) / kPairTile);
+    s->slabs = 0;
+    s->slab_cols = 0;
+    const size_t es = s->precision == MPLAK_PREC_F64 ? sizeof(double) : sizeof(float);
+    const size_t pairs = (size_t)pair_count(s->tiles);
+    s->reserved = parts;
+    return align_up((size_t)(parts + 1) * pairs * (size_t)s->nrhs * kPairTile * es, 256) +
+           align_up((size_t)parts * pairs * sizeof(int32_t), 256);
+  }
+  s->scheme = MPLAK_RAGGED_SLABS;
+  return (size_t)s->slabs * (size_t)s->nrhs * (size_t)s->n * sizeof(double);
+}
+
+// Workgroups per tile pair in a mixed launch, from n alone: the largest power of
+// two up to 8 that keeps pairs times workgroups below 1200.  One workgroup a
+// pair leaves a 13455-point system's 378 pairs on 256 CUs, two on some and one
+// on the others; each further part is another row set for the finish to read
+// (twelve requests of up to 24576 points: 60.1 ms at 1200, 61.8 ms at 600).
+int mixed_parts(int64_t n) {
+  const int64_t pairs = pair_count((n + kPairTile - 1) / kPairTile);
+  int k = 1;
+  while (k < kPairGroups && pairs * (2 * k) < 1200) k *= 2;
+  return k;
+}
 
 }  // namespace
 }  // namespace mplak
@@ -690,43 +867,28 @@ using namespace mplak;
 extern "C" {
 
 size_t mplak_ragged_plan(mplak_ragged_system* s) {
-  if (s == nullptr || s->n <= 0 || s->nrhs <= 0 || s->dim < 1 || s->dim > kMaxRaggedDim) return 0;
-  s->rt = rt_class(s->nrhs);
-  s->ctiles = (s->nrhs + s->rt - 1) / s->rt;
-  s->tiles = (int32_t)((s->n + kBlock - 1) / kBlock);
-  int64_t ks = (kRagTargetBlocks + (int64_t)s->tiles * s->ctiles - 1) / ((int64_t)s->tiles * s->ctiles);
-  const int64_t chunks = (s->n + kChunk - 1) / kChunk;
-  if (ks > chunks) ks = chunks;
-  if (ks < 1) ks = 1;
-  const int64_t per = (chunks + ks - 1) / ks;
-  s->slab_cols = per * kChunk;
-  s->slabs = (int32_t)((s->n + s->slab_cols - 1) / s->slab_cols);
-  s->scale = coord_scale(s->kind, s->length_scale);
-  s->drop_s = s->drop_log2 > 0.0 ? drop_distance2(s->kind, s->drop_log2) : 0.0;
-  s->reserved = 0;
-  if (use_pairs(s->n)) {
-    s->scheme = MPLAK_RAGGED_PAIRS;
-    s->tiles = (int32_t)((s->n + kPairTile - 1) / kPairTile);
-    s->slabs = 0;
-    s->slab_cols = 0;
-    const size_t es = s->precision == MPLAK_PREC_F64 ? sizeof(double) : sizeof(float);
-    const size_t pairs = (size_t)pair_count(s->tiles);
-    return align_up(2 * pairs * (size_t)s->nrhs * kPairTile * es, 256) + align_up(pairs * sizeof(int32_t), 256);
-  }
-  s->scheme = MPLAK_RAGGED_SLABS;
-  return (size_t)s->slabs * (size_t)s->nrhs * (size_t)s->n * sizeof(double);
+  return plan_split(s, s != nullptr ? rt_class(s->nrhs) : 1, kRagPairMinN, kChunk, 1);
+}
+
+size_t mplak_ragged_plan_mixed(mplak_ragged_system* s) {
+  if (s == nullptr || s->nrhs <= 0 || s->n <= 0) return 0;
+  // FP64 systems are launched by class, whose column tiles are powers of two
+  const int rt = s->precision == MPLAK_PREC_F64 ? rt_class(s->nrhs) : (s->nrhs < 8 ? s->nrhs : 8);
+  return plan_split(s, rt, kMixedPairMinN, kWave, mixed_parts(s->n));
 }
 
 int64_t mplak_ragged_product_items(const mplak_ragged_system* s, mplak_ragged_item* out, int32_t sys_index) {
   if (s == nullptr || s->tiles <= 0) return 0;
   if (s->scheme == MPLAK_RAGGED_PAIRS) {
     const int64_t pairs = pair_count(s->tiles);
+    const int split = pair_split(*s);
     if (out) {
       int64_t k = 0;
       for (int32_t c = 0; c < s->ctiles; ++c)
-        for (int64_t q = 0; q < pairs; ++q) out[k++] = mplak_ragged_item{sys_index, (int32_t)q, 0, c};
+        for (int64_t q = 0; q < pairs; ++q)
+          for (int32_t u = 0; u < split; ++u) out[k++] = mplak_ragged_item{sys_index, (int32_t)q, u, c};
     }
-    return pairs * s->ctiles;
+    return pairs * split * s->ctiles;
   }
   const int64_t count = (int64_t)s->tiles * s->slabs * s->ctiles;
   if (out) {
@@ -766,11 +928,21 @@ int mplak_ragged_product(const mplak_ragged_system* systems, const mplak_ragged_
   return launch_status();
 }
 
+int mplak_ragged_product_mixed(const mplak_ragged_system* systems, const mplak_ragged_item* items, int64_t count,
+                               mplak_stream_t s) {
+  if (count <= 0) return MPLAK_OK;
+  if (!systems || !items || count > 0x7fffffff) return MPLAK_ERR_ARG;
+  hipLaunchKernelGGL(ragged_mixed_kernel<float>, dim3((unsigned)count), dim3(kBlock), 0, as_stream(s), systems, items);
+  return launch_status();
+}
+
 int mplak_ragged_finish(const mplak_ragged_system* systems, const mplak_ragged_item* items, int64_t count,
                         mplak_stream_t s) {
   if (count <= 0) return MPLAK_OK;
   if (!systems || !items) return MPLAK_ERR_ARG;
-  hipLaunchKernelGGL(ragged_finish_kernel, dim3((unsigned)count), dim3(kBlock), 0, as_stream(s), systems, items);
+  if (count > 0x7fffffff / (kBlock / kWave)) return MPLAK_ERR_ARG;
+  hipLaunchKernelGGL(ragged_finish_kernel, dim3((unsigned)(count * (kBlock / kWave))), dim3(kBlock), 0, as_stream(s),
+                     systems, items);
   return launch_status();
 }
 

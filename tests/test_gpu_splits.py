@@ -247,3 +247,61 @@ def test_hmatrix_near_pairs_and_far_items(lib, am, bm, terms, cols, kind, dim):
             t, m = V[:, cs] @ x[3:][cs], np.abs(V[:, cs]) @ np.abs(x[3:][cs])
             assert np.all(np.abs(far[i, :terms] - t) <= (cols + 8) * EPS * m)
             assert np.all(far[i, terms:] == 7.0)
+
+
+# Mixed launches of the served products: pairs from 2048 points on in 8, 4, 2 or 1
+# parts, slabs below, every column tile width, every dimension, screened or not;
+# each system alone and in the mix gives the same bits.
+MIXED = [(1, 2, 0, 1), (63, 3, 1, 3), (700, 1, 0, 2), (2047, 4, 1, 7), (2048, 2, 1, 5), (3000, 3, 0, 8), (5000, 1, 1, 4),
+         (9000, 3, 1, 6), (12000, 4, 0, 1), (13000, 2, 0, 3), (18000, 2, 1, 2), (900, 3, 0, 10)]
+
+
+@pytest.mark.parametrize("drop", [0.0, 30.0])
+def test_ragged_mixed_launch(lib, drop):
+    import ctypes as C
+
+    import torch
+    systems, keep = [], []
+    for n, dim, kind, nrhs in MIXED:
+        g = torch.Generator(device="cuda").manual_seed(n)
+        P = torch.rand((dim, n), generator=g, dtype=torch.float64, device="cuda")
+        P = P[:, torch.argsort(P[0])].contiguous()  # some blocks are far apart
+        V = torch.randn((nrhs, n), generator=g, dtype=torch.float64, device="cuda")
+        Y = torch.full_like(V, 7.0)
+        ell = (0.05, 0.1)[kind]
+        s = _native.mplak_ragged_system()
+        s.points, s.V, s.Y, s.n, s.dim, s.kind, s.nrhs = P.data_ptr(), V.data_ptr(), Y.data_ptr(), n, dim, kind, nrhs
+        s.precision, s.length_scale, s.nugget, s.drop_log2 = _native.MPLAK_PREC_F32, ell, 0.75, drop
+        part = torch.full((lib.mplak_ragged_plan_mixed(C.byref(s)),), 255, dtype=torch.uint8, device="cuda")  # NaN bits
+        s.part = part.data_ptr()
+        systems.append(s)
+        keep.append((P, V, Y, part, ell))
+
+    def run(members):
+        recs = (_native.mplak_ragged_system * len(members))(*[systems[k] for k in members])
+        tables = []
+        for items_of in (lib.mplak_ragged_product_items, lib.mplak_ragged_finish_items):
+            items = []
+            for j, k in enumerate(members):
+                arr = (_native.mplak_ragged_item * items_of(C.byref(systems[k]), None, j))()
+                items_of(C.byref(systems[k]), arr, j)
+                items += list(arr)
+            tables.append((_native.mplak_ragged_item * len(items))(*items))
+        dev_of = lambda a: torch.frombuffer(bytearray(bytes(a)), dtype=torch.uint8).to("cuda")  # noqa: E731
+        sd, pd, fd = dev_of(recs), dev_of(tables[0]), dev_of(tables[1])
+        ck(lib.mplak_ragged_product_mixed(sd.data_ptr(), pd.data_ptr(), len(tables[0]), stream()))
+        ck(lib.mplak_ragged_finish(sd.data_ptr(), fd.data_ptr(), len(tables[1]), stream()))
+        return [host(keep[k][2]).copy() for k in members]
+
+    together = run(range(len(MIXED)))
+    for k, (n, dim, kind, nrhs) in enumerate(MIXED):
+        P, V, _, _, ell = keep[k]
+        ref, mag = torch.empty_like(V), torch.empty_like(V)
+        for i in range(0, n, 4096):
+            s = sum((P[d, i:i + 4096, None] - P[d][None, :]) ** 2 for d in range(dim))
+            r = (3.0 * s).sqrt() / ell
+            K = (-0.5 * s / ell ** 2).exp() if kind == 0 else (1.0 + r) * (-r).exp()
+            ref[:, i:i + 4096], mag[:, i:i + 4096] = V @ K.t(), V.abs() @ K.t()
+        bar = 2e-5 * host(mag + 0.75 * V.abs()) + (n * 2.0 ** -drop * host(V.abs().amax()) if drop else 0.0)
+        assert np.all(np.abs(together[k] - host(ref + 0.75 * V)) <= bar), MIXED[k]
+        assert np.array_equal(run([k])[0], together[k]), MIXED[k]
