@@ -15,6 +15,7 @@
 #include <float.h>
 #include <math.h>
 
+#include "cg_step.hpp"
 #include "common.hpp"
 
 namespace mplak {
@@ -31,10 +32,6 @@ inline int vec_blocks(int64_t n) {
   if (b < 1) b = 1;
   if (b > kVecMaxBlocks) b = kVecMaxBlocks;
   return static_cast<int>(b);
-}
-
-__device__ __forceinline__ double stop_value(int rule, double rr, double bnorm2, double n_global) {
-  return rule == MPLAK_STOP_RMS ? sqrt(rr / n_global) : sqrt(rr) / sqrt(bnorm2);
 }
 
 __global__ __launch_bounds__(kBlock) void cg_start_kernel(int64_t n, const double* __restrict__ b,
@@ -74,7 +71,7 @@ __global__ __launch_bounds__(kBlock) void cg_start_final_kernel(const double* __
     s.bnorm2 = bb;
     s.eps = eps;
     s.n_global = n_global;
-    s.rel = stop_value(rule, rr, bb, n_global);
+    s.rel = cg_stop_value(rule, rr, bb, n_global);
     s.alpha = 0.0;
     s.beta = 0.0;
     s.k = 0;
@@ -146,7 +143,7 @@ __global__ __launch_bounds__(kBlock) void cg_direct_kernel(int64_t n, const doub
   const double alpha = s_in.rr / dz;
   const double beta = rr_new / s_in.rr;
   const int k = s_in.k + 1;
-  const double rel = stop_value(s_in.rule, rr_new, s_in.bnorm2, s_in.n_global);
+  const double rel = cg_stop_value(s_in.rule, rr_new, s_in.bnorm2, s_in.n_global);
   const bool conv = rel < s_in.eps;
   const bool limit = k >= s_in.iter_max - 1;
   // The reference breaks before the direction update only on convergence;
@@ -166,6 +163,30 @@ __global__ __launch_bounds__(kBlock) void cg_direct_kernel(int64_t n, const doub
     s.done = conv ? MPLAK_CONVERGED : (limit ? MPLAK_ITER_LIMIT : MPLAK_RUNNING);
     *out = s;
   }
+}
+
+// The iteration of up to kCgStepMax elements in one launch, one workgroup per
+// column.
+template <int E>
+__global__ __launch_bounds__(kCgStepThreads) void cg_step_kernel(int64_t n, double* __restrict__ x,
+                                                                 double* __restrict__ r, double* __restrict__ d,
+                                                                 const double* __restrict__ z,
+                                                                 const mplak_cg_state* __restrict__ in,
+                                                                 mplak_cg_state* __restrict__ out) {
+  __shared__ double scratch[kCgStepThreads / kWave];
+  const int64_t off = (int64_t)blockIdx.x * n;
+  cg_step<E>(n, x + off, r + off, d + off, z + off, in + blockIdx.x, out + blockIdx.x, scratch);
+}
+
+void launch_cg_step(int64_t n, int64_t columns, double* x, double* r, double* d, const double* z,
+                    const mplak_cg_state* in, mplak_cg_state* out, hipStream_t s) {
+  const dim3 grid((unsigned)columns), block(kCgStepThreads);
+  if (n <= 2 * kCgStepThreads)
+    hipLaunchKernelGGL(cg_step_kernel<2>, grid, block, 0, s, n, x, r, d, z, in, out);
+  else if (n <= 4 * kCgStepThreads)
+    hipLaunchKernelGGL(cg_step_kernel<4>, grid, block, 0, s, n, x, r, d, z, in, out);
+  else
+    hipLaunchKernelGGL(cg_step_kernel<6>, grid, block, 0, s, n, x, r, d, z, in, out);
 }
 
 // Single-reduction CG (Chronopoulos & Gear, J. Comput. Appl. Math. 25, 1989;
@@ -210,7 +231,7 @@ __global__ __launch_bounds__(kBlock) void cg1_update_kernel(int64_t n, double* _
   }
   double gam, del;
   reduce_partials2<kBlock>(dots, dots + nd, nd, scratch, gam, del);
-  const double rel = stop_value(s_in.rule, gam, s_in.bnorm2, s_in.n_global);
+  const double rel = cg_stop_value(s_in.rule, gam, s_in.bnorm2, s_in.n_global);
   const bool conv = rel < s_in.eps;
   const double beta = first ? 0.0 : gam / s_in.rr;
   const double alpha = first ? gam / del : gam / (del - beta * gam / s_in.alpha);
@@ -558,7 +579,7 @@ __global__ __launch_bounds__(kBlock) void bcg_start_final_kernel(const double* _
     s.bnorm2 = bb;
     s.eps = eps;
     s.n_global = n_global;
-    s.rel = stop_value(rule, rr, bb, n_global);
+    s.rel = cg_stop_value(rule, rr, bb, n_global);
     s.alpha = s.beta = 0.0;
     s.k = 0;
     s.iter_max = iter_max;
@@ -637,7 +658,7 @@ __global__ __launch_bounds__(kBlock) void bcg_direct_kernel(int64_t n, const dou
   const double rr_new = reduce_partials<kBlock>(part + (nrhs + c) * G, G, scratch);
   const double beta = rr_new / s_in.rr;
   const int k = s_in.k + 1;
-  const double rel = stop_value(s_in.rule, rr_new, s_in.bnorm2, s_in.n_global);
+  const double rel = cg_stop_value(s_in.rule, rr_new, s_in.bnorm2, s_in.n_global);
   const bool conv = rel < s_in.eps;
   const bool limit = k >= s_in.iter_max - 1;
   if (!conv) {
@@ -718,6 +739,10 @@ int mplak_cg_iterate(int64_t n, double* x, double* r, double* d, const double* z
   const int g = vec_blocks(n);
   double* part = static_cast<double*>(work);
   hipStream_t hs = as_stream(s);
+  if (n <= kCgStepMax) {
+    launch_cg_step(n, 1, x, r, d, z, in, out, hs);
+    return launch_status();
+  }
   hipLaunchKernelGGL(cg_dz_kernel, dim3(g), dim3(kBlock), 0, hs, n, d, z, in, part);
   int st = launch_status();
   if (st != MPLAK_OK) return st;
@@ -898,13 +923,18 @@ int mplak_bcg_iterate(int64_t n, int64_t nrhs, double* X, double* R, double* D, 
   if (work == nullptr || work_bytes < mplak_bcg_workspace_bytes(n, nrhs)) return MPLAK_ERR_WORKSPACE;
   double* part = static_cast<double*>(work);
   hipStream_t hs = as_stream(s);
-  hipLaunchKernelGGL(bcg_dz_kernel, grid, dim3(kBlock), 0, hs, n, D, Z, in, part);
-  int st = launch_status();
-  if (st != MPLAK_OK) return st;
-  hipLaunchKernelGGL(bcg_update_kernel, grid, dim3(kBlock), 0, hs, n, X, R, D, Z, in, nrhs, part);
-  st = launch_status();
-  if (st != MPLAK_OK) return st;
-  hipLaunchKernelGGL(bcg_direct_kernel, grid, dim3(kBlock), 0, hs, n, R, D, in, out, nrhs, part);
+  int st;
+  if (n <= kCgStepMax) {
+    launch_cg_step(n, nrhs, X, R, D, Z, in, out, hs);
+  } else {
+    hipLaunchKernelGGL(bcg_dz_kernel, grid, dim3(kBlock), 0, hs, n, D, Z, in, part);
+    st = launch_status();
+    if (st != MPLAK_OK) return st;
+    hipLaunchKernelGGL(bcg_update_kernel, grid, dim3(kBlock), 0, hs, n, X, R, D, Z, in, nrhs, part);
+    st = launch_status();
+    if (st != MPLAK_OK) return st;
+    hipLaunchKernelGGL(bcg_direct_kernel, grid, dim3(kBlock), 0, hs, n, R, D, in, out, nrhs, part);
+  }
   st = launch_status();
   if (st != MPLAK_OK) return st;
   hipLaunchKernelGGL(bcg_group_kernel, dim3(1), dim3(kBlock), 0, hs, out, (int)nrhs, group);

@@ -305,3 +305,61 @@ def test_ragged_mixed_launch(lib, drop):
         bar = 2e-5 * host(mag + 0.75 * V.abs()) + (n * 2.0 ** -drop * host(V.abs().amax()) if drop else 0.0)
         assert np.all(np.abs(together[k] - host(ref + 0.75 * V)) <= bar), MIXED[k]
         assert np.array_equal(run([k])[0], together[k]), MIXED[k]
+
+
+# One launch per CG iteration up to 6144 elements (2, 4 and 6 per thread of one
+# workgroup), three beyond: one iteration of a running column, of one that
+# converges in it (its direction is kept), of one that stops at its limit and of
+# one that had stopped before (nothing moves).
+@pytest.mark.parametrize("n", [1, 63, 1024, 2047, 2048, 2049, 4096, 4097, 6143, 6144, 6145])
+@pytest.mark.parametrize("block", [False, True])
+def test_cg_iteration_in_one_launch(lib, n, block):
+    import ctypes as C
+    rng = np.random.default_rng(n)
+    cols = 4
+    x, r, d, z = (rng.uniform(0.5, 1.5, (cols, n)) for _ in range(4))
+    states = (_native.mplak_cg_state * cols)()
+    for c, s in enumerate(states):
+        s.rr, s.bnorm2, s.n_global, s.eps = float(r[c] @ r[c]), 2.0 * n, n, 1e-30
+        s.rule, s.k, s.iter_max, s.done = c & 1, 3, 1000, 0
+    states[1].eps, states[2].iter_max, states[3].done = 1e30, 5, 2
+    ss = C.sizeof(_native.mplak_cg_state)
+    X, R, D, Z = dev(x), dev(r), dev(d), dev(z)
+    sin = dev(np.frombuffer(bytes(states), dtype=np.float64).copy())
+    sout = dev(np.zeros(cols * ss // 8))
+    if block:
+        group = dev(np.zeros(8))
+        wb = lib.mplak_bcg_workspace_bytes(n, cols)
+        w = workspace(wb)
+        ck(lib.mplak_bcg_iterate(n, cols, X.data_ptr(), R.data_ptr(), D.data_ptr(), Z.data_ptr(), sin.data_ptr(),
+                                 sout.data_ptr(), group.data_ptr(), w.data_ptr(), wb, stream()))
+    else:
+        wb = lib.mplak_cg_workspace_bytes(n)
+        w = workspace(wb)
+        for c in range(cols):
+            o = 8 * n * c
+            ck(lib.mplak_cg_iterate(n, X.data_ptr() + o, R.data_ptr() + o, D.data_ptr() + o, Z.data_ptr() + o,
+                                    sin.data_ptr() + ss * c, sout.data_ptr() + ss * c, w.data_ptr(), wb, stream()))
+    out = (_native.mplak_cg_state * cols).from_buffer_copy(host(sout).tobytes())
+    gx, gr, gd = host(X), host(R), host(D)
+    u = (n + 8) * EPS  # any order of n products, then the few operations on the sums
+    for c, s in enumerate(states):
+        if c == 3:
+            assert bytes(out[c]) == bytes(s)
+            assert np.array_equal(gx[c], x[c]) and np.array_equal(gr[c], r[c]) and np.array_equal(gd[c], d[c])
+            continue
+        alpha = s.rr / float(d[c] @ z[c])
+        assert abs(out[c].alpha / alpha - 1) <= 2 * u
+        rv = r[c] - out[c].alpha * z[c]
+        xv = x[c] + out[c].alpha * d[c]
+        bound = EPS * 2 * (np.abs(r[c]) + np.abs(out[c].alpha * z[c]))
+        assert np.all(np.abs(gr[c] - rv) <= bound)
+        assert np.all(np.abs(gx[c] - xv) <= EPS * 2 * (np.abs(x[c]) + np.abs(out[c].alpha * d[c])))
+        rr = float(gr[c] @ gr[c])
+        assert abs(out[c].rr - rr) <= 2 * u * rr
+        rel = np.sqrt(out[c].rr / n) if s.rule == _native.MPLAK_STOP_RMS else np.sqrt(out[c].rr) / np.sqrt(s.bnorm2)
+        assert abs(out[c].rel - rel) <= 8 * EPS * rel and out[c].k == 4
+        assert out[c].done == (1 if c == 1 else 2 if c == 2 else 0)
+        beta = 0.0 if c == 1 else out[c].rr / s.rr
+        dv = d[c] if c == 1 else gr[c] + beta * d[c]
+        assert np.all(np.abs(gd[c] - dv) <= 4 * EPS * (np.abs(gr[c]) + np.abs(beta * d[c])) * (c != 1))
