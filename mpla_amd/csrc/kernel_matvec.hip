@@ -314,6 +314,18 @@ struct PairPart {
         groups(SPLIT ? ((1u << ((kSymTile / kWave) / s)) - 1u) << (sub * ((kSymTile / kWave) / s)) : 0xffu) {}
 };
 
+// decode_pair of a pair that a plan lists (a 32-bit index, the same for the whole
+// workgroup): the root in FP32, whose result is off by less than 1 (J < 92682),
+// then whole numbers on the scalar unit.
+__device__ __forceinline__ void decode_listed_pair(uint32_t p, int64_t& I, int64_t& J) {
+  const float root = (__builtin_amdgcn_sqrtf(8.0f * (float)p + 1.0f) - 1.0f) * 0.5f;
+  uint64_t j = (uint32_t)__builtin_amdgcn_readfirstlane((int)root);
+  while (j * (j + 1) / 2 > p) --j;
+  while ((j + 1) * (j + 2) / 2 <= p) ++j;
+  I = (int64_t)(p - j * (j + 1) / 2);
+  J = (int64_t)j;
+}
+
 enum SymMode { kSymExact = 0, kSymScreened = 1, kSymPlanned = 2 };
 
 // One tile pair (I, J) of the symmetric product on the vector unit.
@@ -553,13 +565,17 @@ __global__ __launch_bounds__(kBlock) void kmv_sym_kernel(
 // Planned FP32 product (plan built for FP32, no coincidence shift): one
 // workgroup per listed tile pair, heaviest first.
 //
-// Compact target tile: matrix-core form.  In coordinates centred on the
-// target tile, s = |p - q|^2 = n_p + n_q - 2 p.q (n = squared norm), and
+// Compact target tile: 16 x 16 tiles.  In coordinates centred on the
+// target tile, s = |p - q|^2 = n_p + n_q - 2 p.q (n = squared norm).  In 3-D
 // v_mfma_f32_16x16x4f32 with A = [p, n_p] (16 targets), B = [-2 q, 1] (16
-// sources) and C = n_q (one value per lane) gives s for a 16 x 16 tile in
+// sources) and C = n_q (one value per lane) gives s for such a tile in
 // the accumulator layout: lane 16 r + c holds targets 4 r + v (v < 4)
 // against source c.  The vector unit is left with the exponential and the
-// two accumulations.  The tile-centred norms are small (half-diagonal^2 <=
+// two accumulations.  In 1-D and 2-D the vector unit forms s in the same layout:
+// an FP32 matrix instruction holds the SIMD's vector unit up for its 32 cycles
+// (a loop of it and of this arithmetic took the sum of both, 115 cycles per
+// tile for 43 + 64), and 2 or 3 operations per entry are fewer; the next target
+// slab's operands are read a slab ahead.  The tile-centred norms are small (half-diagonal^2 <=
 // kCenterRadius2), so the cancellation error stays at the level of the FP32
 // coordinates themselves.  Both tiles are staged in LDS in operand layout.
 // Wave w takes the target slabs 4 a + w (a < 8; interleaved, which balances
@@ -644,15 +660,17 @@ __device__ __forceinline__ float rows4_reduce_scatter(const float (&v)[4], int r
 // of the targets (lane 16 k + c: coordinate k of target 16 slab + c for
 // k < 3, at k = 3 its norm (Matern) or 1 (Gaussian)) and of the sources
 // (-2 x coordinate k; at k = 3: 1 (Matern) or the source norm (Gaussian)),
-// then source norms (Matern), source values, target values (Gaussian: times
-// 2^-n_p) and, Gaussian, the target row scales 2^-n_p.
+// then source norms (Matern) or the target row scales 2^-n_p (Gaussian),
+// source values, target values (Gaussian: times 2^-n_p) and the column sums of
+// the four waves.
 constexpr int kMfOp = kSlabs * kWave;
 constexpr int kMfB = kMfOp;
 constexpr int kMfNorm = 2 * kMfOp;
 constexpr int kMfXs = kMfNorm + kSymTile;
 constexpr int kMfXt = kMfXs + kSymTile;
-constexpr int kMfScale = kMfXt + kSymTile;
-constexpr int kMfFloats = kMfScale + kSymTile;
+constexpr int kMfScale = kMfNorm;  // one or the other
+constexpr int kMfCol = kMfXt + kSymTile;
+constexpr int kMfFloats = kMfCol + (kBlock / kWave) * kSymTile;
 
 // Gaussian entries factor as 2^-s = 2^-n_p 2^-t with t = n_q - 2 p.q, so the
 // matrix cores give t with no C operand (A = [p, 1], B = [-2 q, n_q]); the
@@ -661,7 +679,7 @@ constexpr int kMfFloats = kMfScale + kSymTile;
 // 2^-t stays in range.  Matern entries are not a product of that form and
 // take s = t + n_p with C = n_q.
 template <int KIND, int DIM, typename P>
-__device__ __forceinline__ void sym_mfma_pair(const double* const* __restrict__ points, int64_t off, int64_t n,
+__device__ __forceinline__ void sym_mfma_pair(const double* const (&coord)[3], int64_t n,
                                               double scale, const double* __restrict__ x, P* __restrict__ rows_i,
                                               P* __restrict__ rows_j, int64_t p, int64_t I, int64_t J,
                                               float4 centre, const uint32_t* __restrict__ tmask, uint32_t groups,
@@ -684,7 +702,7 @@ __device__ __forceinline__ void sym_mfma_pair(const double* const* __restrict__ 
       const int64_t j = (side == 0 ? J : I) * kSymTile + tid + it * kBlock;
       const int64_t jc = j < n ? j : n - 1;
 #pragma unroll
-      for (int d = 0; d < DIM; ++d) pc[side][it][d] = global_load(points[d] + off + jc);
+      for (int d = 0; d < DIM; ++d) pc[side][it][d] = global_load(coord[d] + jc);
       pv[side][it] = global_load(x + jc);
     }
   }
@@ -728,13 +746,15 @@ __device__ __forceinline__ void sym_mfma_pair(const double* const* __restrict__ 
     gmask[g] = (groups >> g) & 1u ? (uint32_t)__builtin_amdgcn_readfirstlane((int)tm[g]) : 0u;
   __syncthreads();
 
+  constexpr bool DOT = DIM < 3;  // s on the vector unit (pt, xt: one 16-byte read per lane row)
   float A[8], accR[8][4];
 #pragma unroll
   for (int a = 0; a < 8; ++a) {
-    A[a] = mf[(4 * a + w) * kWave + lane];
+    if (!DOT) A[a] = mf[(4 * a + w) * kWave + lane];
 #pragma unroll
     for (int v = 0; v < 4; ++v) accR[a][v] = 0.0f;
   }
+  const float* pt = &mf[w * kWave + 4 * r4];  // pt[256 a + 16 d + v]: coordinate d (3: the norm) of that target
   const float* xt = &mf[kMfXt + 16 * w + 4 * r4];  // xt[64 a + v]: target 16 (4 a + w) + 4 r + v
   // One 64-source group: target slabs a (outer) against the group's four
   // source slabs b; the kept MFMAs of slab a are issued before their results
@@ -742,39 +762,66 @@ __device__ __forceinline__ void sym_mfma_pair(const double* const* __restrict__ 
   // order whatever the mask.
   auto mfma_group = [&](int g, uint32_t gm, auto diagonal) -> float {
     constexpr bool DIAG = decltype(diagonal)::value;
-    float bv[4], xn[4];
+    float bv[4], xn[4], q[4][DIM], nq[4];
     f32x4 cq[4];
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
-      bv[b] = mf[kMfB + (g * 4 + b) * kWave + lane];
       xn[b] = mf[kMfXs + g * kWave + 16 * b + c16];
-      cq[b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-      if (!FACTOR) {
-        const float nq = mf[kMfNorm + g * kWave + 16 * b + c16];
-        cq[b] = f32x4{nq, nq, nq, nq};
+      const float* op = &mf[kMfB + (g * 4 + b) * kWave];
+      if (DOT || !FACTOR) nq[b] = FACTOR ? op[48 + c16] : mf[kMfNorm + g * kWave + 16 * b + c16];
+      if constexpr (DOT) {
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) q[b][d] = op[16 * d + c16];
+      } else {
+        bv[b] = op[lane];
+        cq[b] = FACTOR ? f32x4{0.0f, 0.0f, 0.0f, 0.0f} : f32x4{nq[b], nq[b], nq[b], nq[b]};
       }
     }
     float accC[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    f32x4 next[DIM + 1], nextx;
+    auto fetch = [&](int a) {
+#pragma unroll
+      for (int d = 0; d < DIM + (FACTOR ? 0 : 1); ++d)
+        next[d] = *reinterpret_cast<const f32x4*>(&pt[256 * a + (d < DIM ? 16 * d : 48)]);
+      nextx = *reinterpret_cast<const f32x4*>(&xt[64 * a]);
+    };
+    if (DOT) fetch(0);
 #pragma unroll
     for (int a = 0; a < 8; ++a) {
+      f32x4 pc[DIM + 1], xm;
+      if (DOT) {
+#pragma unroll
+        for (int d = 0; d < DIM + (FACTOR ? 0 : 1); ++d) pc[d] = next[d];
+        xm = nextx;
+        if (a < 7) fetch(a + 1);
+      }
       // bit b: tile (a, b) kept (bit 8 b + a of gm)
       const uint32_t cm = ((gm >> a) & 1u) | ((gm >> (7 + a)) & 2u) | ((gm >> (14 + a)) & 4u) | ((gm >> (21 + a)) & 8u);
       if (cm == 0) continue;
-      const f32x4 xm = *reinterpret_cast<const f32x4*>(&xt[64 * a]);
+      if (!DOT) xm = *reinterpret_cast<const f32x4*>(&xt[64 * a]);
       // diagonal pair: the tile of target slab 4 a + w against source slab
       // 4 g + b is on the diagonal for a = g, b = w (rows only); the plan
       // keeps no tile below it
       const int dtile = DIAG && a == g ? w : -1;
       f32x4 s[4];
+      if constexpr (!DOT) {
 #pragma unroll
-      for (int b = 0; b < 4; ++b)
-        if ((cm >> b) & 1u) s[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(A[a], bv[b], cq[b], 0, 0, 0);
+        for (int b = 0; b < 4; ++b)
+          if ((cm >> b) & 1u) s[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(A[a], bv[b], cq[b], 0, 0, 0);
+      }
 #pragma unroll
       for (int b = 0; b < 4; ++b) {
         if (((cm >> b) & 1u) == 0) continue;
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-          float sv = s[b][v];
+          float sv;
+          if constexpr (DOT) {
+            sv = FACTOR ? nq[b] : pc[DIM][v] + nq[b];
+#pragma unroll
+            for (int d = 0; d < DIM; ++d) sv = fmaf(pc[d][v], q[b][d], sv);
+          } else {
+            sv = s[b][v];
+          }
           if (KIND == MPLAK_KERNEL_MATERN32) sv = fmaxf(sv, 0.0f);  // sqrt of a rounding-negative s
           const float e = kernel_entry<float, KIND>(sv, nullptr);
           accR[a][v] = fmaf(e, xn[b], accR[a][v]);
@@ -785,9 +832,7 @@ __device__ __forceinline__ void sym_mfma_pair(const double* const* __restrict__ 
     // lane 16 r + c keeps the sum of source 16 r + c of the group
     return rows4_reduce_scatter(accC, r4);
   };
-  float tg[kSymGroups];
-#pragma unroll
-  for (int g = 0; g < kSymGroups; ++g) tg[g] = 0.0f;
+  float* col = &mf[kMfCol + w * kSymTile + lane];
   // group g's mask: the uniform select over gmask keeps it in scalar registers
   auto group_mask = [&](int g) -> uint32_t {
     uint32_t m = 0;
@@ -800,21 +845,13 @@ __device__ __forceinline__ void sym_mfma_pair(const double* const* __restrict__ 
 #pragma unroll 1
     for (int g = 0; g < kSymGroups; ++g) {
       const uint32_t gm = group_mask(g);
-      if (gm == 0) continue;
-      const float v = mfma_group(g, gm, std::true_type{});
-#pragma unroll
-      for (int q = 0; q < kSymGroups; ++q)
-        if (q == g) tg[q] = v;
+      col[g * kWave] = gm != 0 ? mfma_group(g, gm, std::true_type{}) : 0.0f;
     }
   } else {
 #pragma unroll 1
     for (int g = 0; g < kSymGroups; ++g) {
       const uint32_t gm = group_mask(g);
-      if (gm == 0) continue;
-      const float v = mfma_group(g, gm, std::false_type{});
-#pragma unroll
-      for (int q = 0; q < kSymGroups; ++q)
-        if (q == g) tg[q] = v;
+      col[g * kWave] = gm != 0 ? mfma_group(g, gm, std::false_type{}) : 0.0f;
     }
   }
   // row sums: lane 16 r + c writes rows q = c and q = c + 16 of its lane
@@ -829,16 +866,13 @@ __device__ __forceinline__ void sym_mfma_pair(const double* const* __restrict__ 
   if (I == J) {
     // the column sums of the upper tiles belong to the same rows: the four
     // waves' sums in wave order (FP64), then added to each row's sum
-    __syncthreads();  // every wave is done reading the staged tiles
-#pragma unroll
-    for (int g = 0; g < kSymGroups; ++g) mf[w * kSymTile + g * kWave + lane] = tg[g];
-    __syncthreads();
-    static_assert((kBlock / kWave) * kSymTile + 2 * kSymTile <= kMfScale, "column sums clear of the row scales");
-    double* cs = reinterpret_cast<double*>(mf + (kBlock / kWave) * kSymTile);
+    __syncthreads();  // every wave is done reading the staged operands
+    static_assert(2 * kSymTile <= kMfNorm, "the sums clear of the row scales");
+    double* cs = reinterpret_cast<double*>(mf);
     for (int k = tid; k < kSymTile; k += kBlock) {
-      double sum = (double)mf[k];
+      double sum = (double)mf[kMfCol + k];
 #pragma unroll
-      for (int q = 1; q < kBlock / kWave; ++q) sum += (double)mf[q * kSymTile + k];
+      for (int q = 1; q < kBlock / kWave; ++q) sum += (double)mf[kMfCol + q * kSymTile + k];
       cs[k] = sum;
     }
     __syncthreads();
@@ -857,14 +891,11 @@ __device__ __forceinline__ void sym_mfma_pair(const double* const* __restrict__ 
     rows_i[k] = (P)v;
   }
   if (I != J) {
-    __syncthreads();  // every wave is done reading the staged tiles
-#pragma unroll
-    for (int g = 0; g < kSymGroups; ++g) mf[w * kSymTile + g * kWave + lane] = tg[g];
     __syncthreads();
     for (int k = tid; k < kSymTile; k += kBlock) {
-      double s = (double)mf[k];
+      double s = (double)mf[kMfCol + k];
 #pragma unroll
-      for (int q = 1; q < kBlock / kWave; ++q) s += (double)mf[q * kSymTile + k];
+      for (int q = 1; q < kBlock / kWave; ++q) s += (double)mf[kMfCol + q * kSymTile + k];
       rows_j[k] = (P)s;
     }
   }
@@ -914,31 +945,53 @@ __device__ __forceinline__ int plan_level(const PlanLevels& lv) {
   return l;
 }
 
+// Bound by the vector unit (Matern: busy 92 % of the time in 3-D) and, with the
+// few tiles per pair of a Gaussian, by staging, reductions and latency (63 %).
+// Matern takes 5 waves per SIMD at the price of a few spilled registers outside
+// the loop; 4 leave 5 % more time.  The column sums have LDS rows of their own:
+// held in registers until the tiles are read they cost 8 of them.  Time per
+// product, n = 65536 at drop levels 15 / 10 / 6, before and now: Gaussian 3-D
+// 58.5 / 46.4 / 37.5 and 56.9 / 45.2 / 36.4 us, 2-D 71 / 56 / 44 and 64 / 51 /
+// 40 us; Matern 3-D 520 / 327 / 169 and 495 / 309 / 160 us, 2-D 564 / 387 / 222
+// and 490 / 337 / 195 us.  The vector form in 3-D: Gaussian 60 / 48 / 38 us,
+// Matern 540 / 338 / 174 us.
 template <int KIND, int DIM, bool SPLIT>
-__global__ __launch_bounds__(kBlock) void kmv_sym_planned_kernel(
+__global__ __launch_bounds__(kBlock, KIND == MPLAK_KERNEL_MATERN32 ? 5 : 1) void kmv_sym_planned_kernel(
     const double* const* __restrict__ points, int64_t off, int64_t n, double scale, const double* __restrict__ x,
     float* __restrict__ part, const PlanLevels lv, const int32_t* __restrict__ skip) {
-  if (skip != nullptr && *skip != 0) return;
-  const int lev = plan_level(lv);
+  // Every load that does not wait for another one first: the flag, the
+  // selector, each level's count and list entry and the coordinate pointers (an
+  // entry past the count is not used).
   const PairPart<SPLIT> part_of(lv.split);
-  if (part_of.item >= *level_pick(lv.count, lev)) return;
-  const uint32_t* __restrict__ list = level_pick(lv.list, lev);
+  const int32_t skipped = skip != nullptr ? *skip : 0;
+  int64_t counts[kMaxLevels];
+  uint32_t pairs[kMaxLevels];
+#pragma unroll
+  for (int l = 0; l < kMaxLevels; ++l) {
+    counts[l] = *lv.count[l];
+    pairs[l] = lv.list[l][part_of.item];
+  }
+  const double* coord[3];
+#pragma unroll
+  for (int d = 0; d < DIM; ++d) coord[d] = points[d] + off;
+  const int lev = plan_level(lv);
+  if (skipped != 0 || part_of.item >= level_pick(counts, lev)) return;
+  const uint32_t p = level_pick(pairs, lev);
   const float4* __restrict__ tinfo = level_pick(lv.tinfo, lev);
   const uint32_t* __restrict__ bmask = level_pick(lv.bmask, lev);
   const uint32_t* __restrict__ tmask = level_pick(lv.tmask, lev);
   __shared__ __attribute__((aligned(16))) float mf[kMfFloats];
-  static_assert((kBlock / kWave) * kSymTile <= kMfFloats, "column sums reuse the staging buffer");
   static_assert(sizeof(SymSrc<float>) * kSymGroups <= sizeof(mf), "vector-unit staging fits");
   const int32_t* __restrict__ slots = level_pick(lv.slots, lev);
-  const int64_t p = (int64_t)list[part_of.item];
   int64_t I, J;
-  decode_pair(p, I, J);
+  decode_listed_pair(p, I, J);
   const int64_t pcap = lv.pcap * part_of.split;
-  float* rows_i = slot_row(part, I, J, slots[2 * p] * part_of.split + part_of.sub, pcap);
-  float* rows_j = I != J ? slot_row(part, J, I, slots[2 * p + 1] * part_of.split + part_of.sub, pcap) : rows_i;
+  float* rows_i = slot_row(part, I, J, slots[2 * (size_t)p] * part_of.split + part_of.sub, pcap);
+  float* rows_j =
+      I != J ? slot_row(part, J, I, slots[2 * (size_t)p + 1] * part_of.split + part_of.sub, pcap) : rows_i;
   const float4 centre = tinfo[I];
   if (centre.w != 0.0f) {
-    sym_mfma_pair<KIND, DIM, float>(points, off, n, scale, x, rows_i, rows_j, p, I, J, centre, tmask, part_of.groups, mf);
+    sym_mfma_pair<KIND, DIM, float>(coord, n, scale, x, rows_i, rows_j, p, I, J, centre, tmask, part_of.groups, mf);
   } else {
     sym_valu_pair<float, KIND, DIM, false, true, true, false, float>(
         points, off, n, scale, 0.0, 0.0, 0.0, x, rows_i, rows_j, p, bmask[p], part_of.groups,
@@ -1330,17 +1383,18 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 4))) 
     double* __restrict__ part, const uint32_t* __restrict__ list, const int64_t* __restrict__ count,
     const uint32_t* __restrict__ tmask, const float4* __restrict__ tinfo, const int32_t* __restrict__ slots,
     int64_t pair_pcap, int split, const int32_t* __restrict__ skip) {
-  if (skip != nullptr && *skip != 0) return;
   const PairPart<SPLIT> part_of(split);
-  if (part_of.item >= *count) return;
+  const int32_t skipped = skip != nullptr ? *skip : 0;
+  const uint32_t p = list[part_of.item];  // not used past the count
+  if (skipped != 0 || part_of.item >= *count) return;
   constexpr int kBufDoubles = kM64Doubles > kT64Doubles ? kM64Doubles : kT64Doubles;
   __shared__ __attribute__((aligned(16))) double buf[kBufDoubles];
-  const int64_t p = (int64_t)list[part_of.item];
   int64_t I, J;
-  decode_pair(p, I, J);
+  decode_listed_pair(p, I, J);
   const int64_t pcap = pair_pcap * part_of.split;
-  double* rows_i = slot_row(part, I, J, slots[2 * p] * part_of.split + part_of.sub, pcap);
-  double* rows_j = I != J ? slot_row(part, J, I, slots[2 * p + 1] * part_of.split + part_of.sub, pcap) : rows_i;
+  double* rows_i = slot_row(part, I, J, slots[2 * (size_t)p] * part_of.split + part_of.sub, pcap);
+  double* rows_j =
+      I != J ? slot_row(part, J, I, slots[2 * (size_t)p + 1] * part_of.split + part_of.sub, pcap) : rows_i;
   // FP64 plans mark compact tiles 2, the others 1 (both take the tile screen)
   const float4 centre = tinfo[I];
   if (KIND == MPLAK_KERNEL_GAUSSIAN && centre.w == 2.0f)
@@ -1693,15 +1747,18 @@ PlanLayout plan_layout(int64_t n) {
   return L;
 }
 
-// Level l of `lv` from the plan at `base`.
+// Level l of `lv` from the plan at `base`; level 0 also stands in for the levels
+// that are not there (the kernels read every level's count, then take one).
 void plan_level_view(const PlanLayout& L, char* base, int l, PlanLevels& lv) {
-  lv.list[l] = reinterpret_cast<const uint32_t*>(base + L.list);
-  lv.count[l] = reinterpret_cast<const int64_t*>(base + L.count);
-  lv.tinfo[l] = reinterpret_cast<const float4*>(base + L.tinfo);
-  lv.bmask[l] = reinterpret_cast<const uint32_t*>(base + L.bmask);
-  lv.tmask[l] = reinterpret_cast<const uint32_t*>(base + L.tmask);
-  lv.pcount[l] = reinterpret_cast<const int32_t*>(base + L.pcount);
-  lv.slots[l] = reinterpret_cast<const int32_t*>(base + L.slots);
+  for (int q = l; q < (l == 0 ? kMaxLevels : l + 1); ++q) {
+    lv.list[q] = reinterpret_cast<const uint32_t*>(base + L.list);
+    lv.count[q] = reinterpret_cast<const int64_t*>(base + L.count);
+    lv.tinfo[q] = reinterpret_cast<const float4*>(base + L.tinfo);
+    lv.bmask[q] = reinterpret_cast<const uint32_t*>(base + L.bmask);
+    lv.tmask[q] = reinterpret_cast<const uint32_t*>(base + L.tmask);
+    lv.pcount[q] = reinterpret_cast<const int32_t*>(base + L.pcount);
+    lv.slots[q] = reinterpret_cast<const int32_t*>(base + L.slots);
+  }
   lv.pcap = L.pcap;
 }
 
