@@ -110,23 +110,31 @@ __global__ __launch_bounds__(kBlock) void dot_final_kernel(const double* __restr
 // matrices had before, ran a 30001 x 20003 product at 2.9 TB/s; 16-byte loads
 // run it at 6.4 TB/s (1663 -> 751 us).
 //
-// Two geometries:
+// Geometries:
 // * streamed (RL = 64, 4 waves): each load instruction reads 1 KiB of one
 //   column; bound by HBM or the Infinity Cache.  A product keeps the memory
 //   system busy from about 152 workgroups, and above 256 (one per CU) a last
 //   round that is nearly empty costs up to a third (n = 16385: 465 us at 258
 //   workgroups, 363 us at 2064), so the slab count is the smallest with 152
-//   to 256 workgroups, or else with at least 90 % of the last round filled.
-// * panels of 16 rows (RL = 8, 16 waves): a matrix of up to 40 MB has too few
-//   128-row panels to fill the chip and is bound by latency; 16-row panels
-//   put 16 waves on each of m / 16 CUs with every load of a wave in flight
-//   at once and mostly need no second kernel (1000 x 1000: 4.9 us against
-//   9.9 us streamed, 1500 x 1500: 7.0 us against 7.4 us; 2500 x 2500: 14.1 us
-//   against 11.7 us, so the line lies between the last two).  Fewer than 256
-//   columns leave its 128 column slots idle (30000 x 64: 12.4 us against
-//   4.3 us streamed).  Matrices of up to 64 rows take it at any size: most
-//   lanes of a 128-row panel would hold no row (64 x 30000: 7.5 us in 32
-//   slabs).
+//   to 256 workgroups, or else with at least 90 % of the last round filled; one
+//   from 4 rounds of panels (200000 x 256: 63 us, in two slabs 67 us).
+// * panels of 16 rows (RL = 8, 16 waves): a matrix of up to 40 MB and 4096
+//   rows has too few 128-row panels to fill the chip and is bound by latency;
+//   16-row panels put 16 waves on each of m / 16 CUs with every load of a wave
+//   in flight at once and mostly need no second kernel (1000 x 1000: 4.9 us
+//   against 9.9 us streamed, 1500 x 1500: 7.0 us against 7.4 us, 226 x 208: 3.6
+//   us against 6.0 us).  Matrices of up to 64 rows take it at any size: most
+//   lanes of a 128-row panel would hold no row (64 x 30000: 7.5 us in 32 slabs).
+// * the panels between (RL = 16 or 32 with 16 waves, RL = 64 with 8), the
+//   lowest that give at most one panel per CU, for matrices that fit the
+//   Infinity Cache: all columns in one workgroup save the slab sum and its
+//   launch (streamed / so: 4096 x 4096 24.4 / 21.5 us, 4200 x 1000 12.7 / 8.4
+//   us, 10000 x 2500 32.5 / 29.8 us, 16384 x 4000 83 / 75 us, 20000 x 1000
+//   23.9 / 23.4 us; 120 MB as 3000 x 5000, on 94 panels, 23.6 / 25.2 us).
+//   Fewer than 128 columns leave too little for their waves and are streamed in
+//   one slab (12000 x 64: 3.5 us, panels 3.9 us, two slabs 6.5 us), and so are
+//   small matrices whose 32-row panels are more than the CUs (8200 x 256: 4.0
+//   us, 64-row panels 4.3 us; 12000 x 256, 25 MB: 5.8 and 5.0 us).
 //
 // A matrix larger than the 256 MiB Infinity Cache is read with nontemporal
 // loads (STREAM): every element is used once, and the hint keeps the stream
@@ -137,11 +145,12 @@ __global__ __launch_bounds__(kBlock) void dot_final_kernel(const double* __restr
 // ---------------------------------------------------------------------------
 
 constexpr int kGvUnroll = 8;                                // columns of a lane in flight
-constexpr int kGvStreamLanes = 64, kGvStreamWaves = 4;      // 128-row panels
-constexpr int kGvPanelLanes = 8, kGvPanelWaves = 16;        // 16-row panels
+constexpr int kGvStreamLanes = 64, kGvPanelLanes = 8;       // 128-row and 16-row panels
 constexpr double kGvPanelBytes = 40e6;                      // largest matrix of the 16-row panels
 constexpr int64_t kGvPanelRows = 64;                        // or most rows at any size
-constexpr int64_t kGvPanelCols = 256;                       // fewest columns
+constexpr int64_t kGvPanelCols = 128;                       // fewest columns of the panels between,
+constexpr int64_t kGvWholeTiles = 120;                      // fewest of those panels
+constexpr double kGvSmallBytes = 22e6;                      // and smallest matrix of more than 8192 rows
 constexpr int64_t kGvCus = 256;
 constexpr int64_t kGvBusy = 152;                            // workgroups that saturate the memory system
 constexpr int64_t kGvStreamBytes = int64_t(256) << 20;      // Infinity Cache capacity
@@ -156,20 +165,35 @@ __device__ __forceinline__ gv_f64x2 gv_load2(const double* p) {
 }
 
 struct GemvPlan {
-  bool panels;  // 16-row panels
+  int lanes, waves;  // RL, NW
   int64_t row_tiles, slabs, slab_cols;
 };
 
 inline GemvPlan gemv_plan(int64_t m, int64_t n) {
   GemvPlan p;
-  p.panels = n >= kGvPanelCols && (m <= kGvPanelRows || (double)m * (double)n * sizeof(double) <= kGvPanelBytes);
-  const int64_t rows = 2 * (p.panels ? kGvPanelLanes : kGvStreamLanes);
-  p.row_tiles = (m + rows - 1) / rows;
+  const double bytes = (double)m * (double)n * sizeof(double);
+  auto tiles = [&](int lanes) { return (m + 2 * lanes - 1) / (2 * lanes); };
+  p.lanes = kGvStreamLanes;
+  p.waves = 4;
+  bool whole = false;  // one slab
+  if (m <= kGvPanelRows || (m <= kGvCus * 2 * kGvPanelLanes && bytes <= kGvPanelBytes)) {
+    p.lanes = kGvPanelLanes;
+  } else if (n < kGvPanelCols || (tiles(2 * kGvPanelLanes) > kGvCus && bytes <= kGvSmallBytes)) {
+    whole = true;
+  } else if (bytes <= kGvStreamBytes) {
+    int lanes = 2 * kGvPanelLanes;
+    while (lanes < kGvStreamLanes && tiles(lanes) > kGvCus) lanes *= 2;
+    whole = tiles(lanes) >= kGvWholeTiles;
+    if (whole) p.lanes = lanes;
+    if (whole && tiles(lanes) <= kGvCus) p.waves = 8;
+  }
+  if (p.lanes < kGvStreamLanes) p.waves = 16;
+  p.row_tiles = tiles(p.lanes);
   int64_t ks = 1;
-  if (p.panels) {
+  if (p.lanes == kGvPanelLanes) {
     // a lane walks n / 128 columns: wide matrices of few rows are split further
     if (n >= 4096) ks = std::min((kGvCus + p.row_tiles - 1) / p.row_tiles, n / 1024);
-  } else {
+  } else if (!whole && p.row_tiles < 4 * kGvCus) {
     const int64_t most = std::min<int64_t>(std::max<int64_t>(n / (8 * kGvUnroll), 1), 4096);
     double best = 0.0;
     for (int64_t k = 1; k <= most; ++k) {
@@ -227,7 +251,8 @@ __global__ __launch_bounds__(NW* kWave) void dgemv_partial_kernel(int64_t m, int
   double acc0 = 0.0, acc1 = 0.0;
   int64_t j = j0 + 2 * g;
   const double* a = A + b + j * lda;
-  for (int64_t jw = j0; jw + U * CG <= j1; jw += U * CG) {
+  int64_t jw = j0;
+  for (; jw + U * CG <= j1; jw += U * CG) {
     gv_f64x2 v[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) v[u] = load(a + col(u) * lda);
@@ -251,7 +276,7 @@ __global__ __launch_bounds__(NW* kWave) void dgemv_partial_kernel(int64_t m, int
     j += U * CG;
     a += (int64_t)(U * CG) * lda;
   }
-  {
+  if (jw < j1) {
     // the last columns of the share, fewer than U CG: an absent column is
     // neither loaded nor multiplied
     gv_f64x2 v[U];
@@ -395,10 +420,16 @@ int mplak_dgemv_f64(int64_t m, int64_t n, const double* A, int64_t lda, const do
   if (work_bytes < need || (need > 0 && work == nullptr)) return MPLAK_ERR_WORKSPACE;
   double* out = p.slabs > 1 ? static_cast<double*>(work) : y;
   const bool stream = (double)m * (double)n * sizeof(double) > (double)kGvStreamBytes;
-  if (p.panels)
-    launch_gemv<kGvPanelLanes, kGvPanelWaves>(p, stream, m, n, A, lda, x, out, skip_if, as_stream(s));
+  if (p.lanes == 8)
+    launch_gemv<8, 16>(p, stream, m, n, A, lda, x, out, skip_if, as_stream(s));
+  else if (p.lanes == 16)
+    launch_gemv<16, 16>(p, stream, m, n, A, lda, x, out, skip_if, as_stream(s));
+  else if (p.lanes == 32)
+    launch_gemv<32, 16>(p, stream, m, n, A, lda, x, out, skip_if, as_stream(s));
+  else if (p.waves == 8)
+    launch_gemv<64, 8>(p, stream, m, n, A, lda, x, out, skip_if, as_stream(s));
   else
-    launch_gemv<kGvStreamLanes, kGvStreamWaves>(p, stream, m, n, A, lda, x, out, skip_if, as_stream(s));
+    launch_gemv<64, 4>(p, stream, m, n, A, lda, x, out, skip_if, as_stream(s));
   int st = launch_status();
   if (st != MPLAK_OK || p.slabs == 1) return st;
   hipLaunchKernelGGL(slab_sum_kernel, dim3(elementwise_grid(m)), dim3(kBlock), 0, as_stream(s), m,

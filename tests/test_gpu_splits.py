@@ -21,13 +21,17 @@ def ck(status):
     _native.check(status)
 
 
-# 16-row panels (m n up to 40 MB or m up to 64, n from 256) with their column
+# 16-row panels (m n up to 40 MB and m up to 4096, or m up to 64) with their column
 # remainders and slabs (n from 4096); 128-row panels otherwise, one slab and
-# several; rows that end inside a panel; odd strides and an 8-byte aligned base.
+# several; 32-, 64- and 128-row panels of all columns between (from 128 columns;
+# above 8192 rows from 22 MB); rows that end inside a panel; odd strides and an
+# 8-byte aligned base.
 @pytest.mark.parametrize("m,n,lda,shift", [
     (1, 255, 3, 0), (1, 4097, 1, 1), (2, 256, 2, 1), (15, 257, 15, 0), (16, 383, 17, 1), (17, 1030, 17, 0),
     (33, 9001, 35, 1), (64, 4096, 64, 0), (65, 255, 65, 1), (127, 100, 129, 0), (129, 63, 129, 1), (1001, 777, 1001, 1),
-    (2200, 2300, 2201, 0), (2301, 2302, 2301, 1), (257, 20011, 257, 0)])
+    (2200, 2300, 2201, 0), (2301, 2302, 2301, 1), (257, 20011, 257, 0),
+    (226, 208, 226, 0), (4096, 1300, 4097, 1), (4097, 127, 4097, 0), (4097, 128, 4097, 1), (8191, 700, 8193, 0),
+    (8193, 300, 8193, 0), (8193, 401, 8193, 1), (16384, 169, 16384, 0), (16385, 337, 16387, 1), (32769, 130, 32769, 0)])
 def test_dgemv_panels_slabs_and_strides(lib, m, n, lda, shift):
     rng = np.random.default_rng(m * 7 + n)
     A = rng.uniform(-1, 1, shift + lda * n)
