@@ -128,7 +128,7 @@ __global__ __launch_bounds__(kBlock) void dot_final_kernel(const double* __restr
 // * the panels between (RL = 16 or 32 with 16 waves, RL = 64 with 8), the
 //   lowest that give at most one panel per CU, for matrices that fit the
 //   Infinity Cache: all columns in one workgroup save the slab sum and its
-//   launch (streamed / so: 4096 x 4096 24.4 / 21.5 us, 4200 x 1000 12.7 / 8.4
+//   launch (streamed / so: 4096 x 4000 24.4 / 21.5 us, 4200 x 1000 12.7 / 8.4
 //   us, 10000 x 2500 32.5 / 29.8 us, 16384 x 4000 83 / 75 us, 20000 x 1000
 //   23.9 / 23.4 us; 120 MB as 3000 x 5000, on 94 panels, 23.6 / 25.2 us).
 //   Fewer than 128 columns leave too little for their waves and are streamed in

@@ -38,7 +38,7 @@ namespace {
 
 constexpr int kChunk = 256;          // sources per LDS chunk
 constexpr int kMaxDim = 16;
-constexpr int kTargetBlocks = 2048;
+constexpr int kValuUnit = 32;  // sources a slab of the vector kernel is a multiple of
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -50,22 +50,8 @@ struct Slabs {
   int64_t tiles, slabs, slab_cols;
 };
 
-inline Slabs slab_plan(int64_t rows, int64_t cols, int tile_rows, int64_t col_tiles) {
-  Slabs p;
-  p.tiles = (rows + tile_rows - 1) / tile_rows;
-  int64_t ks = (kTargetBlocks + p.tiles * col_tiles - 1) / (p.tiles * col_tiles);
-  const int64_t chunks = (cols + kChunk - 1) / kChunk;
-  if (ks > chunks) ks = chunks;
-  if (ks < 1) ks = 1;
-  if (ks > 65535) ks = 65535;
-  const int64_t per = (chunks + ks - 1) / ks;
-  p.slab_cols = per * kChunk;
-  p.slabs = (cols + p.slab_cols - 1) / p.slab_cols;
-  return p;
-}
-
-// Split of the sources for a matrix-core kernel with `occ` workgroups resident
-// per CU: the slab count (of whole chunks of 64 sources) that minimises, in
+// Split of the sources for a kernel with `occ` workgroups resident
+// per CU: the slab count (of whole chunks of sources) that minimises, in
 // units of one workgroup's chunk on a full CU, the chunks of the busiest CU
 // plus the slabs' partials, written and read back once each.  A CU with fewer
 // than `occ` workgroups takes a chunk down to a quarter of that time.  Measured:
@@ -73,18 +59,19 @@ inline Slabs slab_plan(int64_t rows, int64_t cols, int tile_rows, int64_t col_ti
 // 27 us, 16 slabs 25 us), against 8 us for a 64-column BF16x3 chunk and 18 us for an
 // FP64 one (n = 20001, 64 columns in FP64: 1.44 ms in 8 slabs, five workgroups
 // on the busiest CU; 1.66 ms in 4, three).
-inline Slabs balanced_slabs(int64_t rows, int64_t cols, int tile_rows, int chunk, int occ, int64_t R) {
+inline Slabs balanced_slabs(int64_t rows, int64_t cols, int tile_rows, int chunk, int occ, int64_t R,
+                            int64_t col_tiles = 1, double slab_weight = 1.0) {
   constexpr int64_t kCus = 256;
   Slabs p;
   p.tiles = (rows + tile_rows - 1) / tile_rows;
   const int64_t chunks = (cols + chunk - 1) / chunk;
-  const int64_t most = std::min<int64_t>(chunks, std::max<int64_t>(4 * kCus * occ / p.tiles, 1));
-  const double slab_cost = 0.02 + 2.4e-7 * (double)rows * (double)R;
+  const int64_t most = std::min<int64_t>(chunks, std::max<int64_t>(4 * kCus * occ / (p.tiles * col_tiles), 1));
+  const double slab_cost = slab_weight * (0.02 + 2.4e-7 * (double)rows * (double)R);
   double best = 0.0;
   for (int64_t ks = 1; ks <= most; ++ks) {
     const int64_t per = (chunks + ks - 1) / ks;
     const int64_t slabs = (chunks + per - 1) / per;
-    const double m = (double)((p.tiles * slabs + kCus - 1) / kCus) / occ;  // of the busiest CU, in full CUs
+    const double m = (double)((p.tiles * col_tiles * slabs + kCus - 1) / kCus) / occ;  // of the busiest CU, in full CUs
     const double cost = (double)per * (m >= 1.0 ? m : 0.25 + 0.75 * m) + slab_cost * (double)slabs;
     if (ks == 1 || cost < best) {
       best = cost;
@@ -97,7 +84,11 @@ inline Slabs balanced_slabs(int64_t rows, int64_t cols, int tile_rows, int chunk
 
 // ---------------------------------------------------------------------------
 // VALU kernel.  grid = (target tiles of 256, slabs, column tiles of RT).
-// part layout: part[(slab * R + r) * rows + i].
+// part layout: part[(slab * R + r) * rows + i].  Bound by the vector unit, and
+// while slabs were whole 256-source chunks by a few waves of long serial loops;
+// slabs are now multiples of 32 sources, as many as the balance below gives (2-D
+// Matern in FP64, 5 columns: n = 1797 38 -> 15 us, n = 6000 86 -> 54 us, n =
+// 12000 242 -> 181 us; 3-D Gaussian in FP32: 22 -> 13, 46 -> 31, 115 -> 100 us).
 
 template <typename T, int KIND, int DIM, int RT>
 __global__ __launch_bounds__(kBlock) void mrhs_valu_kernel(
@@ -135,8 +126,9 @@ __global__ __launch_bounds__(kBlock) void mrhs_valu_kernel(
     T cacc[RT];
 #pragma unroll
     for (int q = 0; q < RT; ++q) cacc[q] = T(0);
+    const int jn = (int)(c1 - cb < kChunk ? c1 - cb : kChunk);
 #pragma unroll 2
-    for (int jj = 0; jj < kChunk; ++jj) {
+    for (int jj = 0; jj < jn; ++jj) {
       T s = T(0);
 #pragma unroll
       for (int d = 0; d < MD; ++d)
@@ -612,7 +604,10 @@ inline MrhsPlan make_plan(const mplak_kernel_desc* d, int precision, int64_t R) 
   } else {
     p.rt = valu_rt(R);
     const int64_t ctiles = (R + p.rt - 1) / p.rt;
-    p.s = slab_plan(d->row_count, d->col_count, kBlock, ctiles);
+    // a 32-source unit of the double form takes about the chunk's 8 us; a third of
+    // that in FP32, three times as long past 3 dimensions (the runtime-dim loop)
+    const double weight = d->dim > 3 ? 0.3 : (precision == MPLAK_PREC_F64 ? 1.0 : 3.0);
+    p.s = balanced_slabs(d->row_count, d->col_count, kBlock, kValuUnit, 4, R, ctiles, weight);
     p.vpk_bytes = 0;
   }
   p.part_bytes = align_up((size_t)p.s.slabs * (size_t)R * (size_t)d->row_count * (p.mfma ? sizeof(float) : sizeof(double)),

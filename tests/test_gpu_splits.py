@@ -95,10 +95,12 @@ def test_planned_product_pair_splits(lib, n, kind, dim, ordered):
 # FP64 multi-right-hand-side products on the matrix cores (from 9 columns):
 # rows around the 16-row blocks and 128-row tiles, columns around the 16- and
 # 64-column blocks, sources around the 64-point chunks, blocks off the diagonal,
-# padded leading dimensions; 8 columns and 5 dimensions take the vector unit.
+# padded leading dimensions; up to 8 columns, and 5 dimensions, take the vector
+# unit, in slabs of 32 sources and more.
 @pytest.mark.parametrize("rows,cols,row_off,R,dim", [
     (1, 1, 0, 9, 1), (15, 63, 3, 16, 2), (17, 65, 0, 17, 3), (127, 64, 0, 33, 4), (128, 130, 5, 48, 3),
-    (129, 129, 0, 64, 2), (1000, 517, 100, 65, 3), (700, 1500, 0, 73, 2), (300, 300, 0, 8, 3), (300, 300, 0, 20, 5)])
+    (129, 129, 0, 64, 2), (1000, 517, 100, 65, 3), (700, 1500, 0, 73, 2), (300, 300, 0, 8, 3), (300, 300, 0, 20, 5),
+    (1, 1, 0, 1, 1), (33, 31, 2, 2, 2), (257, 33, 0, 3, 3), (255, 257, 1, 5, 2), (600, 289, 0, 8, 4), (300, 1000, 5, 24, 5)])
 @pytest.mark.parametrize("kind", [0, 1])
 def test_mrhs_f64_tiles(lib, rows, cols, row_off, R, dim, kind):
     import ctypes as C
