@@ -59,8 +59,16 @@ struct Slabs {
 // 27 us, 16 slabs 25 us), against 8 us for a 64-column BF16x3 chunk and 18 us for an
 // FP64 one (n = 20001, 64 columns in FP64: 1.44 ms in 8 slabs, five workgroups
 // on the busiest CU; 1.66 ms in 4, three).
+// `drain`: share of a long workgroup's chunks (those past kDrainChunks) that the
+// chip is partly idle at the end of a product.  Workgroups that start together
+// end 10 % apart and more, so that one even round of long ones loses to several
+// rounds of shorter ones (BF16, n = 131072, 64 columns: 6.41 ms in 2 slabs, 5.70
+// ms in 8); short ones lose less than their slabs cost (n = 12000: 2 % per
+// iteration with the share taken of every chunk).
+constexpr double kMfmaDrain = 0.12;
+constexpr int64_t kDrainChunks = 64;
 inline Slabs balanced_slabs(int64_t rows, int64_t cols, int tile_rows, int chunk, int occ, int64_t R,
-                            int64_t col_tiles = 1, double slab_weight = 1.0) {
+                            int64_t col_tiles = 1, double slab_weight = 1.0, double drain = 0.0) {
   constexpr int64_t kCus = 256;
   Slabs p;
   p.tiles = (rows + tile_rows - 1) / tile_rows;
@@ -72,7 +80,8 @@ inline Slabs balanced_slabs(int64_t rows, int64_t cols, int tile_rows, int chunk
     const int64_t per = (chunks + ks - 1) / ks;
     const int64_t slabs = (chunks + per - 1) / per;
     const double m = (double)((p.tiles * col_tiles * slabs + kCus - 1) / kCus) / occ;  // of the busiest CU, in full CUs
-    const double cost = (double)per * (m >= 1.0 ? m : 0.25 + 0.75 * m) + slab_cost * (double)slabs;
+    const double cost = (double)per * (m >= 1.0 ? m : 0.25 + 0.75 * m) +
+                        drain * (double)std::max<int64_t>(per - kDrainChunks, 0) + slab_cost * (double)slabs;
     if (ks == 1 || cost < best) {
       best = cost;
       p.slabs = slabs;
@@ -598,7 +607,8 @@ inline MrhsPlan make_plan(const mplak_kernel_desc* d, int precision, int64_t R) 
   if (p.mfma) {
     p.mode = precision == MPLAK_PREC_BF16 ? kModeBf16 : (precision == MPLAK_PREC_BF16X3 ? kModeBf16x3 : kModeF32);
     p.cblocks = (R + 31) / 32;
-    p.s = balanced_slabs(d->row_count, d->col_count, kMfmaTile, kMfmaSlab, mfma_waves((int)p.cblocks), R);
+    p.s = balanced_slabs(d->row_count, d->col_count, kMfmaTile, kMfmaSlab, mfma_waves((int)p.cblocks), R, 1, 1.0,
+                         kMfmaDrain);
     p.blocks = (d->col_count + kMfmaSlab - 1) / kMfmaSlab;
     p.vpk_bytes = align_up((size_t)p.blocks * (size_t)block_bytes(p.mode, (int)p.cblocks) + kPackAlign, 256);
   } else {
