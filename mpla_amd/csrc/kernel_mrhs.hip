@@ -57,8 +57,9 @@ struct Slabs {
 // than `occ` workgroups takes a chunk down to a quarter of that time.  Measured:
 // partials 4 TB/s and 0.15 us of latency a slab (n = 3000, 16 columns: 47 slabs
 // 27 us, 16 slabs 25 us), against 8 us for a 64-column BF16x3 chunk and 18 us for an
-// FP64 one (n = 20001, 64 columns in FP64: 1.44 ms in 8 slabs, five workgroups
-// on the busiest CU; 1.66 ms in 4, three).
+// FP64 one (n = 20001, 64 columns in FP64, at three waves a SIMD: 1.44 ms in 8
+// slabs, five workgroups on the busiest CU; 1.66 ms in 4, three).  At most 16
+// workgroups a CU, or four rounds of the resident ones.
 // `drain`: share of a long workgroup's chunks (those past kDrainChunks) that the
 // chip is partly idle at the end of a product.  Workgroups that start together
 // end 10 % apart and more, so that one even round of long ones loses to several
@@ -73,7 +74,8 @@ inline Slabs balanced_slabs(int64_t rows, int64_t cols, int tile_rows, int chunk
   Slabs p;
   p.tiles = (rows + tile_rows - 1) / tile_rows;
   const int64_t chunks = (cols + chunk - 1) / chunk;
-  const int64_t most = std::min<int64_t>(chunks, std::max<int64_t>(4 * kCus * occ / (p.tiles * col_tiles), 1));
+  const int64_t most =
+      std::min<int64_t>(chunks, std::max<int64_t>(kCus * std::max(4 * occ, 16) / (p.tiles * col_tiles), 1));
   const double slab_cost = slab_weight * (0.02 + 2.4e-7 * (double)rows * (double)R);
   double best = 0.0;
   for (int64_t ks = 1; ks <= most; ++ks) {
@@ -423,6 +425,16 @@ mrhs_mfma_kernel(const double* const* __restrict__ points, int64_t row_off, int6
 // products at 78.6 TFLOP/s, on top of 270 us for the entries), so the gain is
 // the entries and LDS reads saved.
 //
+// Sums: 256 sources in the matrix cores' accumulators, then added to the slab's
+// sum, as the vector-unit form sums them.  One chain over a slab of thousands
+// of sources loses accuracy with its root (relative error, 2-norm, n = 20001:
+// 1.7e-15 against 5.9e-16; n = 50000: 3.1e-15 against 6.8e-16).  The second set
+// of accumulators leaves two waves per SIMD at 64 columns (n = 20001 1166 us;
+// one chain, three waves 1136 us; Matern 1264 and 1261 us) and three at 32 (683 and
+// 674 us at four).  At 48 three waves fit with the wave's index in a scalar register,
+// so that the staging addresses are scalar too (920 us; two waves 952 us, one
+// chain 882 us); at 64 and 32 columns that form is slower (1204 and 703 us).
+//
 // Row 4 v + r of A takes target 4 r + v of the block, so result v of lane
 // 16 r + c is target 4 r + v, column c, and a lane's four results are
 // consecutive rows of the partials.
@@ -430,8 +442,9 @@ mrhs_mfma_kernel(const double* const* __restrict__ points, int64_t row_off, int6
 constexpr int kSrc64 = 64;                                 // sources per LDS chunk
 constexpr int kTile64 = 32 * (kBlock / kWave);             // 128 targets per workgroup
 constexpr int kSteps64 = kSrc64 / 4;
-// resident waves per SIMD (and workgroups per CU) by column blocks
-constexpr int waves64(int cblocks) { return cblocks <= 2 ? 4 : 3; }
+constexpr int kSumChunks64 = 256 / kSrc64;                 // LDS chunks of one inner sum
+// resident waves per SIMD (and workgroups per CU) by column blocks: above
+constexpr int waves64(int cblocks) { return cblocks == 1 ? 4 : (cblocks <= 3 ? 3 : 2); }
 
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 typedef double f64x2u __attribute__((ext_vector_type(2), aligned(8)));
@@ -449,7 +462,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(waves64(
   __shared__ double lp[DIM][kSrc64];
   __shared__ double tab[kExp2Table];
   fill_exp2_table(tab);  // first read after the chunk barrier below
-  const int tid = threadIdx.x, lane = tid & (kWave - 1), w = tid / kWave;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1);
+  const int w = CB == 3 ? __builtin_amdgcn_readfirstlane(tid / kWave) : tid / kWave;
   const int c16 = lane & 15, r4 = lane >> 4;
   const int64_t base = (int64_t)blockIdx.x * kTile64 + w * 32;
 
@@ -461,14 +475,15 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(waves64(
 #pragma unroll
     for (int d = 0; d < DIM; ++d) p[h][d] = points[d][row_off + i] * scale;
   }
-  f64x4 acc[2][CB];
+  f64x4 acc[2][CB], total[2][CB];
 #pragma unroll
   for (int h = 0; h < 2; ++h)
 #pragma unroll
-    for (int c = 0; c < CB; ++c) acc[h][c] = f64x4{0.0, 0.0, 0.0, 0.0};
+    for (int c = 0; c < CB; ++c) acc[h][c] = total[h][c] = f64x4{0.0, 0.0, 0.0, 0.0};
 
   const int64_t c0 = (int64_t)blockIdx.y * slab_cols;
   const int64_t c1 = c0 + slab_cols < cols ? c0 + slab_cols : cols;
+  int left = kSumChunks64;  // chunks until the inner sum is added to the total
   for (int64_t cb = c0; cb < c1; cb += kSrc64) {
     // lane = source, wave w takes columns w, w + 4, ...: all loads before the
     // barrier, sources and columns past the end are zero
@@ -508,6 +523,16 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(waves64(
         for (int h = 0; h < 2; ++h) acc[h][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(e[h], b, acc[h][c], 0, 0, 0);
       }
     }
+    if (--left == 0 || cb + kSrc64 >= c1) {
+      left = kSumChunks64;
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int c = 0; c < CB; ++c) {
+          total[h][c] += acc[h][c];
+          acc[h][c] = f64x4{0.0, 0.0, 0.0, 0.0};
+        }
+    }
   }
 #pragma unroll
   for (int h = 0; h < 2; ++h)
@@ -517,14 +542,15 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(waves64(
       if (r >= R) continue;
       const int64_t i = base + 16 * h + 4 * r4;
       double* out = part + ((int64_t)blockIdx.y * R + r) * rows + i;
-      const f64x2u lo = {acc[h][c][0], acc[h][c][1]}, hi = {acc[h][c][2], acc[h][c][3]};
+      const f64x4 sum = total[h][c];
+      const f64x2u lo = {sum[0], sum[1]}, hi = {sum[2], sum[3]};
       if (i + 4 <= rows) {
         *reinterpret_cast<f64x2u*>(out) = lo;
         *reinterpret_cast<f64x2u*>(out + 2) = hi;
       } else {
 #pragma unroll
         for (int v = 0; v < 4; ++v)
-          if (i + v < rows) out[v] = acc[h][c][v];
+          if (i + v < rows) out[v] = sum[v];
       }
     }
 }

@@ -1,0 +1,54 @@
+"""Accuracy of the multi-right-hand-side products' sums over many sources.
+
+A running sum of k terms of random sign, rms sigma, has rms sqrt(k) sigma, and
+each of its roundings is a uniform error of rms 0.425 u of the sum (u half the
+spacing at 1; averaged over the logarithm of the mantissa).  A chain of L terms
+therefore errs by 0.425 u sigma L / sqrt(2), n / L such chains by 0.425 u sigma
+sqrt(n L / 2), and relative to the result, of rms sqrt(n) sigma, by 0.425 u
+sqrt(L / 2) whatever n."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from mpla_amd import _native
+from tests.gpu_util import host, require_gpu, stream, workspace
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def lib():
+    require_gpu()
+    return _native.mplak()
+
+
+def sum_error(lib, n, R, kind, prec, rows=64, cols=16):
+    """Relative 2-norm error of the first rows and columns of K V, V of random sign."""
+    import torch
+    dim, ell = (3, 2)[kind], 0.3
+    g = torch.Generator(device="cuda").manual_seed(n + R)
+    P = torch.rand((dim, n), generator=g, dtype=torch.float64, device="cuda")
+    V = torch.rand((R, n), generator=g, dtype=torch.float64, device="cuda") - 0.5
+    Y = torch.empty_like(V)
+    table = torch.tensor([P[d].data_ptr() for d in range(dim)], dtype=torch.int64, device="cuda")
+    desc = _native.mplak_kernel_desc(table.data_ptr(), dim, kind, ell, 0.0, 0.0, 0, n, 0, n)
+    wb = lib.mplak_kernel_mrhs_workspace_bytes(C.byref(desc), prec, R)
+    w = workspace(wb)
+    _native.check(lib.mplak_kernel_mrhs(C.byref(desc), prec, R, V.data_ptr(), n, Y.data_ptr(), n, w.data_ptr(), wb,
+                                        None, stream()))
+    got = host(Y)[:cols, :rows]
+    Pl = host(P).astype(np.longdouble)
+    s = sum((Pl[d, :rows, None] - Pl[d][None]) ** 2 for d in range(dim))
+    r = np.sqrt(3 * s) / np.longdouble(ell)
+    K = np.exp(-s / (2 * np.longdouble(ell) ** 2)) if kind == 0 else (1 + r) * np.exp(-r)
+    ref = host(V)[:cols].astype(np.longdouble) @ K.T
+    return float(np.sqrt(((got - ref) ** 2).sum() / (ref ** 2).sum()))
+
+
+# FP64 on the matrix cores (one to four 16-column blocks): chains of 256 sources.
+# With u for 0.425 u, and 8 u for the entries and the sums of chains and slabs.
+@pytest.mark.parametrize("R", [16, 32, 48, 64])
+@pytest.mark.parametrize("kind", [0, 1])
+def test_mrhs_f64_sums_in_short_chains(lib, R, kind):
+    assert sum_error(lib, 50000, R, kind, _native.MPLAK_PREC_F64) <= 2.0 ** -53 * (np.sqrt(256 / 2) + 8)
