@@ -68,29 +68,47 @@ struct Slabs {
 // iteration with the share taken of every chunk).
 constexpr double kMfmaDrain = 0.12;
 constexpr int64_t kDrainChunks = 64;
+// `longest`: most sources of a slab.
 inline Slabs balanced_slabs(int64_t rows, int64_t cols, int tile_rows, int chunk, int occ, int64_t R,
-                            int64_t col_tiles = 1, double slab_weight = 1.0, double drain = 0.0) {
+                            int64_t col_tiles = 1, double slab_weight = 1.0, double drain = 0.0,
+                            int64_t longest = INT64_MAX) {
   constexpr int64_t kCus = 256;
   Slabs p;
   p.tiles = (rows + tile_rows - 1) / tile_rows;
   const int64_t chunks = (cols + chunk - 1) / chunk;
+  const int64_t least = longest < cols ? (chunks + longest / chunk - 1) / (longest / chunk) : 1;
   const int64_t most =
-      std::min<int64_t>(chunks, std::max<int64_t>(kCus * std::max(4 * occ, 16) / (p.tiles * col_tiles), 1));
+      std::min<int64_t>(chunks, std::max<int64_t>(kCus * std::max(4 * occ, 16) / (p.tiles * col_tiles), least));
   const double slab_cost = slab_weight * (0.02 + 2.4e-7 * (double)rows * (double)R);
   double best = 0.0;
-  for (int64_t ks = 1; ks <= most; ++ks) {
+  for (int64_t ks = least; ks <= most; ++ks) {
     const int64_t per = (chunks + ks - 1) / ks;
     const int64_t slabs = (chunks + per - 1) / per;
     const double m = (double)((p.tiles * col_tiles * slabs + kCus - 1) / kCus) / occ;  // of the busiest CU, in full CUs
     const double cost = (double)per * (m >= 1.0 ? m : 0.25 + 0.75 * m) +
                         drain * (double)std::max<int64_t>(per - kDrainChunks, 0) + slab_cost * (double)slabs;
-    if (ks == 1 || cost < best) {
+    if (ks == least || cost < best) {
       best = cost;
       p.slabs = slabs;
       p.slab_cols = per * chunk;
     }
   }
   return p;
+}
+
+// Most sources of a slab that the matrix cores add up in FP32.  The error of
+// such a sum grows with the root of its length, so a slab is never longer than
+// the share of one of 2048 workgroups of 256 targets: 256 sources up to 11520
+// points, 512 to 16384, 1024 at 20001, 4608 at 50000, 32768 at 131072.  The
+// balance alone would take 704 sources at 9000 points and 1344 at 16000 (relative
+// error of FP32 products 5.0e-7 and 6.6e-7; so bounded 3.2e-7 and 4.3e-7).  The
+// additional partials cost 64 columns, BF16x3, at 9000 points 82 -> 89 us, at 16000
+// 179 -> 185 us, at 50000 nothing.
+inline int64_t longest_fp32_slab(int64_t rows, int64_t cols) {
+  constexpr int64_t kTile = 256, kWorkgroups = 2048;
+  const int64_t tiles = (rows + kTile - 1) / kTile, chunks = (cols + kTile - 1) / kTile;
+  const int64_t slabs = std::min((kWorkgroups + tiles - 1) / tiles, chunks);
+  return (chunks + slabs - 1) / slabs * kTile;
 }
 
 // ---------------------------------------------------------------------------
@@ -634,7 +652,7 @@ inline MrhsPlan make_plan(const mplak_kernel_desc* d, int precision, int64_t R) 
     p.mode = precision == MPLAK_PREC_BF16 ? kModeBf16 : (precision == MPLAK_PREC_BF16X3 ? kModeBf16x3 : kModeF32);
     p.cblocks = (R + 31) / 32;
     p.s = balanced_slabs(d->row_count, d->col_count, kMfmaTile, kMfmaSlab, mfma_waves((int)p.cblocks), R, 1, 1.0,
-                         kMfmaDrain);
+                         kMfmaDrain, longest_fp32_slab(d->row_count, d->col_count));
     p.blocks = (d->col_count + kMfmaSlab - 1) / kMfmaSlab;
     p.vpk_bytes = align_up((size_t)p.blocks * (size_t)block_bytes(p.mode, (int)p.cblocks) + kPackAlign, 256);
   } else {

@@ -52,3 +52,12 @@ def sum_error(lib, n, R, kind, prec, rows=64, cols=16):
 @pytest.mark.parametrize("kind", [0, 1])
 def test_mrhs_f64_sums_in_short_chains(lib, R, kind):
     assert sum_error(lib, 50000, R, kind, _native.MPLAK_PREC_F64) <= 2.0 ** -53 * (np.sqrt(256 / 2) + 8)
+
+
+# FP32 on the matrix cores: chains of at most 512 sources at 16000 points (FP64
+# sums of them); a quarter on top for the entries' few roundings.
+@pytest.mark.parametrize("R", [32, 64])
+@pytest.mark.parametrize("kind", [0, 1])
+def test_mrhs_f32_sums_in_short_chains(lib, R, kind):
+    bound = 1.25 * 0.425 * 2.0 ** -24 * np.sqrt(512 / 2)
+    assert sum_error(lib, 16000, R, kind, _native.MPLAK_PREC_F32) <= bound
