@@ -145,6 +145,7 @@ __global__ __launch_bounds__(kBlock) void dot_final_kernel(const double* __restr
 // ---------------------------------------------------------------------------
 
 constexpr int kGvUnroll = 8;                                // columns of a lane in flight
+constexpr int kGvSumRounds = 256 / kGvUnroll;               // rounds of them in one running sum
 constexpr int kGvStreamLanes = 64, kGvPanelLanes = 8;       // 128-row and 16-row panels
 constexpr double kGvPanelBytes = 40e6;                      // largest matrix of the 16-row panels
 constexpr int64_t kGvPanelRows = 64;                        // or most rows at any size
@@ -248,7 +249,10 @@ __global__ __launch_bounds__(NW* kWave) void dgemv_partial_kernel(int64_t m, int
   // column offset of the lane's u-th load of a round
   auto col = [](int u) { return (u / 2) * 2 * CG + (u & 1); };
 
-  double acc0 = 0.0, acc1 = 0.0;
+  // running sums of 256 columns, then their sum: a single one over the thousands
+  // of columns of a wave would lose accuracy with the root of its length
+  double sum0 = 0.0, sum1 = 0.0, acc0 = 0.0, acc1 = 0.0;
+  int left = kGvSumRounds;
   int64_t j = j0 + 2 * g;
   const double* a = A + b + j * lda;
   int64_t jw = j0;
@@ -275,6 +279,12 @@ __global__ __launch_bounds__(NW* kWave) void dgemv_partial_kernel(int64_t m, int
     }
     j += U * CG;
     a += (int64_t)(U * CG) * lda;
+    if (--left == 0) {
+      left = kGvSumRounds;
+      sum0 += acc0;
+      sum1 += acc1;
+      acc0 = acc1 = 0.0;
+    }
   }
   if (jw < j1) {
     // the last columns of the share, fewer than U CG: an absent column is
@@ -299,6 +309,8 @@ __global__ __launch_bounds__(NW* kWave) void dgemv_partial_kernel(int64_t m, int
       }
     }
   }
+  acc0 += sum0;
+  acc1 += sum1;
 #pragma unroll
   for (int s = RL; s < kWave; s <<= 1) {
     acc0 += __shfl_xor(acc0, s, kWave);

@@ -1,4 +1,4 @@
-"""Accuracy of the multi-right-hand-side products' sums over many sources.
+"""Accuracy of the products' sums over many sources or columns.
 
 A running sum of k terms of random sign, rms sigma, has rms sqrt(k) sigma, and
 each of its roundings is a uniform error of rms 0.425 u of the sum (u half the
@@ -61,3 +61,23 @@ def test_mrhs_f64_sums_in_short_chains(lib, R, kind):
 def test_mrhs_f32_sums_in_short_chains(lib, R, kind):
     bound = 1.25 * 0.425 * 2.0 ** -24 * np.sqrt(512 / 2)
     assert sum_error(lib, 16000, R, kind, _native.MPLAK_PREC_F32) <= bound
+
+
+# Streamed dense products: running sums of 256 columns, added over a wave's
+# thousands of columns (one slab and several; odd strides), then over the waves.
+@pytest.mark.parametrize("m,n,lda", [(20000, 16000, 20000), (16385, 16385, 16387), (140000, 4001, 140000)])
+def test_dgemv_sums_in_short_chains(lib, m, n, lda):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(n)
+    A = torch.rand((n, lda), generator=g, dtype=torch.float64, device="cuda") - 0.5
+    x = torch.rand(n, generator=g, dtype=torch.float64, device="cuda") - 0.5
+    y = torch.empty(m, dtype=torch.float64, device="cuda")
+    wb = lib.mplak_dgemv_workspace_bytes(m, n)
+    w = workspace(wb)
+    _native.check(lib.mplak_dgemv_f64(m, n, A.data_ptr(), lda, x.data_ptr(), y.data_ptr(), w.data_ptr(), wb, None,
+                                      stream()))
+    rows = slice(m // 2, m // 2 + 200)
+    ref = host(A[:, rows]).T.astype(np.longdouble) @ host(x).astype(np.longdouble)
+    error = float(np.sqrt(((host(y)[rows] - ref) ** 2).sum() / (ref ** 2).sum()))
+    # chains of 256, up to n / 256 of them in a row, and the last sums
+    assert error <= 0.425 * 2.0 ** -53 * (np.sqrt(256 / 2) + np.sqrt(n / 256 / 2) + 2)
