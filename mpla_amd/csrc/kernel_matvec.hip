@@ -816,9 +816,11 @@ __device__ __forceinline__ void sym_mfma_pair(const double* const (&coord)[3], i
         for (int v = 0; v < 4; ++v) {
           float sv;
           if constexpr (DOT) {
-            sv = FACTOR ? nq[b] : pc[DIM][v] + nq[b];
+            // as the matrix cores add: the target's norm last
+            sv = nq[b];
 #pragma unroll
             for (int d = 0; d < DIM; ++d) sv = fmaf(pc[d][v], q[b][d], sv);
+            if (!FACTOR) sv += pc[DIM][v];
           } else {
             sv = s[b][v];
           }

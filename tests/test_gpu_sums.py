@@ -81,3 +81,34 @@ def test_dgemv_sums_in_short_chains(lib, m, n, lda):
     error = float(np.sqrt(((host(y)[rows] - ref) ** 2).sum() / (ref ** 2).sum()))
     # chains of 256, up to n / 256 of them in a row, and the last sums
     assert error <= 0.425 * 2.0 ** -53 * (np.sqrt(256 / 2) + np.sqrt(n / 256 / 2) + 2)
+
+
+# Planned FP32 Matern products form squared distances on the vector unit in 1-D
+# and 2-D, on the matrix cores in 3-D: the same points with coordinates of zero
+# added are as accurate either way.
+@pytest.mark.parametrize("n", [2000, 4096, 8000])
+@pytest.mark.parametrize("dim,ell", [(1, 0.02), (2, 0.1)])
+def test_planned_fp32_distances_of_both_forms(lib, n, dim, ell):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(n)
+    P = torch.rand((dim, n), generator=g, dtype=torch.float64, device="cuda")
+    table = torch.tensor([P[d].data_ptr() for d in range(dim)], dtype=torch.int64, device="cuda")
+    ob = lib.mplak_spatial_order_workspace_bytes(n, dim)
+    w, perm = workspace(ob), torch.empty(n, dtype=torch.int64, device="cuda")
+    _native.check(lib.mplak_spatial_order(table.data_ptr(), dim, 0, n, perm.data_ptr(), w.data_ptr(), ob, stream()))
+    P = torch.cat([P[:, perm], torch.zeros((3 - dim, n), dtype=torch.float64, device="cuda")]).contiguous()
+    x = torch.rand(n, generator=g, dtype=torch.float64, device="cuda") - 0.5
+    r = (3.0 * sum((P[d, :, None] - P[d][None]) ** 2 for d in range(dim))).sqrt() / ell
+    ref = ((1.0 + r) * (-r).exp()) @ x + x
+    table = torch.tensor([P[d].data_ptr() for d in range(3)], dtype=torch.int64, device="cuda")
+    error = {}
+    for form in (dim, 3):
+        desc = _native.mplak_kernel_desc(table.data_ptr(), form, 1, ell, 1.0, 0.0, 0, n, 0, n)
+        pb = lib.mplak_screen_plan_bytes(C.byref(desc))
+        plan, y = workspace(pb), torch.empty_like(x)
+        _native.check(lib.mplak_screen_plan_build(C.byref(desc), _native.MPLAK_PREC_F32, 40.0, plan.data_ptr(), pb,
+                                                  stream()))
+        _native.check(lib.mplak_kernel_matvec_planned(C.byref(desc), _native.MPLAK_PREC_F32, 40.0, plan.data_ptr(), pb,
+                                                      x.data_ptr(), y.data_ptr(), None, stream()))
+        error[form] = float((y - ref).norm() / ref.norm())
+    assert error[dim] <= 1.05 * error[3]
