@@ -545,7 +545,7 @@ typedef struct mplak_ragged_system {
                             reference counterpart); 0: exact product */
   double drop_s;         /* planned */
   int32_t scheme;        /* planned: MPLAK_RAGGED_SLABS or MPLAK_RAGGED_PAIRS */
-  int32_t reserved;      /* planned: workgroups per tile pair (0 and 1: one) */
+  int32_t reserved;      /* planned: PAIRS: workgroups per tile pair (0 and 1: one); SLABS: nonzero for FP32 partials */
 } mplak_ragged_system;
 
 /* Work split of a ragged product.
@@ -572,11 +572,16 @@ typedef struct mplak_ragged_item {
  * needs. */
 size_t mplak_ragged_plan(mplak_ragged_system* s);
 
-/* Host only: the same for mplak_ragged_product_mixed (FP32) and, by class, FP64
- * products of the same system: pairs from n = 2048, shared by up to 8 workgroups
- * each (`reserved`; the item's slab field is the part), shorter slabs, and FP32
- * column tiles of min(nrhs, 8). */
+/* Host only: the same for FP32 products by mplak_ragged_product_mixed: pairs from
+ * n = 2048, shared by up to 8 workgroups each (`reserved`; the item's slab field
+ * is the part), shorter slabs, and column tiles of min(nrhs, 8), as far as the
+ * partials fit the bytes of the system's FP64 plan.  FP64 systems are planned as
+ * by mplak_ragged_plan. */
 size_t mplak_ragged_plan_mixed(mplak_ragged_system* s);
+
+/* Host only: the same for a `part` buffer of `bytes` (at least those of the
+ * system's FP64 plan). */
+size_t mplak_ragged_plan_within(mplak_ragged_system* s, size_t bytes);
 
 /* Host only: number of product / finish work items of a planned system; when
  * `out` is non-NULL also writes them (sys field = sys_index). */

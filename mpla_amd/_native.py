@@ -202,6 +202,7 @@ MPLAK_SIGNATURES = {
     "mplak_bcg_copy_states": (C.c_int, [_vp, _vp, _i64, _vp, _vp]),
     "mplak_ragged_plan": (_sz, [_vp]),
     "mplak_ragged_plan_mixed": (_sz, [_vp]),
+    "mplak_ragged_plan_within": (_sz, [_vp, _sz]),
     "mplak_ragged_product_mixed": (C.c_int, [_vp, _vp, _i64, _vp]),
     "mplak_ragged_product_items": (_i64, [_vp, _vp, _i32]),
     "mplak_ragged_finish_items": (_i64, [_vp, _vp, _i32]),

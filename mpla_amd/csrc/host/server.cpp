@@ -90,7 +90,7 @@ Layout layout_for(int64_t n, int dim, int nrhs) {
   s.kind = MPLAK_KERNEL_GAUSSIAN;
   s.length_scale = 1.0;
   s.precision = MPLAK_PREC_F64;
-  L.part = align256(mplak_ragged_plan_mixed(&s));
+  L.part = align256(mplak_ragged_plan(&s));
   L.cgpart = align256(mplak_ragged_cg_part_bytes(n, nrhs));
   L.perm = align256(sizeof(int64_t) * (size_t)n);
   L.total = L.points + 6 * L.vec + L.part + L.cgpart + L.perm;  // points, B, X, R, D, Z, E, spatial order
@@ -109,6 +109,7 @@ struct Request {
   size_t block_bytes = 0;
   double *points = nullptr, *B = nullptr, *X = nullptr, *R = nullptr, *D = nullptr, *Z = nullptr, *E = nullptr;
   double *part = nullptr, *cgpart = nullptr;
+  size_t part_bytes = 0;
   int64_t* perm = nullptr;  // spatial order (mixed mode): stored row k is request row perm[k]
   bool ordered = false;
   double residual_drop = 0.0;  // screen of the FP64 products (mixed mode; 0 = exact)
@@ -231,7 +232,7 @@ mplak_ragged_system product_system(const Request& r, int precision, const double
   sy.kind = r.req.kind;
   sy.nrhs = r.req.nrhs;
   sy.precision = precision;
-  mplak_ragged_plan_mixed(&sy);
+  if (mplak_ragged_plan_within(&sy, r.part_bytes) > r.part_bytes) fail("server product", "partials exceed the request's buffer");
   return sy;
 }
 
@@ -343,11 +344,14 @@ bool admit(mpla_server* s, Request* r) {
     *v = reinterpret_cast<double*>(p);
     p += L.vec;
   }
-  r->part = reinterpret_cast<double*>(p);
-  p += L.part;
   r->cgpart = reinterpret_cast<double*>(p);
   p += L.cgpart;
   r->perm = reinterpret_cast<int64_t*>(p);
+  p += L.perm;
+  // the partials take the rest of the block: its rounding lets the FP32 products
+  // of small requests be split further
+  r->part = reinterpret_cast<double*>(p);
+  r->part_bytes = need - (L.total - L.part);
   const int64_t n = r->req.n;
   const int dim = r->req.dim;
   r->ordered = s->cfg.mode == MPLA_SERVE_MIXED_BATCHED && (s->inner_drop > 0.0 || s->residual_drop > 0.0);

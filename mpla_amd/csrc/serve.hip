@@ -53,6 +53,10 @@ struct SlabLds {
   double exp_tab[Exp2Lds<T>::size];
 };
 
+// A mixed plan's FP32 slabs of one chunk leave FP32 partials, the values of the
+// FP64 ones in half the bytes.
+__host__ __device__ inline bool narrow_slabs(const mplak_ragged_system& S) { return S.reserved != 0; }
+
 // DIM > 0: the system has that dimension; DIM == 0: any dimension <=
 // kMaxRaggedDim (coordinates past it are zero).
 template <typename T, int RT, int DIM>
@@ -172,9 +176,14 @@ __device__ __forceinline__ void slab_item(const mplak_ragged_item& it, const mpl
     for (int q = 0; q < RT; ++q) acc[q] += (double)cacc[q];
   }
   if (active) {
+    float* part32 = reinterpret_cast<float*>(S.part);
 #pragma unroll
-    for (int q = 0; q < RT; ++q)
-      if (r0 + q < R) S.part[((int64_t)it.slab * R + r0 + q) * n + i] = acc[q];
+    for (int q = 0; q < RT; ++q) {
+      if (r0 + q >= R) continue;
+      const int64_t k = ((int64_t)it.slab * R + r0 + q) * n + i;
+      if (sizeof(T) == 4 && narrow_slabs(S)) part32[k] = (float)acc[q];
+      else S.part[k] = acc[q];
+    }
   }
 }
 
@@ -544,6 +553,23 @@ __device__ __forceinline__ double pair_finish_row(const mplak_ragged_system& S, 
   return s;
 }
 
+// Slice k of the partials p[0], p[stride], ... of an entry's slabs.
+template <typename T>
+__device__ __forceinline__ double slab_finish_row(const T* __restrict__ p, int32_t slabs, int64_t stride, int k) {
+  double s = 0.0;
+  for (int64_t m0 = k; m0 < slabs; m0 += kFinishLoads * kFinishSlices) {
+    double v[kFinishLoads];
+#pragma unroll
+    for (int u = 0; u < kFinishLoads; ++u) {
+      const int64_t m = m0 + u * kFinishSlices;
+      v[u] = m < slabs ? (double)p[m * stride] : 0.0;
+    }
+#pragma unroll
+    for (int u = 0; u < kFinishLoads; ++u) s += v[u];
+  }
+  return s;
+}
+
 // items: (system, block) over n * nrhs entries of Y, 256 per item in four
 // workgroups
 __global__ __launch_bounds__(kBlock) void ragged_finish_kernel(const mplak_ragged_system* __restrict__ systems,
@@ -563,17 +589,8 @@ __global__ __launch_bounds__(kBlock) void ragged_finish_kernel(const mplak_ragge
     if (S.scheme == MPLAK_RAGGED_PAIRS) {
       s = S.precision == MPLAK_PREC_F64 ? pair_finish_row<double>(S, i, r, k) : pair_finish_row<float>(S, i, r, k);
     } else {
-      const double* p = S.part + r * n + i;
-      for (int64_t m0 = k; m0 < S.slabs; m0 += kFinishLoads * kFinishSlices) {
-        double v[kFinishLoads];
-#pragma unroll
-        for (int u = 0; u < kFinishLoads; ++u) {
-          const int64_t m = m0 + u * kFinishSlices;
-          v[u] = m < S.slabs ? p[m * R * n] : 0.0;
-        }
-#pragma unroll
-        for (int u = 0; u < kFinishLoads; ++u) s += v[u];
-      }
+      s = narrow_slabs(S) ? slab_finish_row(reinterpret_cast<const float*>(S.part) + r * n + i, S.slabs, R * n, k)
+                          : slab_finish_row(S.part + r * n + i, S.slabs, R * n, k);
     }
   }
   red[k][lane] = s;
@@ -814,11 +831,9 @@ bool use_pairs(int64_t n, int64_t least) {
 
 static_assert(kPairGroups == 8, "pair_finish_row: parts of 8 groups");
 
-// Work split of a system whose column tiles are `rt` wide: tile pairs from
-// `pairs_from` points on, shared by `parts` workgroups each, and slabs of at
-// least `unit` sources otherwise.
-size_t plan_split(mplak_ragged_system* s, int rt, int64_t pairs_from, int64_t unit, int parts) {
-  if (s == nullptr || s->n <= 0 || s->nrhs <= 0 || s->dim < 1 || s->dim > kMaxRaggedDim) return 0;
+// Scale, tiles and, in slabs of whole `unit`s of sources, the split of a system
+// whose column tiles are `rt` wide.
+void plan_slabs(mplak_ragged_system* s, int rt, int64_t unit) {
   s->rt = rt;
   s->ctiles = (s->nrhs + s->rt - 1) / s->rt;
   s->tiles = (int32_t)((s->n + kBlock - 1) / kBlock);
@@ -831,31 +846,46 @@ size_t plan_split(mplak_ragged_system* s, int rt, int64_t pairs_from, int64_t un
   s->slabs = (int32_t)((s->n + s->slab_cols - 1) / s->slab_cols);
   s->scale = coord_scale(s->kind, s->length_scale);
   s->drop_s = s->drop_log2 > 0.0 ? drop_distance2(s->kind, s->drop_log2) : 0.0;
-  s->reserved = 0;
-  if (use_pairs(s->n, pairs_from)) {
-    s->scheme = MPLAK_RAGGED_PAIRS;
-    s->tiles = (int32_t)((s->n + kPairTile - 1) / kPairTile);
-    s->slabs = 0;
-    s->slab_cols = 0;
-    const size_t es = s->precision == MPLAK_PREC_F64 ? sizeof(double) : sizeof(float);
-    const size_t pairs = (size_t)pair_count(s->tiles);
-    s->reserved = parts;
-    return align_up((size_t)(parts + 1) * pairs * (size_t)s->nrhs * kPairTile * es, 256) +
-           align_up((size_t)parts * pairs * sizeof(int32_t), 256);
-  }
   s->scheme = MPLAK_RAGGED_SLABS;
-  return (size_t)s->slabs * (size_t)s->nrhs * (size_t)s->n * sizeof(double);
+  s->reserved = 0;
 }
 
-// Workgroups per tile pair in a mixed launch, from n alone: the largest power of
-// two up to 8 that keeps pairs times workgroups below 1200.  One workgroup a
-// pair leaves a 13455-point system's 378 pairs on 256 CUs, two on some and one
-// on the others; each further part is another row set for the finish to read
-// (twelve requests of up to 24576 points: 60.1 ms at 1200, 61.8 ms at 600).
-int mixed_parts(int64_t n) {
-  const int64_t pairs = pair_count((n + kPairTile - 1) / kPairTile);
+size_t slab_part_bytes(const mplak_ragged_system* s) {
+  return (size_t)s->slabs * (size_t)s->nrhs * (size_t)s->n * (narrow_slabs(*s) ? sizeof(float) : sizeof(double));
+}
+
+// Partials of a system in pairs shared by `parts` workgroups each.
+size_t pair_part_bytes(const mplak_ragged_system* s, int parts) {
+  const size_t es = s->precision == MPLAK_PREC_F64 ? sizeof(double) : sizeof(float);
+  const size_t pairs = (size_t)pair_count((s->n + kPairTile - 1) / kPairTile);
+  return align_up((size_t)(parts + 1) * pairs * (size_t)s->nrhs * kPairTile * es, 256) +
+         align_up((size_t)parts * pairs * sizeof(int32_t), 256);
+}
+
+size_t plan_pairs(mplak_ragged_system* s, int parts) {
+  s->scheme = MPLAK_RAGGED_PAIRS;
+  s->tiles = (int32_t)((s->n + kPairTile - 1) / kPairTile);
+  s->slabs = 0;
+  s->slab_cols = 0;
+  s->reserved = parts;
+  return pair_part_bytes(s, parts);
+}
+
+bool plannable(const mplak_ragged_system* s) {
+  return s != nullptr && s->n > 0 && s->nrhs > 0 && s->dim >= 1 && s->dim <= kMaxRaggedDim;
+}
+
+// Workgroups per tile pair in a mixed launch: the largest power of two up to 8
+// that keeps pairs times workgroups below 1200 and the partials within `bytes`
+// (0 if none does).  One workgroup a pair leaves a 13455-point system's 378 pairs
+// on 256 CUs, two on some and one on the others; each further part is another
+// row set for the finish to read (twelve requests of up to 24576 points: 60.1 ms
+// at 1200, 61.8 ms at 600).
+int mixed_parts(const mplak_ragged_system* s, size_t bytes) {
+  const int64_t pairs = pair_count((s->n + kPairTile - 1) / kPairTile);
   int k = 1;
   while (k < kPairGroups && pairs * (2 * k) < 1200) k *= 2;
+  while (k > 0 && pair_part_bytes(s, k) > bytes) k /= 2;
   return k;
 }
 
@@ -867,14 +897,32 @@ using namespace mplak;
 extern "C" {
 
 size_t mplak_ragged_plan(mplak_ragged_system* s) {
-  return plan_split(s, s != nullptr ? rt_class(s->nrhs) : 1, kRagPairMinN, kChunk, 1);
+  if (!plannable(s)) return 0;
+  plan_slabs(s, rt_class(s->nrhs), kChunk);
+  return use_pairs(s->n, kRagPairMinN) ? plan_pairs(s, 1) : slab_part_bytes(s);
 }
 
 size_t mplak_ragged_plan_mixed(mplak_ragged_system* s) {
-  if (s == nullptr || s->nrhs <= 0 || s->n <= 0) return 0;
-  // FP64 systems are launched by class, whose column tiles are powers of two
-  const int rt = s->precision == MPLAK_PREC_F64 ? rt_class(s->nrhs) : (s->nrhs < 8 ? s->nrhs : 8);
-  return plan_split(s, rt, kMixedPairMinN, kWave, mixed_parts(s->n));
+  if (!plannable(s)) return 0;
+  mplak_ragged_system wide = *s;
+  wide.precision = MPLAK_PREC_F64;
+  return mplak_ragged_plan_within(s, mplak_ragged_plan(&wide));
+}
+
+size_t mplak_ragged_plan_within(mplak_ragged_system* s, size_t bytes) {
+  // FP64 systems are launched by class
+  if (!plannable(s) || s->precision == MPLAK_PREC_F64) return mplak_ragged_plan(s);
+  const int rt = s->nrhs < 8 ? s->nrhs : 8;
+  plan_slabs(s, rt, kWave);
+  // whole pairs would sum 512 sources in FP32 where slabs sum 256
+  const int parts = use_pairs(s->n, kMixedPairMinN) ? mixed_parts(s, bytes) : 0;
+  if (parts > (use_pairs(s->n, kRagPairMinN) ? 0 : 1)) return plan_pairs(s, parts);
+  for (int64_t unit = kWave;; unit *= 2) {
+    plan_slabs(s, rt, unit);
+    s->reserved = s->slab_cols <= kChunk;
+    const size_t need = slab_part_bytes(s);
+    if (need <= bytes || unit == kChunk) return need;
+  }
 }
 
 int64_t mplak_ragged_product_items(const mplak_ragged_system* s, mplak_ragged_item* out, int32_t sys_index) {

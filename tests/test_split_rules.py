@@ -36,3 +36,33 @@ def test_fp32_sums_of_block_products_stay_short(lib, prec, rows, cols, R):
     packed = -(-(-(-cols // 64) * (64 * 16 + ops) + 16) // 256) * 256
     slabs = (lib.mplak_kernel_mrhs_workspace_bytes(C.byref(desc(rows, cols)), prec, R) - packed) // (4 * R * rows)
     assert slabs * longest >= cols
+
+
+# A served request's buffer of partials is that of its FP64 products by class; its
+# FP32 products in mixed launches are split as far as the same buffer allows.
+@pytest.mark.parametrize("n", [1, 64, 300, 1000, 2047, 2048, 4096, 6001, 8000, 8191, 8192, 9999, 12288, 13455, 20000])
+@pytest.mark.parametrize("nrhs", [1, 3, 8, 17, 64])
+@pytest.mark.parametrize("pairs", [None, "0", "1"])
+def test_served_partials_fit_the_fp64_plan(lib, monkeypatch, n, nrhs, pairs):
+    from mpla_amd import mpla
+    monkeypatch.delenv("MPLAK_RAGGED_PAIRS", raising=False)
+    if pairs is not None:
+        monkeypatch.setenv("MPLAK_RAGGED_PAIRS", pairs)
+
+    def plan(query, prec):
+        s = _native.mplak_ragged_system()
+        s.n, s.nrhs, s.dim, s.kind, s.length_scale, s.precision = n, nrhs, 3, 0, 0.5, prec
+        return query(C.byref(s)), s
+
+    tiles = -(-n // 512)
+    by_class, s = plan(lib.mplak_ragged_plan, F64)
+    if pairs == "0" or (pairs is None and n < 8192):
+        assert s.scheme == 0 and s.slab_cols % 256 == 0 and by_class == 8 * s.slabs * nrhs * n
+    else:
+        assert s.scheme == 1 and 0 <= by_class - 8 * 512 * tiles * (tiles + 1) * nrhs <= 8 * tiles * (tiles + 1) + 512
+    assert plan(lib.mplak_ragged_plan_mixed, F64)[0] == by_class
+    assert 0 < plan(lib.mplak_ragged_plan_mixed, F32)[0] <= by_class
+    assert 0 < plan(lambda s: lib.mplak_ragged_plan_within(s, by_class + 300000), F32)[0] <= by_class + 300000
+    up = lambda b, to=256: -(-b // to) * to  # noqa: E731
+    total = up(24 * n) + 6 * up(8 * n * nrhs) + up(by_class) + up(lib.mplak_ragged_cg_part_bytes(n, nrhs)) + up(8 * n)
+    assert mpla.lib().mpla_server_request_bytes(n, 3, nrhs) == up(total, 1 << 20)
