@@ -356,6 +356,34 @@ __global__ __launch_bounds__(hm::kHmRows) void pairs_finish_kernel(
   y[i] = s;
 }
 
+// Far field and near partials of one apply chunk in one launch: wave p of the
+// workgroup's 8 adds the chunk's partial blocks p, p + 8, ... and its share of the
+// admissible blocks; the eight sums of a row are added in wave order.
+__global__ __launch_bounds__(hm::kHmApplyThreads) void apply_pairs_kernel(
+    const mplak_hm_chunk* __restrict__ chunks, const int64_t* __restrict__ chunk_near,
+    const int64_t* __restrict__ near_start, const int64_t* __restrict__ ent_ptr, const int64_t* __restrict__ ent,
+    const double* __restrict__ part, const int64_t* __restrict__ far_ptr, const int32_t* __restrict__ far_blk,
+    const mplak_hm_block* __restrict__ blocks, const int32_t* __restrict__ rank, int kmax,
+    const double* __restrict__ U, const double* __restrict__ t, double* __restrict__ ys) {
+  __shared__ double red[hm::kHmParts][hm::kHmRows];
+  const mplak_hm_chunk c = chunks[blockIdx.x];
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+  int64_t row[hm::kHmLaneRows];
+  bool valid[hm::kHmLaneRows];
+  hm::item_rows(c, row, valid);
+  const int64_t nc = chunk_near[blockIdx.x];
+  const int64_t off = c.r0 - near_start[nc];
+  double acc[hm::kHmLaneRows] = {};
+  for (int64_t k = ent_ptr[nc] + w; k < ent_ptr[nc + 1]; k += hm::kHmParts) {
+    const double* blk = part + ent[k] * kPairRows + off;
+#pragma unroll
+    for (int h = 0; h < hm::kHmLaneRows; ++h)
+      if (valid[h]) acc[h] += blk[h * kWave + lane];
+  }
+  hm::far_rows<false>(row, valid, far_ptr, far_blk, c.leaf, blocks, rank, kmax, U, t, w, hm::kHmParts, acc);
+  hm::finish_rows(acc, row, valid, ys, red);
+}
+
 // Kernel and dimension of `p` as compile-time values for `go`.
 template <typename F>
 void with_points(const mplak_hm_points* p, F&& go) {
@@ -568,14 +596,10 @@ int mplak_hm_apply_pairs(const mplak_hm_chunk* chunks, int64_t nchunks, const in
   if (chunks == nullptr || chunk_near == nullptr || near_start == nullptr || ent_ptr == nullptr || far_ptr == nullptr ||
       ys == nullptr)
     return MPLAK_ERR_ARG;
-  // no pairs in this launch: any kernel and dimension do
-  hipLaunchKernelGGL((rows_near_kernel<MPLAK_KERNEL_GAUSSIAN, 1, false>), dim3((unsigned)nchunks), dim3(kBlock), 0,
-                     as_stream(stream), chunks, far_ptr, far_blk, blocks, rank, kmax, U, t, ys, nullptr, nullptr, 0,
-                     nullptr, 0, nullptr);
-  const int st = launch_status();
-  if (st != MPLAK_OK) return st;
-  return mplak_hm_pairs_finish(chunks, nchunks, chunk_near, near_start, ent_ptr, ent, part, ys, nullptr, 0.0, nullptr,
-                               0, 0, nullptr, stream);
+  hipLaunchKernelGGL(apply_pairs_kernel, dim3((unsigned)nchunks), dim3(hm::kHmApplyThreads), 0, as_stream(stream),
+                     chunks, chunk_near, near_start, ent_ptr, ent, part, far_ptr, far_blk, blocks, rank, kmax, U, t,
+                     ys);
+  return launch_status();
 }
 
 int mplak_hm_apply_stored(const mplak_hm_chunk* chunks, int64_t nchunks, const int64_t* leaf_range,
