@@ -61,7 +61,8 @@ constexpr int kKmvChunk = kBlock;              // sources per LDS chunk
 constexpr int kKmvMaxDim = 16;
 constexpr int kKmvMinSlab = 32;                // fewest sources of a slab
 constexpr int64_t kKmvMaxSlabs = 64;
-constexpr int64_t kKmvMaxBlocks = 8192;        // bounds the partials at 16.8 MB
+constexpr int64_t kKmvFewBlocks = 1024;        // workgroups up to which few targets have more slabs
+constexpr int64_t kKmvMaxBlocks = 8192;        // bounds the partials of several slabs at 16.8 MB
 constexpr int kFinishLoads = 16;               // slab partials in flight per row
 
 struct KmvPlan {
@@ -74,10 +75,16 @@ struct KmvPlan {
 // 64 / 32 sources: n = 1000 19.6 / 12.6 / 9.5 / 8.8 us, n = 3001 21.1 / 18.6 /
 // 16.7 / 18.3 us, n = 8000 51.7 / 51.4 / 54.3 / 62.5 us.  One target a thread
 // is faster than two at every size there (n = 3001: 16.7 against 19.8 us).
+// Fewer targets still (up to 3840) against more than 4096 sources would leave CUs
+// idle: the slab count then balances a slab's chain (0.064 us a source) and the
+// finish (0.06 us a slab) at the root of the sources, up to four workgroups a CU.
+// FP64 Gaussian in 3-D, 64 slabs / balanced: 1 x 65536 66 / 34 us, 256 x 1000000 915 /
+// 208 us, 512 x 65536 66 / 42 us, 1024 x 65536 66 / 58 us, 2048 x 65536 95 / 91 us.
 inline KmvPlan kmv_plan(int64_t rows, int64_t cols) {
   KmvPlan p;
   p.row_tiles = (rows + kBlock - 1) / kBlock;
-  const int64_t most = std::max<int64_t>(std::min(kKmvMaxSlabs, kKmvMaxBlocks / p.row_tiles), 1);
+  const int64_t few = std::min((int64_t)std::sqrt((double)cols), kKmvFewBlocks / p.row_tiles);
+  const int64_t most = std::max<int64_t>(std::min(std::max(kKmvMaxSlabs, few), kKmvMaxBlocks / p.row_tiles), 1);
   p.slab_cols = kKmvMinSlab;
   while (p.slab_cols < kKmvChunk && (cols + p.slab_cols - 1) / p.slab_cols > most) p.slab_cols *= 2;
   if ((cols + p.slab_cols - 1) / p.slab_cols > most) {

@@ -66,3 +66,13 @@ def test_served_partials_fit_the_fp64_plan(lib, monkeypatch, n, nrhs, pairs):
     up = lambda b, to=256: -(-b // to) * to  # noqa: E731
     total = up(24 * n) + 6 * up(8 * n * nrhs) + up(by_class) + up(lib.mplak_ragged_cg_part_bytes(n, nrhs)) + up(8 * n)
     assert mpla.lib().mpla_server_request_bytes(n, 3, nrhs) == up(total, 1 << 20)
+
+
+# Exact products of few targets and many sources: at least one workgroup (256
+# targets, one slab) per CU, and partials that stay within 17 MB.
+@pytest.mark.parametrize("rows,cols", [(1, 65536), (256, 65536), (200, 1000000), (257, 65536), (512, 131072),
+                                       (1000, 65536), (2048, 65536), (3840, 65535), (3841, 65536), (8192, 65536)])
+def test_few_targets_fill_the_chip(lib, rows, cols):
+    partials = lib.mplak_kernel_matvec_workspace_bytes(C.byref(desc(rows, cols)))
+    slabs = partials // (8 * rows)
+    assert -(-rows // 256) * slabs >= 256 and partials <= 17e6
