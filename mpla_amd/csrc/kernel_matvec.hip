@@ -1617,21 +1617,14 @@ inline int planned_split(int64_t nt) {
 }
 
 // Workgroups per pair of the vector unit's symmetric products (exact, screened
-// and, with a coincidence shift, planned, whose sums are bitwise the same): the
-// largest power of two up to 8 that keeps pairs times workgroups within 7000, below 820 pairs (n =
-// 20000).  Few whole pairs leave CUs idle or their last round nearly empty.
-// FP64, 3-D Gaussian, at 1 / 2 / 4 / 8 workgroups a pair: n = 5000 60.8 / 35.0 /
-// 24.2 / 21.2 us, n = 16000 140 / 118 / 114 / 110 us.  From 820 pairs on the
-// workspace stays at two row sets a pair, its documented size; there the gain
-// falls from 12 % (n = 20000, 183 / 165 / 162 / 161 us) to nothing (n = 30000,
-// 318 / 322 / 335 / 336 us).
-inline int sym_split(int64_t nt) {
-  const int64_t np = nt * (nt + 1) / 2;
-  int k = 1;
-  if (np < 820)
-    while (k < kSymGroups && np * (2 * k) <= 7000) k *= 2;
-  return k;
-}
+// and, with a coincidence shift, planned, whose sums are bitwise the same): one
+// per source group below 820 pairs (n = 19969), where few whole pairs leave CUs
+// idle or their last round nearly empty.  FP64, 3-D Gaussian, at 1 / 2 / 4 / 8
+// workgroups a pair: n = 5000 60.8 / 35.0 / 24.2 / 21.2 us, n = 16000 140 / 118 /
+// 114 / 110 us.  From 820 pairs on the workspace stays at two row sets a pair, its
+// documented size; there the gain falls from 12 % (n = 20000, 183 / 165 / 162 /
+// 161 us) to nothing (n = 30000, 318 / 322 / 335 / 336 us).
+inline int sym_split(int64_t nt) { return nt * (nt + 1) / 2 < 820 ? kSymGroups : 1; }
 
 // A row set per part for tile I of every pair and one for tile J.
 size_t sym_workspace_bytes(int64_t n) {
