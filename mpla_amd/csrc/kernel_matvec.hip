@@ -1626,6 +1626,12 @@ inline int planned_split(int64_t nt) {
 // 161 us) to nothing (n = 30000, 318 / 322 / 335 / 336 us).
 inline int sym_split(int64_t nt) { return nt * (nt + 1) / 2 < 820 ? kSymGroups : 1; }
 
+// Workgroups per listed pair of a planned product.
+inline int plan_split(const mplak_kernel_desc* d) {
+  const int64_t nt = sym_tiles(d->row_count);
+  return d->coincident_shift != 0.0 ? sym_split(nt) : planned_split(nt);
+}
+
 // A row set per part for tile I of every pair and one for tile J.
 size_t sym_workspace_bytes(int64_t n) {
   const int64_t nt = sym_tiles(n);
@@ -1641,7 +1647,7 @@ int run_sym(const mplak_kernel_desc* d, int precision, int mode, double drop_s, 
   SymArgs a;
   const bool coinc = d->coincident_shift != 0.0;
   const int64_t nt = sym_tiles(d->row_count);
-  a.split = mode == kSymPlanned && !coinc ? planned_split(nt) : sym_split(nt);
+  a.split = mode == kSymPlanned ? plan_split(d) : sym_split(nt);
   if (lv != nullptr) lv->split = a.split;
   // planned FP32 without coincidence shift: the planned kernel, FP32 partials
   const bool tiles = mode == kSymPlanned && precision == MPLAK_PREC_F32 && lv != nullptr && !coinc;
@@ -1719,9 +1725,9 @@ struct PlanLayout {
   int64_t pcap;  // partner slots per (tile, slice)
 };
 
-PlanLayout plan_layout(int64_t n) {
+PlanLayout plan_layout(const mplak_kernel_desc* d) {
   PlanLayout L{};
-  const int64_t nt = sym_tiles(n);
+  const int64_t nt = sym_tiles(d->row_count);
   const size_t np = (size_t)(nt * (nt + 1) / 2);
   L.count = 0;
   L.tinfo = 256;
@@ -1743,7 +1749,7 @@ PlanLayout plan_layout(int64_t n) {
   L.slots = L.pcount + align_up(sizeof(int32_t) * kFinishSlices * (size_t)nt, 256);
   L.part = L.slots + align_up(sizeof(int32_t) * 2 * np, 256);
   // partial rows: by pair (2 per pair) without a plan, slotted with one
-  const int split = std::max(planned_split(nt), sym_split(nt));
+  const int split = plan_split(d);
   const size_t rows = std::max((size_t)2 * np, (size_t)nt * kFinishSlices * (size_t)(L.pcap * split));
   L.total = L.part + rows * kSymTile * sizeof(double);
   return L;
@@ -2096,7 +2102,7 @@ int mplak_kernel_matvec_screened(const mplak_kernel_desc* d, int precision, doub
 
 size_t mplak_screen_plan_bytes(const mplak_kernel_desc* d) {
   if (d == nullptr || d->row_count <= 0 || !sym_eligible(d)) return 0;
-  return plan_layout(d->row_count).total;
+  return plan_layout(d).total;
 }
 
 int mplak_screen_plan_build(const mplak_kernel_desc* d, int precision, double drop_log2, void* plan,
@@ -2106,7 +2112,7 @@ int mplak_screen_plan_build(const mplak_kernel_desc* d, int precision, double dr
   if (precision != MPLAK_PREC_F64 && precision != MPLAK_PREC_F32) return MPLAK_ERR_ARG;
   if (!(drop_log2 > 0.0) || drop_log2 > 2000.0) return MPLAK_ERR_ARG;
   if (!sym_eligible(d) || d->row_count == 0) return MPLAK_ERR_ARG;
-  const PlanLayout L = plan_layout(d->row_count);
+  const PlanLayout L = plan_layout(d);
   if (L.total == 0) return MPLAK_ERR_HIP;
   if (plan == nullptr || plan_bytes < L.total) return MPLAK_ERR_WORKSPACE;
   char* base = static_cast<char*>(plan);
@@ -2148,7 +2154,7 @@ int mplak_screen_plan_counts(const mplak_kernel_desc* d, const void* plan, size_
                              mplak_stream_t s) {
   if (d == nullptr || plan == nullptr || counts == nullptr || d->row_count <= 0 || !sym_eligible(d))
     return MPLAK_ERR_ARG;
-  const PlanLayout L = plan_layout(d->row_count);
+  const PlanLayout L = plan_layout(d);
   if (L.total == 0) return MPLAK_ERR_HIP;
   if (plan_bytes < L.total) return MPLAK_ERR_WORKSPACE;
   const int64_t nt = sym_tiles(d->row_count);
@@ -2169,7 +2175,7 @@ int mplak_kernel_matvec_planned(const mplak_kernel_desc* d, int precision, doubl
   if (!(drop_log2 > 0.0) || drop_log2 > 2000.0) return MPLAK_ERR_ARG;
   if (!sym_eligible(d) || d->row_count == 0) return MPLAK_ERR_ARG;
   if (x == nullptr || y == nullptr) return MPLAK_ERR_ARG;
-  const PlanLayout L = plan_layout(d->row_count);
+  const PlanLayout L = plan_layout(d);
   if (L.total == 0) return MPLAK_ERR_HIP;
   if (plan == nullptr || plan_bytes < L.total) return MPLAK_ERR_WORKSPACE;
   char* base = static_cast<char*>(plan);
@@ -2191,7 +2197,7 @@ int mplak_kernel_matvec_planned_dots(const mplak_kernel_desc* d, int precision, 
   if (!(drop_log2 > 0.0) || drop_log2 > 2000.0) return MPLAK_ERR_ARG;
   if (!sym_eligible(d) || d->row_count == 0) return MPLAK_ERR_ARG;
   if (x == nullptr || y == nullptr || dots == nullptr) return MPLAK_ERR_ARG;
-  const PlanLayout L = plan_layout(d->row_count);
+  const PlanLayout L = plan_layout(d);
   if (L.total == 0) return MPLAK_ERR_HIP;
   if (plan == nullptr || plan_bytes < L.total) return MPLAK_ERR_WORKSPACE;
   char* base = static_cast<char*>(plan);
@@ -2212,7 +2218,7 @@ int mplak_kernel_matvec_planned_relaxed(const mplak_kernel_desc* d, int nlev, co
   if (nlev > 1 && (sel == nullptr || sel_below == nullptr)) return MPLAK_ERR_ARG;
   if (!sym_eligible(d) || d->row_count == 0 || d->coincident_shift != 0.0) return MPLAK_ERR_ARG;
   if (x == nullptr || y == nullptr) return MPLAK_ERR_ARG;
-  const PlanLayout L = plan_layout(d->row_count);
+  const PlanLayout L = plan_layout(d);
   if (L.total == 0) return MPLAK_ERR_HIP;
   if (plan_bytes < L.total) return MPLAK_ERR_WORKSPACE;
   PlanLevels lv{};

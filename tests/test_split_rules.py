@@ -76,3 +76,17 @@ def test_few_targets_fill_the_chip(lib, rows, cols):
     partials = lib.mplak_kernel_matvec_workspace_bytes(C.byref(desc(rows, cols)))
     slabs = partials // (8 * rows)
     assert -(-rows // 256) * slabs >= 256 and partials <= 17e6
+
+
+# A plan holds the partial rows of the split its products take: without a
+# coincidence shift that of the 16 x 16 tiles (pairs times workgroups below 2400),
+# with one that of the vector unit (eight below 820 pairs).
+@pytest.mark.parametrize("n", [4096, 8192, 13000, 16000, 19968, 20480, 40000])
+def test_plans_hold_the_rows_of_their_split(lib, n):
+    tiles = -(-n // 512)
+    pairs = tiles * (tiles + 1) // 2
+    split = max(k for k in (1, 2, 4, 8) if k == 1 or pairs * k < 2400)
+    slots = 4 * -(-tiles // 4)
+    plain, shifted = (lib.mplak_screen_plan_bytes(C.byref(desc(n, n, shift=s))) for s in (0.0, 1e-3))
+    rows = [max(2 * pairs, tiles * slots * k) for k in (split, 8 if pairs < 820 else 1)]
+    assert shifted - plain == (rows[1] - rows[0]) * 512 * 8
