@@ -81,7 +81,7 @@ inline Slabs balanced_slabs(int64_t rows, int64_t cols, int tile_rows, int chunk
       std::min<int64_t>(chunks, std::max<int64_t>(kCus * std::max(4 * occ, 16) / (p.tiles * col_tiles), least));
   const double slab_cost = slab_weight * (0.02 + 2.4e-7 * (double)rows * (double)R);
   double best = 0.0;
-  for (int64_t ks = least; ks <= most; ++ks) {
+  for (int64_t ks = least; ks <= most;) {
     const int64_t per = (chunks + ks - 1) / ks;
     const int64_t slabs = (chunks + per - 1) / per;
     const double m = (double)((p.tiles * col_tiles * slabs + kCus - 1) / kCus) / occ;  // of the busiest CU, in full CUs
@@ -92,6 +92,8 @@ inline Slabs balanced_slabs(int64_t rows, int64_t cols, int tile_rows, int chunk
       p.slabs = slabs;
       p.slab_cols = per * chunk;
     }
+    if (per == 1) break;
+    ks = (chunks + per - 2) / (per - 1);  // the next count has shorter slabs: few counts of many chunks do
   }
   return p;
 }
@@ -636,18 +638,23 @@ inline int valu_rt(int64_t R) {
   return 16;
 }
 
-inline MrhsPlan make_plan(const mplak_kernel_desc* d, int precision, int64_t R) {
+// The kernel of a product, without its slabs.
+inline MrhsPlan make_kernel(const mplak_kernel_desc* d, int precision, int64_t R) {
   MrhsPlan p{};
-  if (precision == MPLAK_PREC_F64 && R >= kMfma64MinR && d->dim <= 4) {
-    p.mfma64 = true;
+  p.mfma64 = precision == MPLAK_PREC_F64 && R >= kMfma64MinR && d->dim <= 4;
+  p.mfma = (precision == MPLAK_PREC_BF16 || precision == MPLAK_PREC_BF16X3 ||
+            (precision == MPLAK_PREC_F32 && R >= 16)) && d->dim <= 4;
+  return p;
+}
+
+inline MrhsPlan make_plan(const mplak_kernel_desc* d, int precision, int64_t R) {
+  MrhsPlan p = make_kernel(d, precision, R);
+  if (p.mfma64) {
     p.cblocks = (R + 15) / 16;
     p.s = balanced_slabs(d->row_count, d->col_count, kTile64, kSrc64, waves64((int)std::min<int64_t>(p.cblocks, 4)), R);
     p.part_bytes = align_up((size_t)p.s.slabs * (size_t)R * (size_t)d->row_count * sizeof(double), 256);
     return p;
   }
-  const bool wide = R >= 16;
-  p.mfma = (precision == MPLAK_PREC_BF16 || precision == MPLAK_PREC_BF16X3 ||
-            (precision == MPLAK_PREC_F32 && wide)) && d->dim <= 4;
   if (p.mfma) {
     p.mode = precision == MPLAK_PREC_BF16 ? kModeBf16 : (precision == MPLAK_PREC_BF16X3 ? kModeBf16x3 : kModeF32);
     p.cblocks = (R + 31) / 32;
@@ -671,7 +678,7 @@ inline MrhsPlan make_plan(const mplak_kernel_desc* d, int precision, int64_t R) 
 
 // Columns per launch: the matrix-core kernels hold at most kMfmaGroup.
 inline int64_t column_group(const mplak_kernel_desc* d, int precision, int64_t nrhs) {
-  const MrhsPlan p = make_plan(d, precision, nrhs);
+  const MrhsPlan p = make_kernel(d, precision, nrhs);
   return p.mfma || p.mfma64 ? kMfmaGroup : nrhs;
 }
 

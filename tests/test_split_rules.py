@@ -90,3 +90,18 @@ def test_plans_hold_the_rows_of_their_split(lib, n):
     plain, shifted = (lib.mplak_screen_plan_bytes(C.byref(desc(n, n, shift=s))) for s in (0.0, 1e-3))
     rows = [max(2 * pairs, tiles * slots * k) for k in (split, 8 if pairs < 820 else 1)]
     assert shifted - plain == (rows[1] - rows[0]) * 512 * 8
+
+
+# Planning a product of few targets and a million sources: the search for the slab
+# count takes microseconds (every count one by one: 150 to 220 us a query).
+@pytest.mark.parametrize("rows,prec,R", [(1, F64, 1), (256, F32, 4), (256, BF16, 64), (100, F64, 64)])
+def test_planning_is_quick(lib, rows, prec, R):
+    import time
+    d = desc(rows, 1000000)
+
+    def query():
+        t = time.perf_counter()
+        lib.mplak_kernel_mrhs_workspace_bytes(C.byref(d), prec, R)
+        return time.perf_counter() - t
+
+    assert min(query() for _ in range(100)) < 75e-6
