@@ -609,6 +609,76 @@ __global__ __launch_bounds__(kBlock) void mrhs_finish_kernel(int64_t rows, int64
   }
 }
 
+// The same where few targets have many slabs, the sum of a row being a chain of
+// latencies: 2^shift rows per workgroup, whose other threads are slices k of the
+// slabs (k, k + slices, ...); the slices' sums are added in a tree.
+template <typename PT>
+__global__ __launch_bounds__(kBlock) void mrhs_finish_sliced_kernel(int64_t rows, int64_t R, int64_t slabs, int shift,
+                                                                    const PT* __restrict__ part, int64_t row_off,
+                                                                    int64_t col_off, int64_t cols, double nugget,
+                                                                    const double* __restrict__ V, int64_t ldv,
+                                                                    double* __restrict__ Y, int64_t ldy,
+                                                                    const int32_t* __restrict__ skip) {
+  if (skip != nullptr && *skip != 0) return;
+  __shared__ double red[kBlock];
+  const int tid = threadIdx.x, slices = kBlock >> shift, slice = tid >> shift;
+  const int64_t i = ((int64_t)blockIdx.x << shift) + (tid & ((1 << shift) - 1));
+  for (int64_t r = blockIdx.y; r < R; r += gridDim.y) {
+    double s = 0.0;
+    if (i < rows) {
+      const PT* p = part + r * rows + i;
+      for (int64_t k = slice; k < slabs; k += kFinishBatch * slices) {
+        PT v[kFinishBatch];
+#pragma unroll
+        for (int u = 0; u < kFinishBatch; ++u) {
+          const int64_t q = k + u * slices;
+          v[u] = q < slabs ? p[q * R * rows] : PT(0);
+        }
+#pragma unroll
+        for (int u = 0; u < kFinishBatch; ++u)
+          if (k + u * slices < slabs) s += (double)v[u];
+      }
+    }
+    red[tid] = s;
+    __syncthreads();
+    for (int h = kBlock / 2; h >= (1 << shift); h >>= 1) {
+      if (tid < h) red[tid] += red[tid + h];
+      __syncthreads();
+    }
+    if (slice == 0 && i < rows) {
+      s = red[tid];
+      const int64_t jd = row_off + i - col_off;
+      if (nugget != 0.0 && jd >= 0 && jd < cols) s = fma(nugget, V[r * ldv + jd], s);
+      Y[r * ldy + i] = s;
+    }
+    __syncthreads();
+  }
+}
+
+// Rows of a finish workgroup, as a power of two: 256, halved while the launch has
+// fewer than 1024 workgroups and a thread more than 32 slabs.  The whole product with one row a thread / so: BF16x3 in 3-D,
+// 64 columns, 256 x 300000 421 / 166 us, 200 x 65536 104 / 49 us, 1000 x 20000 58 / 45
+// us; FP64, 8 columns, 200 x 65536 51 / 38 us.  Two slices of 32 slabs lose
+// (8000 points, FP32, 8 columns: 53 / 57 us).
+inline int finish_shift(int64_t rows, int64_t R, int64_t slabs) {
+  int shift = 8;
+  while (shift > 0 && ((rows + (int64_t(1) << shift) - 1) >> shift) * R < 1024 && slabs > int64_t(32) << (8 - shift)) --shift;
+  return shift;
+}
+
+template <typename PT>
+void launch_finish(const mplak_kernel_desc* d, hipStream_t st, int64_t R, int64_t slabs, const PT* part,
+                   const double* V, int64_t ldv, double* Y, int64_t ldy, const int32_t* skip) {
+  const int shift = finish_shift(d->row_count, R, slabs);
+  const dim3 grid((unsigned)((d->row_count + (int64_t(1) << shift) - 1) >> shift), (unsigned)std::min<int64_t>(R, 65535));
+  if (shift == 8)
+    hipLaunchKernelGGL(mrhs_finish_kernel<PT>, grid, dim3(kBlock), 0, st, d->row_count, R, slabs, part, d->row_offset,
+                       d->col_offset, d->col_count, d->nugget, V, ldv, Y, ldy, skip);
+  else
+    hipLaunchKernelGGL(mrhs_finish_sliced_kernel<PT>, grid, dim3(kBlock), 0, st, d->row_count, R, slabs, shift, part,
+                       d->row_offset, d->col_offset, d->col_count, d->nugget, V, ldv, Y, ldy, skip);
+}
+
 // ---------------------------------------------------------------------------
 // host-side planning and dispatch
 
@@ -862,13 +932,10 @@ int mplak_kernel_mrhs(const mplak_kernel_desc* d, int precision, int64_t nrhs, c
     }
     st = launch_status();
     if (st != MPLAK_OK) return st;
-    const dim3 fgrid((unsigned)((d->row_count + kBlock - 1) / kBlock), (unsigned)std::min<int64_t>(R, 65535));
     if (p.mfma)
-      hipLaunchKernelGGL(mrhs_finish_kernel<float>, fgrid, dim3(kBlock), 0, hs, d->row_count, R, p.s.slabs, part32,
-                         d->row_offset, d->col_offset, d->col_count, d->nugget, Vg, ldv, Yg, ldy, skip_if);
+      launch_finish(d, hs, R, p.s.slabs, part32, Vg, ldv, Yg, ldy, skip_if);
     else
-      hipLaunchKernelGGL(mrhs_finish_kernel<double>, fgrid, dim3(kBlock), 0, hs, d->row_count, R, p.s.slabs, part,
-                         d->row_offset, d->col_offset, d->col_count, d->nugget, Vg, ldv, Yg, ldy, skip_if);
+      launch_finish(d, hs, R, p.s.slabs, part, Vg, ldv, Yg, ldy, skip_if);
     st = launch_status();
     if (st != MPLAK_OK) return st;
   }

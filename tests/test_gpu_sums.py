@@ -112,3 +112,31 @@ def test_planned_fp32_distances_of_both_forms(lib, n, dim, ell):
                                                       x.data_ptr(), y.data_ptr(), None, stream()))
         error[form] = float((y - ref).norm() / ref.norm())
     assert error[dim] <= 1.05 * error[3]
+
+
+# Few targets and many sources: many slabs, whose partials a finish workgroup adds
+# in 2 to 256 slices (256 to 1 rows), and just too few slabs or too many rows for it.
+@pytest.mark.parametrize("rows,cols,R", [(1, 20011, 1), (2, 3000, 64), (3, 70001, 16), (65, 20000, 9), (127, 2111, 5),
+                                         (200, 65536, 64), (257, 30000, 8), (1000, 20000, 64), (1, 500, 3)])
+@pytest.mark.parametrize("prec,bar", [(_native.MPLAK_PREC_F64, 1e-12), (_native.MPLAK_PREC_F32, 2e-5),
+                                      (_native.MPLAK_PREC_BF16X3, 1e-4)])
+def test_mrhs_few_targets(lib, rows, cols, R, prec, bar):
+    import torch
+    dim, ell, off, nugget, ldv, ldy = 3, 0.3, 5, 0.7, cols + 1, rows + 2
+    g = torch.Generator(device="cuda").manual_seed(cols + R)
+    P = torch.rand((dim, cols + off), generator=g, dtype=torch.float64, device="cuda")
+    V = torch.randn((R, ldv), generator=g, dtype=torch.float64, device="cuda")
+    Y = torch.full((R, ldy), 7.0, dtype=torch.float64, device="cuda")
+    K = (-sum((P[d, off:off + rows, None] - P[d][None, :cols]) ** 2 for d in range(dim)) / (2 * ell ** 2)).exp()
+    K[torch.arange(rows), torch.arange(rows) + off] += nugget
+    ref, mag = host(V[:, :cols] @ K.t()), host(V[:, :cols].abs() @ K.t())
+    table = torch.tensor([P[d].data_ptr() for d in range(dim)], dtype=torch.int64, device="cuda")
+    desc = _native.mplak_kernel_desc(table.data_ptr(), dim, 0, ell, nugget, 0.0, off, rows, 0, cols)
+    wb = lib.mplak_kernel_mrhs_workspace_bytes(C.byref(desc), prec, R)
+    w = workspace(wb)
+    w.fill_(float("nan"))
+    _native.check(lib.mplak_kernel_mrhs(C.byref(desc), prec, R, V.data_ptr(), ldv, Y.data_ptr(), ldy, w.data_ptr(), wb,
+                                        None, stream()))
+    got = host(Y)
+    err = np.linalg.norm(got[:, :rows] - ref, axis=1)
+    assert np.all(err <= bar * np.linalg.norm(mag, axis=1)) and np.all(got[:, rows:] == 7.0)
