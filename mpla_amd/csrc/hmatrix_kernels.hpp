@@ -202,10 +202,14 @@ __device__ __forceinline__ double factor_load(const double* p) {
 
 // Far field for the rows of an apply item: sum over the leaf's admissible
 // blocks b (those of part `part` of `parts`, wave-uniform) of
-// U_b(row - r0_b, :) t_b, kHmTerms terms of both rows in flight at a time.
-constexpr int kHmTerms = 8;
+// U_b(row - r0_b, :) t_b, TERMS terms of both rows in flight at a time.  Eight
+// take 76 registers and leave six waves per SIMD, which suits launches of the far
+// field alone.  Kernels whose near field streams take four and keep eight waves:
+// the product with stored entries (4.4 GB and 1 GB of factors at n = 131072, 2-D)
+// 1.62 -> 1.16 ms.
+constexpr int kHmTerms = 8, kHmNearTerms = 4;
 
-template <bool STREAM>
+template <bool STREAM, int TERMS = kHmTerms>
 __device__ __forceinline__ void far_rows(const int64_t (&row)[kHmLaneRows], const bool (&valid)[kHmLaneRows],
                                          const int64_t* __restrict__ far_ptr, const int32_t* __restrict__ far_blk,
                                          int32_t leaf, const mplak_hm_block* __restrict__ blocks,
@@ -221,15 +225,15 @@ __device__ __forceinline__ void far_rows(const int64_t (&row)[kHmLaneRows], cons
     const double* u[kHmLaneRows];
 #pragma unroll
     for (int h = 0; h < kHmLaneRows; ++h) u[h] = U + B.uoff + (row[h] - B.r0);  // rows past the item: its first
-    for (int q0 = 0; q0 < rb; q0 += kHmTerms) {
-      double v[kHmLaneRows][kHmTerms];
+    for (int q0 = 0; q0 < rb; q0 += TERMS) {
+      double v[kHmLaneRows][TERMS];
 #pragma unroll
-      for (int q = 0; q < kHmTerms; ++q)
+      for (int q = 0; q < TERMS; ++q)
 #pragma unroll
         for (int h = 0; h < kHmLaneRows; ++h)
           if (q0 + q < rb) v[h][q] = factor_load<STREAM>(u[h] + (q0 + q) * B.m);
 #pragma unroll
-      for (int q = 0; q < kHmTerms; ++q)
+      for (int q = 0; q < TERMS; ++q)
 #pragma unroll
         for (int h = 0; h < kHmLaneRows; ++h)
           if (q0 + q < rb) acc[h] = valid[h] ? fma(v[h][q], tb[q0 + q], acc[h]) : acc[h];
@@ -333,7 +337,7 @@ __global__ __launch_bounds__(kHmApplyThreads) void apply_kernel(
       }
     }
   }
-  far_rows<false>(row, valid, far_ptr, far_blk, c.leaf, blocks, rank, kmax, U, t, part, kHmParts, acc);
+  far_rows<false, kHmNearTerms>(row, valid, far_ptr, far_blk, c.leaf, blocks, rank, kmax, U, t, part, kHmParts, acc);
   finish_rows(acc, row, valid, ys, red);
 }
 
@@ -368,7 +372,7 @@ __global__ __launch_bounds__(kHmApplyThreads) void apply_generic_kernel(
       for (int64_t s = part; s < cn; s += kHmParts) acc[h] = fma(e(row[h], c0 + s, tab), xs[c0 + s], acc[h]);
     }
   }
-  far_rows<false>(row, valid, far_ptr, far_blk, c.leaf, blocks, rank, kmax, U, t, part, kHmParts, acc);
+  far_rows<false, kHmNearTerms>(row, valid, far_ptr, far_blk, c.leaf, blocks, rank, kmax, U, t, part, kHmParts, acc);
   finish_rows(acc, row, valid, ys, red);
 }
 
@@ -426,7 +430,7 @@ __global__ __launch_bounds__(kHmApplyThreads) void apply_stored_kernel(
         if (valid[h]) acc[h] = fma(a[(row[h] - lo) + s * m], xv, acc[h]);
     }
   }
-  far_rows<false>(row, valid, far_ptr, far_blk, c.leaf, blocks, rank, kmax, U, t, part, kHmParts, acc);
+  far_rows<false, kHmNearTerms>(row, valid, far_ptr, far_blk, c.leaf, blocks, rank, kmax, U, t, part, kHmParts, acc);
   finish_rows(acc, row, valid, ys, red);
 }
 

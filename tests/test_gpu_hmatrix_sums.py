@@ -73,3 +73,46 @@ def test_apply_pairs_in_one_launch(lib, leaves, m, far, rank, ents):
     got = host(r.ys)
     # a sum in any order: at most one rounding of a partial sum per term
     assert np.all(np.abs(got[:-1] - r.ref) <= (far * rank + ents) * 2.0 ** -53 * r.mag) and got[-1] == 7.0
+
+
+def median_us(f, runs=15):
+    import torch
+    times = []
+    for _ in range(runs):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        f()
+        b.record()
+        torch.cuda.synchronize()
+        times.append(a.elapsed_time(b) * 1e3)
+    return sorted(times)[runs // 2]
+
+
+# The per-row product with stored near entries reads 2 GB of them once: it keeps at
+# least three quarters of the rate of a plain sum of the same buffer, so its far
+# field may not take the registers that its resident waves need.
+def test_stored_near_entries_stream(lib):
+    import torch
+    m, leaves, ranges = 512, 256, 4
+    n = m * leaves
+    g = torch.Generator(device="cuda").manual_seed(3)
+    st = torch.rand((leaves, ranges, m, m), generator=g, dtype=torch.float64, device="cuda") - 0.5  # column-major blocks
+    xs = torch.rand(n, generator=g, dtype=torch.float64, device="cuda") - 0.5
+    ys = torch.full((n + 1,), 7.0, dtype=torch.float64, device="cuda")
+    col = [[(leaf + 3 * k) % leaves for k in range(ranges)] for leaf in range(leaves)]
+    ints = lambda a: torch.as_tensor(np.ascontiguousarray(a, dtype=np.int64), device="cuda")  # noqa: E731
+    chunks = (Chunk * (n // 128))(*[(r // m, 128, r) for r in range(0, n, 128)])
+    chunks = torch.frombuffer(bytearray(bytes(chunks)), dtype=torch.uint8).to("cuda")
+    leaf_range, near_ptr = ints([(leaf * m, m) for leaf in range(leaves)]), ints(np.arange(leaves + 1) * ranges)
+    near_cols = ints([(c * m, m) for row in col for c in row])
+    near_off, far_ptr = ints(np.arange(leaves * ranges) * m * m), ints(np.zeros(leaves + 1))
+
+    def product():
+        _native.check(lib.mplak_hm_apply_stored(p(chunks), n // 128, p(leaf_range), p(near_ptr), p(near_cols),
+                                                p(near_off), p(st), p(far_ptr), None, None, None, 1, None, None, p(xs),
+                                                p(ys), torch.cuda.current_stream().cuda_stream))
+
+    product()
+    ref = torch.stack([(st[leaf] * xs.view(leaves, m)[col[leaf]][:, :, None]).sum((0, 1)) for leaf in range(leaves)])
+    assert float((ys[:-1] - ref.reshape(-1)).abs().max()) <= 1e-12 * ranges * m and float(ys[-1]) == 7.0
+    assert median_us(product) <= median_us(lambda: st.sum()) / 0.75
