@@ -416,6 +416,9 @@ __device__ __forceinline__ void sym_valu_pair(const double* const* __restrict__ 
   for (int it = 0; it < kPer; ++it) {
     const int k = tid + it * kBlock;
     const int64_t j = J * kSymTile + k;
+    // other parts' groups are not read: neither staged nor (the larger cost, in a
+    // screened product) reduced to a box
+    if (((groups >> (w + it * (kBlock / kWave))) & 1u) == 0) continue;
     Q q;
     q.x = (T)(sc_[it][0] * scale);
     q.y = T(0);
@@ -1620,8 +1623,10 @@ inline int planned_split(int64_t nt) {
 // and, with a coincidence shift, planned, whose sums are bitwise the same): one
 // per source group below 820 pairs (n = 19969), where few whole pairs leave CUs
 // idle or their last round nearly empty.  FP64, 3-D Gaussian, at 1 / 2 / 4 / 8
-// workgroups a pair: n = 5000 60.8 / 35.0 / 24.2 / 21.2 us, n = 16000 140 / 118 /
-// 114 / 110 us.  From 820 pairs on the workspace stays at two row sets a pair, its
+// workgroups a pair: n = 5000 60.8 / 35.0 / 24.2 / 21.2 us, n = 16000 138 / 117 /
+// 113 / 106 us; n = 19000, the least gain, exact 143 / 143 / 148 / 145 us, screened
+// with little to drop 148 / 148 / 154 / 154 us, with much (length scale 0.05) 144 /
+// 131 / 122 / 118 us.  From 820 pairs on the workspace stays at two row sets a pair, its
 // documented size; there the gain falls from 12 % (n = 20000, 183 / 165 / 162 /
 // 161 us) to nothing (n = 30000, 318 / 322 / 335 / 336 us).
 inline int sym_split(int64_t nt) { return nt * (nt + 1) / 2 < 820 ? kSymGroups : 1; }

@@ -1,5 +1,5 @@
 """Symmetric products with a coincidence shift on both sides of the pair split:
-eight workgroups a tile pair (13000 points) and one (20481), with coincident
+eight workgroups a tile pair (600 and 13000 points) and one (20481), with coincident
 points in tiles of their own and in others."""
 import ctypes as C
 
@@ -18,16 +18,16 @@ def lib():
     return _native.mplak()
 
 
-@pytest.mark.parametrize("n,dim", [(13000, 2), (20481, 3)])
+@pytest.mark.parametrize("n,dim", [(600, 1), (13000, 2), (20481, 3)])
 @pytest.mark.parametrize("kind", [0, 1])
 @pytest.mark.parametrize("prec,bar", [(_native.MPLAK_PREC_F64, 1e-12), (_native.MPLAK_PREC_F32, 2e-5)])
-def test_symmetric_products_with_coincident_points(lib, n, dim, kind, prec, bar):
+def test_symmetric_products_with_coincident_points(lib, monkeypatch, n, dim, kind, prec, bar):
     import torch
     g = torch.Generator(device="cuda").manual_seed(n)
     P = torch.rand((dim, n), generator=g, dtype=torch.float64, device="cuda")
     P = P[:, torch.argsort(P[0])].contiguous()
-    P[:, 9::1000] = P[:, 8::1000][:, :P[:, 9::1000].shape[1]]  # neighbours
-    P[:, n - 40:] = P[:, 100:4100:100]                         # the last tile repeats points of the first ones
+    P[:, 9::100] = P[:, 8::100][:, :P[:, 9::100].shape[1]]  # neighbours
+    P[:, n - 40:] = P[:, 100:500:10]                        # the last tile repeats points of the first one
     x = torch.rand(n, generator=g, dtype=torch.float64, device="cuda") - 0.5
     ell, nugget, shift = (0.05, 0.1)[kind], 0.5, 0.25
     ref, mag = torch.empty_like(x), torch.empty_like(x)
@@ -39,6 +39,7 @@ def test_symmetric_products_with_coincident_points(lib, n, dim, kind, prec, bar)
     ref, mag = host(ref + nugget * x), host(mag + nugget * x.abs())
     table = torch.tensor([P[d].data_ptr() for d in range(dim)], dtype=torch.int64, device="cuda")
     desc = _native.mplak_kernel_desc(table.data_ptr(), dim, kind, ell, nugget, shift, 0, n, 0, n)
+    monkeypatch.setenv("MPLAK_KMV_SYMMETRIC", "1")
     wb = lib.mplak_kernel_matvec_workspace_bytes(C.byref(desc))
     y = torch.empty_like(x)
 
