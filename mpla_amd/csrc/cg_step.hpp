@@ -1,5 +1,5 @@
-// One CG iteration of a column by one workgroup, shared by the single, batched
-// and ragged solvers.
+// One CG iteration of a column by one workgroup, for the single and the batched
+// solver.
 #pragma once
 
 #include "common.hpp"

@@ -273,19 +273,19 @@ void add_products(Upload& u, const std::vector<mplak_ragged_system>& systems, in
     const size_t first = u.items.size();
     for (size_t k : order) add_items(k);
     u.launches.push_back({3, 0, 0, precision, 0, 0.0, first, (int64_t)(u.items.size() - first)});
-  } else
-  // one launch per (scheme, rt, dim) class: kernels specialised for each;
-  // the pair scheme (large systems, heavier items) first
-  for (int scheme : {MPLAK_RAGGED_PAIRS, MPLAK_RAGGED_SLABS})
-    for (int rt : {1, 2, 4, 8})
-      for (int dim = 1; dim <= MPLA_SERVER_MAX_DIM; ++dim) {
-        const size_t first = u.items.size();
-        for (size_t k = 0; k < systems.size(); ++k) {
-          if (systems[k].scheme == scheme && systems[k].rt == rt && systems[k].dim == dim) add_items(k);
+  } else {
+    // one launch per (scheme, rt, dim) class: kernels specialised for each;
+    // the pair scheme (large systems, heavier items) first
+    for (int scheme : {MPLAK_RAGGED_PAIRS, MPLAK_RAGGED_SLABS})
+      for (int rt : {1, 2, 4, 8})
+        for (int dim = 1; dim <= MPLA_SERVER_MAX_DIM; ++dim) {
+          const size_t first = u.items.size();
+          for (size_t k = 0; k < systems.size(); ++k)
+            if (systems[k].scheme == scheme && systems[k].rt == rt && systems[k].dim == dim) add_items(k);
+          const int64_t count = (int64_t)(u.items.size() - first);
+          if (count > 0) u.launches.push_back({0, dim, rt, precision, 0, 0.0, first, count, scheme});
         }
-        const int64_t count = (int64_t)(u.items.size() - first);
-        if (count > 0) u.launches.push_back({0, dim, rt, precision, 0, 0.0, first, count, scheme});
-      }
+  }
   const size_t first = u.items.size();
   for (size_t k = 0; k < systems.size(); ++k) {
     const int64_t c = mplak_ragged_finish_items(&systems[k], nullptr, 0);

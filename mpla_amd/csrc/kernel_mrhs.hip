@@ -66,9 +66,9 @@ struct Slabs {
 // rounds of shorter ones (BF16, n = 131072, 64 columns: 6.41 ms in 2 slabs, 5.70
 // ms in 8); short ones lose less than their slabs cost (n = 12000: 2 % per
 // iteration with the share taken of every chunk).
+// `longest`: most sources of a slab.
 constexpr double kMfmaDrain = 0.12;
 constexpr int64_t kDrainChunks = 64;
-// `longest`: most sources of a slab.
 inline Slabs balanced_slabs(int64_t rows, int64_t cols, int tile_rows, int chunk, int occ, int64_t R,
                             int64_t col_tiles = 1, double slab_weight = 1.0, double drain = 0.0,
                             int64_t longest = INT64_MAX) {

@@ -6,12 +6,14 @@
 // One launch covers every system in the batch: workgroup b processes item b,
 // whose fields name the system and the tile of work.  Each system's tiles,
 // slabs and vector blocks depend only on that system's own (n, nrhs,
-// precision), never on what else is in the batch, so a system's arithmetic,
-// and therefore its result, is bitwise the same alone and in any mix.
+// precision, bytes of its partials), never on what else is in the batch, so a
+// system's arithmetic, and therefore its result, is bitwise the same alone and
+// in any mix.
 //
 // Products, two work splits (mplak_ragged_plan picks one per system from its
-// n alone): SLABS, the VALU scheme of the multi-RHS product (one target per
-// thread, RT columns per thread, sources through LDS, FP64 slab partials);
+// n alone, mplak_ragged_plan_within from the bytes of its partials too): SLABS,
+// the VALU scheme of the multi-RHS product (one target per thread, RT columns per
+// thread, sources through LDS, FP64 slab partials);
 // PAIRS, the symmetric tile-pair form (each off-diagonal entry evaluated once
 // for both of its rows).  The kernel function, dimension (<= 4) and scale
 // come from the system record.
@@ -524,7 +526,7 @@ constexpr int kFinishSlices = kBlock / kWave;
 // leaves a sum that started at +0.0 unchanged.
 template <typename T>
 __device__ __forceinline__ double pair_finish_row(const mplak_ragged_system& S, int64_t i, int64_t r, int k) {
-  // pair indices and parts fit 32 bits (use_pairs, plan_split); the split is a
+  // pair indices and parts fit 32 bits (use_pairs, mixed_parts); the split is a
   // power of two, so there is no division in the loop
   const uint32_t X = (uint32_t)(i / kPairTile), t = (uint32_t)(i % kPairTile), tiles = (uint32_t)S.tiles;
   const uint32_t split = (uint32_t)pair_split(S), shift = (uint32_t)__builtin_ctz(split);
