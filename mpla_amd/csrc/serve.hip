@@ -183,7 +183,7 @@ __device__ __forceinline__ void slab_item(const mplak_ragged_item& it, const mpl
     for (int q = 0; q < RT; ++q) {
       if (r0 + q >= R) continue;
       const int64_t k = ((int64_t)it.slab * R + r0 + q) * n + i;
-      if (sizeof(T) == 4 && narrow_slabs(S)) part32[k] = (float)acc[q];
+      if (narrow_slabs(S)) part32[k] = (float)acc[q];
       else S.part[k] = acc[q];
     }
   }
